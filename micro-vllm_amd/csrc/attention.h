@@ -119,6 +119,9 @@ bool prefill_supported(const AttnArgs& a, int32_t dtype);
 // kernel with its default shape (kStepDecodeWaves waves, two stages).
 constexpr int kStepDecodeWaves = 4;
 bool decode_step_eligible(const AttnArgs& a);
+// The split-KV decode kernels cover this head_dim with this block size and
+// split length (128 always; 64 and 96 with the pipelined kernel only).
+bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens);
 int64_t decode_step_blocks(const AttnArgs& a);  // decode workgroups of the step grid
 int launch_decode_combine(const AttnArgs& a, int32_t dtype, hipStream_t s);
 // `prefill_first`: the prefill workgroups lead the grid (else the decode ones).

@@ -251,24 +251,46 @@ void fill_batch_args(AttnArgs& a, const mvllm_batch* batch, const mvllm_kv_cache
 
 // The cache-side conditions of the MFMA kernels (the query and output add
 // their own): a plan is built whenever a planned call can take that path.
-bool fast_cache(const mvllm_kv_cache* cache, int64_t group) {
+bool fast_cache(const mvllm_kv_cache* cache, const mvllm_batch* batch, int64_t group) {
   const int32_t dtype = cache->dtype;
   const int64_t es = dtype_bytes(dtype);
-  return (dtype == MVLLM_DTYPE_BF16 || dtype == MVLLM_DTYPE_F16) && cache->head_dim == 128 && group <= 16 &&
+  return (dtype == MVLLM_DTYPE_BF16 || dtype == MVLLM_DTYPE_F16) && group <= 16 &&
+         decode_supported(cache->head_dim, cache->block_size,
+                          decode_split_tokens(batch->num_requests, batch->block_table_width * batch->block_size)) &&
          cache->stride[4] == 1 && cache->stride[3] == cache->head_dim && vec16(cache->stride[0], es) &&
          vec16(cache->stride[1], es) && vec16(cache->stride[2], es) && aligned16(cache->data);
 }
 
+// head_dim 64 and 96 take the MFMA kernels because the generic kernel scores
+// one key per lane without matrix instructions: a batch of 30 decodes (128 to
+// 2,048 keys) and two chunks of ~230 tokens with 32/8 heads of 64 took 1,414 us
+// per forward there and takes 47 us here. Both are still answered by the
+// generic kernel, which needs no workspace and has no limits on reach or grid; calls outside the work
+// lists' limits therefore go there instead of failing. At head_dim 128 the
+// limits are errors of their own (bind_workspace, the launchers).
+bool takes_lists(const mvllm_batch* batch, const mvllm_kv_cache* cache, int64_t Hq, const void* workspace,
+                 int64_t workspace_bytes) {
+  if (cache->head_dim == 128) return true;
+  constexpr int64_t kMost = int64_t{1} << 30;
+  const DecodeLayout d = decode_layout(batch, Hq, cache->head_dim);
+  return workspace && aligned16(workspace) && workspace_bytes >= d.total() &&
+         batch->block_table_width * batch->block_size < kMost && batch->num_tokens < kMost &&
+         batch->num_requests * d.max_splits * cache->num_kv_heads < kMost &&
+         (batch->num_tokens / 8 + batch->num_requests) * cache->num_kv_heads < kMost &&
+         batch->num_requests * Hq < kMost;
+}
+
 // The MFMA decode / prefill path (with work lists) applies: 16-byte aligned
-// rows of query, output and cache, head_dim 128, a supported group size and
-// at least one request; otherwise the generic kernel runs.
+// rows of query, output and cache, a supported head_dim (decode_supported)
+// and group size, and at least one request; otherwise the generic kernel runs.
 bool attention_fast_path(const mvllm_tensor3* query, const mvllm_kv_cache* cache, const mvllm_tensor3* out,
-                         const mvllm_batch* batch) {
+                         const mvllm_batch* batch, const void* workspace, int64_t workspace_bytes) {
   if (!query || !cache || !out || !batch || batch->num_requests <= 0) return false;
   const int64_t Hkv = cache->num_kv_heads;
   if (Hkv <= 0 || query->size[1] % Hkv != 0) return false;
   const int64_t es = dtype_bytes(query->dtype);
-  return fast_cache(cache, query->size[1] / Hkv) && query->stride[2] == 1 && vec16(query->stride[0], es) &&
+  return fast_cache(cache, batch, query->size[1] / Hkv) &&
+         takes_lists(batch, cache, query->size[1], workspace, workspace_bytes) && query->stride[2] == 1 && vec16(query->stride[0], es) &&
          vec16(query->stride[1], es) && aligned16(query->data) && out->stride[2] == 1 &&
          vec16(out->stride[0], es) && vec16(out->stride[1], es) && aligned16(out->data);
 }
@@ -301,9 +323,10 @@ int attention_plan(const mvllm_batch* batch, int64_t Hq, const mvllm_kv_cache* c
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0)
     return fail(MVLLM_ERR_INVALID, "query heads %lld not a multiple of KV heads %lld", (long long)Hq,
                 (long long)Hkv);
-  if (batch->num_tokens == 0 || batch->num_requests == 0 || !fast_cache(cache, Hq / Hkv)) return MVLLM_OK;
+  if (batch->num_tokens == 0 || batch->num_requests == 0 || !fast_cache(cache, batch, Hq / Hkv)) return MVLLM_OK;
   AttnArgs a = {};
   fill_batch_args(a, batch, cache, Hq);
+  if (!takes_lists(batch, cache, Hq, workspace, workspace_bytes)) return MVLLM_OK;
   if (int rc = bind_workspace(a, batch, Hq, D, workspace, workspace_bytes)) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (int rc = launch_decode_lists(a, s)) return rc;
@@ -346,7 +369,7 @@ int paged_attention(const mvllm_tensor3* query, const mvllm_kv_cache* cache,
   a.scale_log2 = scale * 1.4426950408889634f;  // log2(e)
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 
-  const bool fast = attention_fast_path(query, cache, out, batch);
+  const bool fast = attention_fast_path(query, cache, out, batch, workspace, workspace_bytes);
   if (!fast) {
     if (fused_kv) {
       // Only the rows: the generic kernel needs no work lists.
@@ -436,7 +459,7 @@ int attention_forward(const mvllm_tensor3* query, const mvllm_tensor3* key,
       return rc;
     // The fused prologue needs the attention's MFMA path (the work lists)
     // and 16-byte rows; everything else writes the rows first, on its own.
-    if (vectorised && attention_fast_path(query, cache, out, batch))
+    if (vectorised && attention_fast_path(query, cache, out, batch, workspace, workspace_bytes))
       return paged_attention(query, cache, batch, out, scale, workspace, workspace_bytes, timing, stream, false,
                              single_stream, &rows);
     if (int rc = mvllm_kv_write(key, value, cache, batch->slot_mapping, batch->num_tokens, stream))

@@ -1,4 +1,5 @@
-// Split-KV ragged decode on gfx950 matrix cores (head_dim 128, bf16/fp16).
+// Split-KV ragged decode on gfx950 matrix cores (bf16/fp16; head_dim 128, and
+// 64 and 96 where the block size is a multiple of 16).
 //
 // Work item: (KV head, split of the visible context, request). One wavefront
 // owns one KV head; a workgroup holds up to 8 waves = 8 consecutive KV heads
@@ -10,9 +11,9 @@
 // Each record carries the request's query token, visible range and the
 // split's key range, so a workgroup needs no metadata loads of its own.
 //
-// Per 16-token tile a wave computes S^T = K . Q^T with four
-// v_mfma_f32_16x16x32 (M = 16 tokens, N = the G query heads of the KV head,
-// padded to 16, K = 128 dims), so K is consumed straight from its natural
+// Per 16-token tile a wave computes S^T = K . Q^T with v_mfma_f32_16x16x32
+// (M = 16 tokens, N = the G query heads of the KV head, padded to 16,
+// K = head_dim), so K is consumed straight from its natural
 // row layout. The softmax runs on the accumulator layout (each lane holds 4
 // tokens of one head: max/sum need only two cross-lane steps). P^T is
 // already the B operand of O^T += V^T . P^T (v_mfma_f32_16x16x16), which
@@ -30,6 +31,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include <hip/hip_ext.h>
 
@@ -40,6 +42,7 @@ namespace {
 
 using namespace dec;
 
+constexpr int kDim = 128;  // head_dim of the general kernel
 constexpr int kRow = 144;  // LDS row stride (elements): 288 B keeps both LDS access patterns conflict-free
 constexpr int kMaxWaves = 8;
 
@@ -120,11 +123,9 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
     }
   }
 
-  float4_t acc[2][4];
+  float4_t acc[kDim / 16];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[j][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < kDim / 16; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   uint16_t* slab = lds[wave];
   const uint16_t* cache = static_cast<const uint16_t*>(a.cache);
@@ -157,9 +158,7 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
     l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     if (__ballot(alpha != 1.f)) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[j][c] *= alpha;
+      for (int b = 0; b < kDim / 16; ++b) acc[b] *= alpha;
     }
     m = mn;
 
@@ -177,22 +176,13 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
       *reinterpret_cast<short8_t*>(slab + col * kRow + 32 * i + 8 * grp) = cur.v[i];
     wave_lds_sync();
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      uint2 rv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        rv[e] = *reinterpret_cast<const uint2*>(slab + (4 * grp + e) * kRow + 64 * j + 4 * col);
-      // A operand c: row col <-> dim 64j + 4col + c; k = tokens 4grp + e.
-      short4_t av[4];
-      av[0] = __builtin_bit_cast(short4_t, uint2{pack_lo16(rv[0].x, rv[1].x), pack_lo16(rv[2].x, rv[3].x)});
-      av[1] = __builtin_bit_cast(short4_t, uint2{pack_hi16(rv[0].x, rv[1].x), pack_hi16(rv[2].x, rv[3].x)});
-      av[2] = __builtin_bit_cast(short4_t, uint2{pack_lo16(rv[0].y, rv[1].y), pack_lo16(rv[2].y, rv[3].y)});
-      av[3] = __builtin_bit_cast(short4_t, uint2{pack_hi16(rv[0].y, rv[1].y), pack_hi16(rv[2].y, rv[3].y)});
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        acc[j][c] = Mfma<T>::k16(av[c], pb_hi, acc[j][c]);
-        acc[j][c] = Mfma<T>::k16(av[c], pb_lo, acc[j][c]);
-      }
+    for (int b = 0; b < kDim / 16; ++b) {
+      // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
+      const uint32_t at = lds_address(slab + (4 * grp + (col >> 2)) * kRow + 16 * b + 4 * (col & 3));
+      const short4_t av = __builtin_bit_cast(
+          short4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(at))));
+      acc[b] = Mfma<T>::k16(av, pb_hi, acc[b]);
+      acc[b] = Mfma<T>::k16(av, pb_lo, acc[b]);
     }
     if constexpr (PREFETCH) {
       cur = nxt;
@@ -203,27 +193,27 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
   if (col >= G) return;
-  write_decode_result<T>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
+  write_decode_result<T, kDim>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
 }
 
 // The pipelined kernel (decode_split_lds_body) for block sizes that are
 // multiples of 16: K and V tiles go straight from HBM to LDS.
-template <typename T, int STAGES>
+template <typename T, int D, int STAGES>
 __global__ __launch_bounds__(256) void decode_split_lds_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  decode_split_lds_body<T, STAGES>(a, smem, blockIdx.x, blockDim.x >> 6);
+  decode_split_lds_body<T, D, STAGES>(a, smem, blockIdx.x, blockDim.x >> 6);
 }
 
 
 // Blocks [0, R * head_groups): merge split partials of multi-split
 // decode requests, kCombineHeads query heads per block, 32 lanes per head
-// (4 dims each). Up to CAP splits are merged from one round of loads (the
+// (4 dims each; at head_dim 64 and 96 the last lanes only merge statistics). Up to CAP splits are merged from one round of loads (the
 // launch picks CAP >= the layout's split count when it is at most 32).
 // Blocks after that: zero tokens outside every request, kZeroTokens each.
 constexpr int kZeroTokens = 16;
 constexpr int kCombineHeads = 8;
 
-template <typename T, int CAP>
+template <typename T, int D, int CAP>
 __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t head_groups) {
   const int64_t R = a.num_requests;
   const int64_t combine_blocks = R * head_groups;
@@ -259,7 +249,8 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
   // request, and a single split has written its output itself.
   const int2 req = a.decode_req[r];
   const int64_t qs = req.x, ns = req.y;
-  const int d0 = (threadIdx.x & 31) * 4;
+  const bool has_dims = 4 * (threadIdx.x & 31) < D;
+  const int d0 = has_dims ? 4 * (threadIdx.x & 31) : 0;
   if (ns < 0 && a.decode_only) {
     // A request with another query count in a batch whose hint promised
     // single-query requests only: no kernel computes its rows, so they are
@@ -270,7 +261,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
     const uint32_t nan2 = nan_bits | (nan_bits << 16);
     for (int64_t t = q0; t < q1; ++t) {
       uint16_t* op = static_cast<uint16_t*>(a.out) + t * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
-      *reinterpret_cast<uint2*>(op + d0) = uint2{nan2, nan2};
+      if (has_dims) *reinterpret_cast<uint2*>(op + d0) = uint2{nan2, nan2};
     }
     return;
   }
@@ -288,12 +279,12 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
     const int cnt = static_cast<int>(ns);
     float2 ml = make_float2(-INFINITY, 0.f);
     if (sub < cnt) ml = a.ws_ml[first_item + sub * a.num_q_heads];
-    const float* accp = a.ws_acc + first_item * kDim + d0;
+    const float* accp = a.ws_acc + first_item * D + d0;
     float4_t v[CAP];
 #pragma unroll
     for (int j = 0; j < CAP; ++j) {
       const int k = j < cnt ? j : cnt - 1;  // indices past the last split re-read it, unused
-      v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * kDim);
+      v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * D);
     }
     float mx = ml.x;  // lanes past the last split hold -inf and a zero sum
 #pragma unroll
@@ -336,7 +327,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
         sum += w * ml.y;
       }
       const int cnt = ns - s0 < 32 ? static_cast<int>(ns - s0) : 32;
-      const float* accp = a.ws_acc + (first_item + s0 * a.num_q_heads) * kDim + d0;
+      const float* accp = a.ws_acc + (first_item + s0 * a.num_q_heads) * D + d0;
       // Eight splits per pass, their loads issued together (indices past
       // the last split re-read it and are not added).
       for (int k0 = 0; k0 < cnt; k0 += 8) {
@@ -346,7 +337,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
         for (int j = 0; j < 8; ++j) {
           const int k = k0 + j < cnt ? k0 + j : cnt - 1;
           wk[j] = __shfl(w, k, 32);
-          v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * kDim);
+          v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * D);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -360,7 +351,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t
     w[1] = Elem<T>::to_bits(o[2] * inv) | (Elem<T>::to_bits(o[3] * inv) << 16);
   }
   uint16_t* op = static_cast<uint16_t*>(a.out) + qs * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
-  *reinterpret_cast<uint2*>(op + d0) = uint2{w[0], w[1]};
+  if (has_dims) *reinterpret_cast<uint2*>(op + d0) = uint2{w[0], w[1]};
 }
 
 
@@ -378,11 +369,12 @@ DecodeTuning decode_tuning(const AttnArgs& a) {
   DecodeTuning t;
   t.lds_pipeline = a.block_size % 16 == 0 && a.split_tokens <= 2048;
   t.waves = 4;
-  t.stages = 2;
+  t.stages = a.head_dim == 64 ? kStages<64> : a.head_dim == 96 ? kStages<96> : kStages<128>;
   t.prefetch = false;
   t.nontemporal = false;
   if (const char* env = std::getenv("MVLLM_DECODE_KERNEL")) {
-    if (std::strcmp(env, "general") == 0) t.lds_pipeline = false;
+    // The general kernel exists at head_dim 128 only.
+    if (std::strcmp(env, "general") == 0 && a.head_dim == kDim) t.lds_pipeline = false;
   }
   if (const char* env = std::getenv("MVLLM_DECODE_WAVES")) {
     const int v = std::atoi(env);
@@ -390,7 +382,7 @@ DecodeTuning decode_tuning(const AttnArgs& a) {
   }
   if (const char* env = std::getenv("MVLLM_DECODE_STAGES")) {
     const int v = std::atoi(env);
-    if (v >= 2 && v <= 4) t.stages = v;
+    if (v >= 2 && v <= 4 && a.head_dim == kDim) t.stages = v;
   }
   if (const char* env = std::getenv("MVLLM_DECODE_PREFETCH")) t.prefetch = std::atoi(env) != 0;
   if (const char* env = std::getenv("MVLLM_DECODE_NT")) t.nontemporal = std::atoi(env) != 0;
@@ -399,26 +391,26 @@ DecodeTuning decode_tuning(const AttnArgs& a) {
   return t;
 }
 
-template <typename T, int STAGES>
+template <typename T, int D, int STAGES>
 int launch_lds_kernel(const AttnArgs& a, dim3 grid, int waves, hipStream_t s, hipEvent_t start,
                       hipEvent_t stop) {
-  const size_t lds = static_cast<size_t>(waves) * STAGES * 2 * kTileBytes;
+  const size_t lds = static_cast<size_t>(waves) * STAGES * 2 * kTileBytesOf<D>;
   if (lds > 64 * 1024) {
     static bool raised = false;  // per instantiation; the attribute is process-wide
     if (!raised) {
-      MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(decode_split_lds_kernel<T, STAGES>),
+      MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(decode_split_lds_kernel<T, D, STAGES>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(lds)));
       raised = true;
     }
   }
-  hipExtLaunchKernelGGL(decode_split_lds_kernel<T, STAGES>, grid, dim3(64 * waves), lds, s, start, stop,
+  hipExtLaunchKernelGGL((decode_split_lds_kernel<T, D, STAGES>), grid, dim3(64 * waves), lds, s, start, stop,
                         0, a);
   MVLLM_LAUNCH_CHECK("decode_split_lds_kernel");
   return MVLLM_OK;
 }
 
-template <typename T>
+template <typename T, int D>
 int launch_combine_t(const AttnArgs& a, hipStream_t s) {
   const int32_t head_groups = (a.num_q_heads + kCombineHeads - 1) / kCombineHeads;
   const int64_t blocks = a.num_requests * head_groups + (a.num_tokens + kZeroTokens - 1) / kZeroTokens;
@@ -427,15 +419,15 @@ int launch_combine_t(const AttnArgs& a, hipStream_t s) {
     // Short splits on small batches give requests up to ~20 splits; they
     // still merge in one round of loads.
     const dim3 grid(static_cast<unsigned>(blocks)), block(32 * kCombineHeads);
-    if (a.max_splits <= 8) hipLaunchKernelGGL((decode_combine_kernel<T, 8>), grid, block, 0, s, a, head_groups);
-    else if (a.max_splits <= 16) hipLaunchKernelGGL((decode_combine_kernel<T, 16>), grid, block, 0, s, a, head_groups);
-    else hipLaunchKernelGGL((decode_combine_kernel<T, 32>), grid, block, 0, s, a, head_groups);
+    if (a.max_splits <= 8) hipLaunchKernelGGL((decode_combine_kernel<T, D, 8>), grid, block, 0, s, a, head_groups);
+    else if (a.max_splits <= 16) hipLaunchKernelGGL((decode_combine_kernel<T, D, 16>), grid, block, 0, s, a, head_groups);
+    else hipLaunchKernelGGL((decode_combine_kernel<T, D, 32>), grid, block, 0, s, a, head_groups);
     MVLLM_LAUNCH_CHECK("decode_combine_kernel");
   }
   return MVLLM_OK;
 }
 
-template <typename T>
+template <typename T, int D>
 int launch_decode_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
   const DecodeTuning tune = decode_tuning(a);
   const int waves = tune.waves;
@@ -451,11 +443,15 @@ int launch_decode_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent
     }
     const dim3 grid(static_cast<unsigned>(blocks));
     const dim3 block(64 * waves);
-    if (tune.lds_pipeline) {
+    if constexpr (D != kDim) {
+      if (!tune.lds_pipeline)
+        return fail(MVLLM_ERR_UNSUPPORTED, "head_dim %d needs block sizes that are multiples of 16", D);
+      if (int rc = launch_lds_kernel<T, D, kStages<D>>(a, grid, waves, s, start, stop)) return rc;
+    } else if (tune.lds_pipeline) {
       int rc = MVLLM_OK;
-      if (tune.stages == 2) rc = launch_lds_kernel<T, 2>(a, grid, waves, s, start, stop);
-      else if (tune.stages == 3) rc = launch_lds_kernel<T, 3>(a, grid, waves, s, start, stop);
-      else rc = launch_lds_kernel<T, 4>(a, grid, waves, s, start, stop);
+      if (tune.stages == 2) rc = launch_lds_kernel<T, D, 2>(a, grid, waves, s, start, stop);
+      else if (tune.stages == 3) rc = launch_lds_kernel<T, D, 3>(a, grid, waves, s, start, stop);
+      else rc = launch_lds_kernel<T, D, 4>(a, grid, waves, s, start, stop);
       if (rc) return rc;
     } else {
       if (tune.prefetch && tune.nontemporal)
@@ -469,7 +465,22 @@ int launch_decode_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent
       MVLLM_LAUNCH_CHECK("decode_split_kernel");
     }
   }
-  return launch_combine_t<T>(a, s);
+  return launch_combine_t<T, D>(a, s);
+}
+
+// Calls f(T{}, integral_constant D) for the decode kernels' types and head
+// dims; `unsupported` for any other.
+template <typename F>
+int for_decode_types(const AttnArgs& a, int32_t dtype, F&& f) {
+  auto dims = [&](auto t) {
+    if (a.head_dim == 128) return f(t, std::integral_constant<int, 128>{});
+    if (a.head_dim == 96) return f(t, std::integral_constant<int, 96>{});
+    if (a.head_dim == 64) return f(t, std::integral_constant<int, 64>{});
+    return fail(MVLLM_ERR_UNSUPPORTED, "decode kernel needs head_dim 64, 96 or 128");
+  };
+  if (dtype == MVLLM_DTYPE_BF16) return dims(bf16_t{});
+  if (dtype == MVLLM_DTYPE_F16) return dims(f16_t{});
+  return fail(MVLLM_ERR_UNSUPPORTED, "decode kernel needs bf16 or fp16");
 }
 
 }  // namespace
@@ -487,19 +498,22 @@ int launch_decode_lists(const AttnArgs& a, hipStream_t s) {
 
 int launch_decode(const AttnArgs& a, int32_t dtype, hipStream_t s, hipEvent_t start,
                   hipEvent_t stop) {
-  if (a.head_dim != kDim) return fail(MVLLM_ERR_UNSUPPORTED, "decode kernel needs head_dim 128");
-  if (dtype == MVLLM_DTYPE_BF16) return launch_decode_t<bf16_t>(a, s, start, stop);
-  if (dtype == MVLLM_DTYPE_F16) return launch_decode_t<f16_t>(a, s, start, stop);
-  return fail(MVLLM_ERR_UNSUPPORTED, "decode kernel needs bf16 or fp16");
+  return for_decode_types(a, dtype, [&](auto t, auto d) {
+    return launch_decode_t<decltype(t), decltype(d)::value>(a, s, start, stop);
+  });
+}
+
+bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens) {
+  return head_dim == 128 || ((head_dim == 64 || head_dim == 96) && block_size % 16 == 0 && split_tokens <= 2048);
 }
 
 bool decode_step_eligible(const AttnArgs& a) {
-  if (a.head_dim != kDim || a.num_requests <= 0) return false;
+  if (!decode_supported(a.head_dim, a.block_size, a.split_tokens) || a.num_requests <= 0) return false;
   // The default shape only (fewer KV heads than waves: the spare waves of
   // the step's workgroups end at once, as the pipelined kernel's do).
   const DecodeTuning tune = decode_tuning(a);
   const int waves = a.num_kv_heads < kStepDecodeWaves ? a.num_kv_heads : kStepDecodeWaves;
-  return tune.lds_pipeline && tune.waves == waves && tune.stages == 2;
+  return tune.lds_pipeline && tune.waves == waves && (a.head_dim != 128 || tune.stages == kStages<128>);
 }
 
 int64_t decode_step_blocks(const AttnArgs& a) {
@@ -507,9 +521,9 @@ int64_t decode_step_blocks(const AttnArgs& a) {
 }
 
 int launch_decode_combine(const AttnArgs& a, int32_t dtype, hipStream_t s) {
-  if (dtype == MVLLM_DTYPE_BF16) return launch_combine_t<bf16_t>(a, s);
-  if (dtype == MVLLM_DTYPE_F16) return launch_combine_t<f16_t>(a, s);
-  return fail(MVLLM_ERR_UNSUPPORTED, "decode kernel needs bf16 or fp16");
+  return for_decode_types(a, dtype, [&](auto t, auto d) {
+    return launch_combine_t<decltype(t), decltype(d)::value>(a, s);
+  });
 }
 
 }  // namespace mvllm

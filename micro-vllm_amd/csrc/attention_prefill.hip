@@ -1,5 +1,5 @@
 // MFMA prefill / chunked-prefill kernel (requests with more than one query),
-// head_dim 128, bf16/fp16, block sizes that are multiples of 16.
+// head_dim 64, 96 or 128, bf16/fp16, block sizes that are multiples of 16.
 //
 // Work item: (request, block of T query tokens, KV head), one workgroup of
 // four waves. The workgroup's 128 rows are (query head of the KV head's
@@ -60,15 +60,15 @@
 namespace mvllm {
 namespace {
 
-constexpr int kDim = 128;
 constexpr int kTileKeys = 64;
 constexpr int kWaves = 4;
 static_assert(kRows == kWaves * 32, "rows per workgroup");
-constexpr int kTileBytes = kTileKeys * kDim * 2;     // one K (or V) tile: 16 KiB
+template <int D> constexpr int kKeyTileBytes = kTileKeys * D * 2;  // one K (or V) tile: 16 KiB at head_dim 128
 constexpr int kChunkTiles = 256;                     // key tiles whose pages are held in LDS at a time
 constexpr int kTableInts = kChunkTiles * 8;          // per tile and wave: (page entry, tile's valid-page mask)
 constexpr int kDummyBytes = 4096;                    // target of V page loads that are switched off
-constexpr size_t kLdsBytes = 4 * kTileBytes + kTableInts * 4 + 16 * 4 + kDummyBytes;  // K, V double buffers
+template <int D>
+constexpr size_t kLdsBytes = 4 * kKeyTileBytes<D> + kTableInts * 4 + 16 * 4 + kDummyBytes;  // K, V double buffers
 
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -138,18 +138,29 @@ __device__ __forceinline__ int32_t wave_max_i(int32_t v) {
   return wave_reduce_i(v, [](int32_t x, int32_t y) { return x > y ? x : y; });
 }
 
-// LDS byte offset of 16-byte chunk `chunk` of tile row `row` (256-byte rows).
-// The chunk is XOR-swizzled with r ^ ((r & 2) << 2), r = row % 16. Both read
-// patterns are then free of bank conflicts: the K reads (32 rows, one chunk:
-// the swizzle is a bijection of r) and the transposing V reads (8 rows 8u ..
-// 8u + 7, chunks 4c .. 4c + 3: every physical chunk is hit exactly twice).
-__device__ __forceinline__ int tile_swizzle(int row) {
+// Physical 16-byte chunk of logical chunk `chunk` in tile row `row`, a
+// permutation within the row that spreads the read patterns over the banks:
+// the K reads (32 rows, one chunk) and the transposing V reads (8 rows 8u ..
+// 8u + 7, chunks 4c .. 4c + 3). D = 128: XOR with r ^ ((r & 2) << 2),
+// r = row % 16, a bijection of r under which the V reads hit every physical
+// chunk exactly twice. The narrower rows use the decode tiles' permutation.
+template <int D>
+__device__ __forceinline__ int row_phys(int row, int chunk) {
   const int r = row & 15;
-  return r ^ ((r & 2) << 2);
+  if constexpr (D == 128) return chunk ^ (r ^ ((r & 2) << 2));
+  else return dec::tile_phys<D>(r, chunk);
 }
 
+// The logical chunk held by physical chunk `phys` of row `row`.
+template <int D>
+__device__ __forceinline__ int row_logical(int row, int phys) {
+  if constexpr (D == 128) return row_phys<D>(row, phys);  // an XOR is its own inverse
+  else return dec::tile_logical<D>(row & 15, phys);
+}
+
+template <int D>
 __device__ __forceinline__ int tile_off(int row, int chunk) {
-  return row * 256 + ((chunk ^ tile_swizzle(row)) << 4);
+  return row * 2 * D + (row_phys<D>(row, chunk) << 4);
 }
 
 __device__ __forceinline__ float max_with_partner(float x) {
@@ -234,8 +245,19 @@ __device__ __forceinline__ void fill_tile_record(int32_t* tbl, const AttnArgs& a
   rec[1] = int4{e[2], static_cast<int32_t>(mask), e[3], static_cast<int32_t>(mask)};
 }
 
-template <typename T>
+// At head_dim 64 and 96 Q is not rescaled (the scale multiplies the fp32
+// scores) and P enters the P.V product as a hi/lo pair of 16-bit values that
+// keeps ~16 bits of its mantissa, the row sum being taken over the fp32
+// probabilities, as in the decode kernel: these rows' requests have always
+// been answered with fp32 probabilities. The narrower accumulators leave the
+// registers for it.
+template <typename T, int D>
 __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, uint8_t* smem, uint32_t wg) {
+  constexpr int kTileBytes = kKeyTileBytes<D>;
+  constexpr int kPageBytes = kTileBytes / 4;  // 16 rows
+  constexpr int kSteps = D / 16;              // 16-dim MFMA steps of a score
+  constexpr int kBlocks = D / 32;             // 32-dim blocks of O^T; also the 1 KiB loads of a page
+  constexpr bool kSplitP = D != 128;
   uint8_t* const kbuf = smem;                   // K stages 0, 1 (16 KiB each)
   uint8_t* const vbuf = smem + 2 * kTileBytes;  // V stages 0, 1
   int32_t* const page_tbl = reinterpret_cast<int32_t*>(smem + 4 * kTileBytes);
@@ -309,14 +331,18 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   // each multiplied by the softmax scale in the exp2 domain (log2(e) /
   // sqrt(D)) and rounded back to the input type, so the MFMAs produce
   // scaled scores and the softmax needs no multiply.
-  short8_t qv[8];
+  short8_t qv[kSteps];
   {
     const short8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + (row_ok ? tok : t0) * a.q_s0 +
                          static_cast<int64_t>(hq) * a.q_s1 + 8 * hh;
 #pragma unroll
-    for (int st = 0; st < 8; ++st) {
+    for (int st = 0; st < kSteps; ++st) {
       const short8_t raw = row_ok ? *reinterpret_cast<const short8_t*>(qp + 16 * st) : zero;
+      if constexpr (kSplitP) {
+        qv[st] = raw;
+        continue;
+      }
       const uint4 w = __builtin_bit_cast(uint4, raw);
       uint32_t sw[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -345,9 +371,9 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
     kmax = hull_hi;
   }
 
-  float16v oacc[4];
+  float16v oacc[kBlocks];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) oacc[c] = float16v{};
+  for (int c = 0; c < kBlocks; ++c) oacc[c] = float16v{};
   // Softmax state of this lane's row, in the exp2 domain. m_c is the
   // running offset (-inf until the row has seen a visible key); the S MFMAs
   // start from the accumulator value -c_in, so they produce scores already
@@ -358,28 +384,28 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   float16v neg_c = float16v{};
   float l = 0.f;          // this lane's share of the row's softmax sum
 
-  const int64_t head_elems = static_cast<int64_t>(h) * kDim;
+  const int64_t head_elems = static_cast<int64_t>(h) * D;
   const int32_t base = kmax >= kmin ? (kmin & ~15) : 0;
   const int32_t ntiles = kmax >= kmin ? (kmax - base) / kTileKeys + 1 : 0;
 
   // Per-lane LDS byte offsets within a tile.
   // K, A operand of S^T: row n (+ 32 bb), chunk 2 st + hh.
-  int koff[8];
+  int koff[kSteps];
 #pragma unroll
-  for (int st = 0; st < 8; ++st) koff[st] = tile_off(n, 2 * st + hh);
+  for (int st = 0; st < kSteps; ++st) koff[st] = tile_off<D>(n, 2 * st + hh);
   // V, transposing reads for the A operand of O^T (dim block c, keys
   // 8 hh + 4 u .. +4): lane (g = lane / 16, j = lane % 16) points at row
   // 8 u + 4 (g / 2) + j / 4 (+ 32 bb + 16 s2), dims 32 c + 16 (g % 2) + 4 (j % 4).
-  int voff[8];
+  int voff[2 * kBlocks];
   {
     const int g = lane >> 4, jj = lane & 15;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < kBlocks; ++c) {
         const int row = 8 * u + 4 * (g >> 1) + (jj >> 2);
         const int dim = 32 * c + 16 * (g & 1) + 4 * (jj & 3);
-        voff[4 * u + c] = tile_off(row, dim >> 3) + 2 * (dim & 7);
+        voff[kBlocks * u + c] = tile_off<D>(row, dim >> 3) + 2 * (dim & 7);
       }
   }
   // LDS byte addresses from the start of dynamic LDS (the static size): as
@@ -389,9 +415,9 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   const uint32_t kaddr = lds0;
   const uint32_t vaddr = lds0 + 2 * kTileBytes;
   const uint32_t daddr = lds0 + static_cast<uint32_t>(dummy - smem);
-  uint32_t klane[8], vlane[8];
+  uint32_t klane[kSteps], vlane[kSteps];
 #pragma unroll
-  for (int x = 0; x < 8; ++x) {
+  for (int x = 0; x < kSteps; ++x) {
     klane[x] = lds0 + koff[x];
     vlane[x] = lds0 + 2 * kTileBytes + voff[x];
     // Opaque to the compiler, so the sums stay in registers instead of
@@ -399,13 +425,16 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
     asm volatile("" : "+v"(klane[x]), "+v"(vlane[x]));
   }
   // Byte offsets within a 16-row page segment of the page loads: instruction
-  // i covers rows 4 i .. 4 i + 3; lane l lands at row 4 i + l / 16, physical
-  // chunk l % 16, so it fetches the logical chunk that the swizzle puts there.
-  uint32_t dma_off[4];
+  // i covers the page's 16-byte chunks 64 i .. 64 i + 63 (rows 4 i .. 4 i + 3
+  // at head_dim 128); lane l lands at chunk 64 i + l, so it fetches the
+  // logical chunk that the permutation puts there.
+  auto page_row = [&](int i) { return (64 * i + lane) / (D / 8); };
+  uint32_t dma_off[kBlocks];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int rip = 4 * i + (lane >> 4);
-    dma_off[i] = static_cast<uint32_t>(2 * (rip * a.c_s[2] + 8 * ((lane & 15) ^ tile_swizzle(rip))));
+  for (int i = 0; i < kBlocks; ++i) {
+    const int rip = page_row(i);
+    const int phys = (64 * i + lane) % (D / 8);
+    dma_off[i] = static_cast<uint32_t>(2 * (rip * a.c_s[2] + 8 * row_logical<D>(rip, phys)));
   }
   const char* const cache_bytes = static_cast<const char*>(a.cache);
   // Byte strides of a block and of a 16-row group (32-bit: see prefill_supported).
@@ -422,27 +451,27 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
       __syncthreads();
     }
 
-    // Wave w moves page w of each tile into LDS (K and V), four 1 KiB
-    // instructions each. Byte address of the K page segment with entry id:
+    // Wave w moves page w of each tile into LDS (K and V), in 1 KiB
+    // instructions. Byte address of the K page segment with entry id:
     auto page_base = [&](int32_t id) {
       const uint32_t u = static_cast<uint32_t>(id);
       return cache_head + static_cast<uint64_t>(u >> 4) * blk_bytes + (u & 15u) * grp_bytes;
     };
     // Unmapped page (or beyond the last visible key): its V rows are zeroed.
     auto zero_v = [&](int stage) {
-      uint8_t* slot = vbuf + stage * kTileBytes + wave * 4096;
+      uint8_t* slot = vbuf + stage * kTileBytes + wave * kPageBytes;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(slot + i * 1024 + 16 * lane) = uint4{0, 0, 0, 0};
+      for (int i = 0; i < kBlocks; ++i) *reinterpret_cast<uint4*>(slot + i * 1024 + 16 * lane) = uint4{0, 0, 0, 0};
     };
     // After the loads landed: zero the V rows of this wave's page that lie
     // outside [kmin, kmax] (they may hold stale or non-finite data).
     auto fix_v = [&](int32_t tl, int stage) {
       const int32_t pos0 = base + kTileKeys * (c0 + tl) + 16 * wave;
       if (pos0 >= kmin && pos0 + 15 <= kmax) return;
-      uint8_t* slot = vbuf + stage * kTileBytes + wave * 4096;
+      uint8_t* slot = vbuf + stage * kTileBytes + wave * kPageBytes;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int32_t p = pos0 + 4 * i + (lane >> 4);
+      for (int i = 0; i < kBlocks; ++i) {
+        const int32_t p = pos0 + page_row(i);
         if (p < kmin || p > kmax) *reinterpret_cast<uint4*>(slot + i * 1024 + 16 * lane) = uint4{0, 0, 0, 0};
       }
     };
@@ -484,8 +513,8 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
       if (tl + 1 < nt && nid < 0) zero_v(stage ^ 1);
       const char* const kp = page_base(nid >= 0 ? nid : 0);
       const char* const vp = kp + 2 * a.c_s[0];
-      const uint32_t kdst = kaddr + (stage ^ 1) * kTileBytes + wave * 4096;
-      const uint32_t vdst = nid >= 0 ? vaddr + (stage ^ 1) * kTileBytes + wave * 4096 : daddr;
+      const uint32_t kdst = kaddr + (stage ^ 1) * kTileBytes + wave * kPageBytes;
+      const uint32_t vdst = nid >= 0 ? vaddr + (stage ^ 1) * kTileBytes + wave * kPageBytes : daddr;
       const int2 fut_rec = tile_rec(tl + 2);
 
       // The tile as two halves of 32 keys, each a full online-softmax
@@ -499,25 +528,19 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         const int32_t k0 = half_k0(bb);
         return k0 < w_lo_max || k0 + 31 > w_hi_min || half_pages(bb) != 3u;
       };
-      auto read_k = [&](int bb, short8_t (&kf)[8]) {
+      auto read_k = [&](int bb, short8_t (&kf)[kSteps]) {
 #pragma unroll
-        for (int st = 0; st < 8; ++st) kf[st] = lds_read_b128_at(klane[st] + stage * kTileBytes + 8192 * bb);
-      };
-      // V operands of both 16-key steps of half bb (transposing reads).
-      auto read_v = [&](int bb, short4v (&vf)[2][8]) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-          for (int x = 0; x < 8; ++x) vf[q][x] = lds_read_tr16_at(vlane[x] + stage * kTileBytes + 8192 * bb + 4096 * q);
+        for (int st = 0; st < kSteps; ++st)
+          kf[st] = lds_read_b128_at(klane[st] + stage * kTileBytes + 2 * kPageBytes * bb);
       };
       // S^T of half bb from the K fragments, starting at `init` (-c_in), with
       // the loads of tile tl + 1 between the MFMAs: K pages with half 0, V
       // pages with half 1. PIN places each load after its MFMA pair.
-      auto s_chain = [&](int bb, const short8_t (&kf)[8], float16v init, auto pin_c) {
+      auto s_chain = [&](int bb, const short8_t (&kf)[kSteps], float16v init, auto pin_c) {
         constexpr bool PIN = decltype(pin_c)::value;
-        float16v s = init;
+        float16v s = kSplitP ? float16v{} : init;
 #pragma unroll
-        for (int st = 0; st < 8; ++st) {
+        for (int st = 0; st < kSteps; ++st) {
           s = Mma32<T>::mma(kf[st], qv[st], s);
           if (st & 1) {
             const int i = st >> 1;
@@ -525,6 +548,10 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
             page_load(bb == 0 ? kp : vp, i, dma_off[i], bb == 0 ? kdst : vdst);
             if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
           }
+        }
+        if constexpr (kSplitP) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], a.scale_log2, -c_in);
         }
         return s;
       };
@@ -545,21 +572,27 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
           s[i] = vis ? s[i] : -INFINITY;
         }
       };
+      // P^T of a half's two 16-key steps as MFMA B operands (lo: kSplitP only).
+      struct PBits {
+        short8_t hi[2], lo[2];
+      };
       // O^T += V^T . P^T over a half's two 16-key steps.
-      auto pv_mma = [&](const short4v (&vf)[2][8], const short8_t (&pb)[2]) {
+      auto pv_mma = [&](const short4v (&vf)[2][kSteps], const PBits& pb) {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const short4v lo4 = vf[q][c], hi4 = vf[q][4 + c];
+          for (int c = 0; c < kBlocks; ++c) {
+            const short4v lo4 = vf[q][c], hi4 = vf[q][kBlocks + c];
             const short8_t av = short8_t{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
-            oacc[c] = Mma32<T>::mma(av, pb[q], oacc[c]);
+            oacc[c] = Mma32<T>::mma(av, pb.hi[q], oacc[c]);
+            if constexpr (kSplitP) oacc[c] = Mma32<T>::mma(av, pb.lo[q], oacc[c]);
           }
       };
       // Probabilities exp2(s + shift) (P^T B operands in pb), the add
       // skipped for SHIFTED false; returns this lane's share of their row
-      // sum, taken over the rounded values the P.V product uses.
-      auto make_p = [&](const float16v& s, float shift, auto shifted_c, short8_t (&pb)[2]) {
+      // sum, taken over the rounded values the P.V product uses (the fp32
+      // values where the product takes them as pairs).
+      auto make_p = [&](const float16v& s, float shift, auto shifted_c, PBits& pb) {
         constexpr bool SHIFTED = decltype(shifted_c)::value;
         float inc = 0.f;
         float p[16];
@@ -570,20 +603,28 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           // P^T B operand: keys 16 s2 + 8 u + 4 hh + e  <->  k = 8 hh + 4 u + e.
-          uint32_t ph[4];
+          uint32_t ph[4], pl[4];
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
-            ph[w] = Mma32<T>::pack2(p[8 * s2 + 2 * w], p[8 * s2 + 2 * w + 1]);
-            inc = Mma32<T>::dot2_ones(ph[w], inc);
+            const float p0 = p[8 * s2 + 2 * w], p1 = p[8 * s2 + 2 * w + 1];
+            ph[w] = Mma32<T>::pack2(p0, p1);
+            if constexpr (kSplitP) {
+              const float2v r = Mma32<T>::unpack2(ph[w]);
+              pl[w] = Mma32<T>::pack2(p0 - r[0], p1 - r[1]);
+              inc += p0 + p1;
+            } else {
+              inc = Mma32<T>::dot2_ones(ph[w], inc);
+            }
           }
-          pb[s2] = __builtin_bit_cast(short8_t, uint4{ph[0], ph[1], ph[2], ph[3]});
+          pb.hi[s2] = __builtin_bit_cast(short8_t, uint4{ph[0], ph[1], ph[2], ph[3]});
+          if constexpr (kSplitP) pb.lo[s2] = __builtin_bit_cast(short8_t, uint4{pl[0], pl[1], pl[2], pl[3]});
         }
         return inc;
       };
       // From the half's row maximum: a new offset when the maximum grew by
       // more than 2^8 over the current one (the accumulators and the sum
       // rescaled), then the probabilities against it; c_in follows.
-      auto softmax_slow = [&](float16v& s, short8_t (&pb)[2]) {
+      auto softmax_slow = [&](float16v& s, PBits& pb) {
         float mx = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
@@ -595,7 +636,7 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
           const float alpha = grow ? __builtin_amdgcn_exp2f(m_c - m_new) : 1.f;
           l *= alpha;
 #pragma unroll
-          for (int c = 0; c < 4; ++c) oacc[c] *= alpha;
+          for (int c = 0; c < kBlocks; ++c) oacc[c] *= alpha;
           m_c = m_new;
         }
         const float m_eff = m_c == -INFINITY ? 0.f : m_c;
@@ -610,7 +651,7 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
       // probabilities summing to at most 2^12 keep each below 2^12, which
       // bf16 and fp16 P and the accumulators hold; otherwise (a maximum that
       // grew, an unset offset, NaN) the half is redone from its maximum.
-      auto softmax_with = [&](float16v& s, short8_t (&pb)[2], auto&& work) {
+      auto softmax_with = [&](float16v& s, PBits& pb, auto&& work) {
         work();
         // Speculative: the probabilities are formed in the same block as
         // `work`, and kept only when every lane has an offset.
@@ -621,14 +662,15 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
       };
 
       // V operands of one 16-key step of half bb.
-      auto read_v1 = [&](int bb, int q, short4v (&vq)[8]) {
+      auto read_v1 = [&](int bb, int q, short4v (&vq)[kSteps]) {
 #pragma unroll
-        for (int x = 0; x < 8; ++x) vq[x] = lds_read_tr16_at(vlane[x] + stage * kTileBytes + 8192 * bb + 4096 * q);
+        for (int x = 0; x < kSteps; ++x)
+          vq[x] = lds_read_tr16_at(vlane[x] + stage * kTileBytes + 2 * kPageBytes * bb + kPageBytes * q);
       };
-      short4v vf[2][8];
+      short4v vf[2][kSteps];
       float16v s0, s1;
       {
-        short8_t kf[8];
+        short8_t kf[kSteps];
         read_k(0, kf);
         __builtin_amdgcn_sched_barrier(0);
         s0 = s_chain(0, kf, neg_c, std::true_type{});
@@ -641,11 +683,11 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         asm volatile("");
         mask(0, s0);
       }
-      short8_t pb0[2];
+      PBits pb0;
       l += softmax_with(s0, pb0, [] {});
       __builtin_amdgcn_sched_barrier(0);
       {
-        short8_t kf[8];
+        short8_t kf[kSteps];
         read_k(1, kf);
         __builtin_amdgcn_sched_barrier(0);
         s1 = s_chain(1, kf, neg_c, std::true_type{});
@@ -657,7 +699,7 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         mask(1, s1);
       }
       // softmax(1) beside P.V(0).
-      short8_t pb1[2];
+      PBits pb1;
       l += softmax_with(s1, pb1, [&] { pv_mma(vf, pb0); });
       __builtin_amdgcn_sched_barrier(0);
       read_v1(1, 0, vf[0]);
@@ -680,9 +722,9 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         zero_v(0);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          lds_dma_load16_sbase(kp, dma_off[i], kaddr + wave * 4096 + i * 1024);
-          lds_dma_load16_sbase(kp + 2 * a.c_s[0], dma_off[i], vaddr + wave * 4096 + i * 1024);
+        for (int i = 0; i < kBlocks; ++i) {
+          lds_dma_load16_sbase(kp, dma_off[i], kaddr + wave * kPageBytes + i * 1024);
+          lds_dma_load16_sbase(kp + 2 * a.c_s[0], dma_off[i], vaddr + wave * kPageBytes + i * 1024);
         }
       }
     }
@@ -705,7 +747,7 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   const float inv = nonempty ? 1.f / lt : NAN;  // an empty visible range is NaN, as in the reference
   uint16_t* op = static_cast<uint16_t*>(a.out) + tok * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < kBlocks; ++c)
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       uint32_t w[2][2];  // [q - 2 p][word]
@@ -729,32 +771,36 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
     }
 }
 
-template <typename T>
+template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void prefill_kernel(AttnArgs a, int32_t lg_tok) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  prefill_body<T>(a, lg_tok, smem, blockIdx.x);
+  prefill_body<T, D>(a, lg_tok, smem, blockIdx.x);
 }
 
 // The one-launch attention step: the decode and prefill workgroups of a
 // forward in one grid. The first `first` workgroups run one kind (the
 // prefill ones when `prefill_first`), the rest the other, each indexing its
 // own work list exactly as in its own kernel. A CU holds two workgroups of
-// either kind (the launch reserves the prefill kernel's LDS, which covers
-// the decode kernel's four waves of two K/V stages), so the grid needs no
-// second stream to run prefill beside decode, and a batch without prefill
-// work pays only for the prefill workgroups that find an empty record.
-static_assert(kStepDecodeWaves * 2 * 2 * dec::kTileBytes <= kLdsBytes,
-              "the step kernel's LDS must hold the decode kernel's tiles");
+// either kind (the launch reserves the larger of the two kernels' LDS), so
+// the grid needs no second stream to run prefill beside decode, and a batch
+// without prefill work pays only for the prefill workgroups that find an
+// empty record.
+template <int D>
+constexpr size_t kStepLdsBytes = kLdsBytes<D> > size_t{kStepDecodeWaves} * dec::kStages<D> * 2 * dec::kTileBytesOf<D>
+                                     ? kLdsBytes<D>
+                                     : size_t{kStepDecodeWaves} * dec::kStages<D> * 2 * dec::kTileBytesOf<D>;
+static_assert(kStepLdsBytes<128> <= 80 * 1024 && kStepLdsBytes<96> <= 80 * 1024 && kStepLdsBytes<64> <= 80 * 1024,
+              "two step workgroups share a CU's LDS");
 
-template <typename T>
+template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void attention_step_kernel(AttnArgs a, int32_t lg_tok, uint32_t first,
                                                                int32_t prefill_first) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t b = blockIdx.x;
   const bool lead = b < first;
   const uint32_t wg = lead ? b : b - first;
-  if (lead == (prefill_first != 0)) prefill_body<T>(a, lg_tok, smem, wg);
-  else dec::decode_split_lds_body<T, 2>(a, smem, wg, kStepDecodeWaves);
+  if (lead == (prefill_first != 0)) prefill_body<T, D>(a, lg_tok, smem, wg);
+  else dec::decode_split_lds_body<T, D, dec::kStages<D>>(a, smem, wg, kStepDecodeWaves);
 }
 
 __global__ __launch_bounds__(kItemThreads) void prefill_items_kernel(AttnArgs a, int32_t lg_tok) {
@@ -762,7 +808,7 @@ __global__ __launch_bounds__(kItemThreads) void prefill_items_kernel(AttnArgs a,
 }
 
 
-template <typename T>
+template <typename T, int D>
 int launch_prefill_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
   const int lg_tok = prefill_lg_tok(a);
   const int64_t nblk = a.num_tokens / (int64_t{1} << lg_tok) + a.num_requests;
@@ -776,18 +822,18 @@ int launch_prefill_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEven
   }
   static bool raised = false;  // per instantiation; the attribute is process-wide
   if (!raised) {
-    MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_kernel<T>),
+    MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_kernel<T, D>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(kLdsBytes)));
+                                      static_cast<int>(kLdsBytes<D>)));
     raised = true;
   }
-  hipExtLaunchKernelGGL(prefill_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(256),
-                        kLdsBytes, s, start, stop, 0, a, lg_tok);
+  hipExtLaunchKernelGGL((prefill_kernel<T, D>), dim3(static_cast<unsigned>(blocks)), dim3(256),
+                        kLdsBytes<D>, s, start, stop, 0, a, lg_tok);
   MVLLM_LAUNCH_CHECK("prefill_kernel");
   return MVLLM_OK;
 }
 
-template <typename T>
+template <typename T, int D>
 int launch_step_t(const AttnArgs& a, bool prefill_first, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
   const int lg_tok = prefill_lg_tok(a);
   const int64_t prefill_blocks = (a.num_tokens / (int64_t{1} << lg_tok) + a.num_requests) * a.num_kv_heads;
@@ -804,16 +850,28 @@ int launch_step_t(const AttnArgs& a, bool prefill_first, hipStream_t s, hipEvent
   }
   static bool raised = false;  // per instantiation; the attribute is process-wide
   if (!raised) {
-    MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_step_kernel<T>),
+    MVLLM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_step_kernel<T, D>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(kLdsBytes)));
+                                      static_cast<int>(kStepLdsBytes<D>)));
     raised = true;
   }
-  hipExtLaunchKernelGGL(attention_step_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(256),
-                        kLdsBytes, s, start, stop, 0, a, lg_tok, static_cast<uint32_t>(first),
+  hipExtLaunchKernelGGL((attention_step_kernel<T, D>), dim3(static_cast<unsigned>(blocks)), dim3(256),
+                        kStepLdsBytes<D>, s, start, stop, 0, a, lg_tok, static_cast<uint32_t>(first),
                         prefill_first ? 1 : 0);
   MVLLM_LAUNCH_CHECK("attention_step_kernel");
   return MVLLM_OK;
+}
+
+// Calls f(T{}, integral_constant D) for a type and head dim that
+// prefill_supported has accepted.
+template <typename F>
+int for_prefill_types(const AttnArgs& a, int32_t dtype, F&& f) {
+  auto dims = [&](auto t) {
+    if (a.head_dim == 64) return f(t, std::integral_constant<int, 64>{});
+    if (a.head_dim == 96) return f(t, std::integral_constant<int, 96>{});
+    return f(t, std::integral_constant<int, 128>{});
+  };
+  return dtype == MVLLM_DTYPE_BF16 ? dims(bf16_t{}) : dims(f16_t{});
 }
 
 }  // namespace
@@ -831,7 +889,7 @@ int launch_prefill_lists(const AttnArgs& a, hipStream_t s) {
 
 bool prefill_supported(const AttnArgs& a, int32_t dtype) {
   if (dtype != MVLLM_DTYPE_BF16 && dtype != MVLLM_DTYPE_F16) return false;
-  if (a.head_dim != kDim || a.block_size % 16 != 0) return false;
+  if ((a.head_dim != 64 && a.head_dim != 96 && a.head_dim != 128) || a.block_size % 16 != 0) return false;
   const int g = a.group;
   if (g != 1 && g != 2 && g != 4 && g != 8 && g != 16) return false;
   // Key positions and block ids are carried as int32 inside the kernel.
@@ -847,10 +905,11 @@ int launch_prefill(const AttnArgs& a, int32_t dtype, hipStream_t s, hipEvent_t s
                    hipEvent_t stop) {
   if (!prefill_supported(a, dtype))
     return fail(MVLLM_ERR_UNSUPPORTED, "prefill kernel does not support this geometry");
-  // P is kept in the input type, as the reference's Triton kernel keeps it
-  // (triton_paged.py:271-277).
-  if (dtype == MVLLM_DTYPE_BF16) return launch_prefill_t<bf16_t>(a, s, start, stop);
-  return launch_prefill_t<f16_t>(a, s, start, stop);
+  // At head_dim 128 P is kept in the input type, as the reference's Triton
+  // kernel keeps it (triton_paged.py:271-277).
+  return for_prefill_types(a, dtype, [&](auto t, auto d) {
+    return launch_prefill_t<decltype(t), decltype(d)::value>(a, s, start, stop);
+  });
 }
 
 int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_t s, hipEvent_t start,
@@ -859,9 +918,10 @@ int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_
     return fail(MVLLM_ERR_UNSUPPORTED, "the attention step kernel does not support this geometry");
   if (a.width * a.block_size > INT32_MAX || a.num_tokens > INT32_MAX)
     return fail(MVLLM_ERR_UNSUPPORTED, "decode positions beyond 2^31 are not supported");
-  int rc = dtype == MVLLM_DTYPE_BF16 ? launch_step_t<bf16_t>(a, prefill_first, s, start, stop)
-                                     : launch_step_t<f16_t>(a, prefill_first, s, start, stop);
-  if (rc) return rc;
+  if (int rc = for_prefill_types(a, dtype, [&](auto t, auto d) {
+        return launch_step_t<decltype(t), decltype(d)::value>(a, prefill_first, s, start, stop);
+      }))
+    return rc;
   return launch_decode_combine(a, dtype, s);
 }
 

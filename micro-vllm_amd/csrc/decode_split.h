@@ -7,11 +7,11 @@
 // owns one KV head; a workgroup holds `waves` consecutive KV heads of the
 // same (request, split), so together they stream whole token rows (all heads
 // of a token are contiguous in the cache). Per 16-token tile a wave computes
-// S^T = K . Q^T with four v_mfma_f32_16x16x32 (M = 16 tokens, N = the G query
-// heads of the KV head, padded to 16, K = 128 dims); the softmax runs on the
-// accumulator layout, and P^T is the B operand of O^T += V^T . P^T
-// (v_mfma_f32_16x16x16), fed as a hi/lo pair so the product keeps ~16
-// mantissa bits.
+// S^T = K . Q^T with v_mfma_f32_16x16x32 (M = 16 tokens, N = the G query heads
+// of the KV head, padded to 16, K = head_dim: 64, 96 or 128); the softmax runs
+// on the accumulator layout, and P^T is the B operand of O^T += V^T . P^T
+// (v_mfma_f32_16x16x16), fed as a hi/lo pair so the product keeps ~16 mantissa
+// bits; the V^T operand comes from transposing LDS reads (ds_read_b64_tr_b16).
 #pragma once
 
 #include <cmath>
@@ -21,7 +21,6 @@
 namespace mvllm {
 namespace {
 namespace dec {
-constexpr int kDim = 128;
 
 template <typename T>
 __device__ __forceinline__ void split_hi_lo(float p, uint32_t& hi, uint32_t& lo) {
@@ -29,74 +28,102 @@ __device__ __forceinline__ void split_hi_lo(float p, uint32_t& hi, uint32_t& lo)
   lo = Elem<T>::to_bits(p - Elem<T>::from_bits(hi));
 }
 
-// Epilogue shared by the decode kernels. acc[j][c][e] is
-// O[head hq][dim 64j + 16grp + 4e + c] (unnormalised), m / lt the running
+// Epilogue shared by the decode kernels. acc[b][e] is
+// O[head hq][dim 16b + 4grp + e] (unnormalised), m / lt the running
 // max (exp2 domain) and the complete softmax denominator of this split. A
 // request with one split gets its output directly; otherwise the partial goes
 // to the workspace for the combine kernel.
-template <typename T>
+template <typename T, int D>
 __device__ __forceinline__ void write_decode_result(const AttnArgs& a, int64_t r, int64_t qs, int hq,
                                                     int split, int64_t ns, float m, float lt,
-                                                    const float4_t (&acc)[2][4], int grp) {
+                                                    const float4_t (&acc)[D / 16], int grp) {
   if (ns == 1) {
     const float inv = 1.f / lt;
     uint16_t* op = static_cast<uint16_t*>(a.out) + qs * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      uint32_t w[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int i0 = 2 * i, i1 = 2 * i + 1;
-        w[i] = Elem<T>::to_bits(acc[j][i0 & 3][i0 >> 2] * inv) |
-               (Elem<T>::to_bits(acc[j][i1 & 3][i1 >> 2] * inv) << 16);
-      }
-      uint4* dst = reinterpret_cast<uint4*>(op + 64 * j + 16 * grp);
-      dst[0] = uint4{w[0], w[1], w[2], w[3]};
-      dst[1] = uint4{w[4], w[5], w[6], w[7]};
+    for (int b = 0; b < D / 16; ++b) {
+      const uint32_t w0 = Elem<T>::to_bits(acc[b][0] * inv) | (Elem<T>::to_bits(acc[b][1] * inv) << 16);
+      const uint32_t w1 = Elem<T>::to_bits(acc[b][2] * inv) | (Elem<T>::to_bits(acc[b][3] * inv) << 16);
+      *reinterpret_cast<uint2*>(op + 16 * b + 4 * grp) = uint2{w0, w1};
     }
     return;
   }
   const int64_t item = (r * a.max_splits + split) * a.num_q_heads + hq;
-  float* wp = a.ws_acc + item * kDim;
+  float* wp = a.ws_acc + item * D;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    float4_t* dst = reinterpret_cast<float4_t*>(wp + 64 * j + 16 * grp);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      dst[e] = float4_t{acc[j][0][e], acc[j][1][e], acc[j][2][e], acc[j][3][e]};
-  }
+  for (int b = 0; b < D / 16; ++b) *reinterpret_cast<float4_t*>(wp + 16 * b + 4 * grp) = acc[b];
   if (grp == 0) a.ws_ml[item] = float2{m, lt};
 }
 
 // ---------------------------------------------------------------------------
 // Pipelined variant for block sizes that are multiples of 16 (every 16-token
 // tile then lies in one block). K and V tiles go straight from HBM to LDS
-// (global_load_lds_dwordx4): each load instruction covers 4 tokens x 256 B,
-// i.e. whole 128-byte lines. Tile slot (token t, 16-byte chunk q) lives at
-// LDS chunk 16t + (q ^ swz(t)) with swz(t) = t ^ ((t & 4) << 1), which keeps
-// 8 consecutive lanes inside one line on the global side and makes both LDS
-// read patterns (K rows as MFMA A operands, V columns for V^T) free of bank
-// conflicts. STAGES tiles per wave are in flight; waits are explicit vmcnt
-// counts because the only vector-memory instructions in the loop are these
-// tile loads (the split's block ids are fetched once, up front). The loads
-// carry the non-temporal hint: every K/V byte is read exactly once, and
-// keeping the stream from displacing other cached lines raised the measured
-// bandwidth from 5.5 to 6.0 TB/s on the Qwen3 decode batch.
+// (global_load_lds_dwordx4): each load instruction covers 1 KiB of whole rows
+// (4 tokens of 256 B at head_dim 128, 8 of 128 B at 64), i.e. whole 128-byte
+// lines, except at head_dim 96 whose 192-byte rows share them. tile_phys gives
+// the 16-byte chunk of a row in which a tile's logical chunk lies; it is a
+// permutation within the row, so the lanes of a load stay inside the same
+// lines on the global side, and it spreads both LDS read patterns over the
+// banks: the K rows as MFMA A operands (16 rows, one chunk) and the
+// transposing V reads (8 rows, two neighbouring chunks). STAGES tiles per wave
+// are in flight; waits are explicit vmcnt counts because the only
+// vector-memory instructions in the loop are these tile loads (the split's
+// block ids are fetched once, up front). The loads carry the non-temporal
+// hint: every K/V byte is read exactly once, and keeping the stream from
+// displacing other cached lines raised the measured bandwidth from 5.5 to
+// 6.0 TB/s on the Qwen3 decode batch.
 
-constexpr int kTileBytes = 16 * 256;  // one 16-token tile of one head, K or V
+template <int D> constexpr int kTileBytesOf = 16 * 2 * D;  // one 16-token tile of one head, K or V
 
-__device__ __forceinline__ int tile_swizzle(int t) { return t ^ ((t & 4) << 1); }
+// Tiles in flight per wave: 32 KiB of K and V per wave for the narrow heads
+// too, whose tiles are smaller (two workgroups of four waves share a CU's LDS).
+template <int D> constexpr int kStages = D == 64 ? 4 : D == 96 ? 3 : 2;
 
-__device__ __forceinline__ void wait_vmcnt_dyn(int n) {
-  // n is wave-uniform; 8 loads per tile in flight, at most 3 tiles ahead.
-  if (n >= 24) wait_vmcnt<24>();
-  else if (n >= 16) wait_vmcnt<16>();
-  else if (n >= 8) wait_vmcnt<8>();
+// Physical 16-byte chunk of logical chunk q in row t (t < 16) of a tile.
+// D = 128 (16 chunks, one bank row): XOR with t rotated left by one bit.
+// D = 64 (8 chunks, two rows per bank row): XOR with the bit-reversed t / 2.
+// D = 96 (12 chunks; row starts fall on four bank offsets): rotated by t / 4.
+template <int D>
+__device__ __forceinline__ int tile_phys(int t, int q) {
+  if constexpr (D == 128) {
+    return q ^ (((t << 1) | (t >> 3)) & 15);
+  } else if constexpr (D == 64) {
+    const int u = (t >> 1) & 7;
+    return q ^ (((u & 1) << 2) | (u & 2) | (u >> 2));
+  } else {
+    const int x = q + (t >> 2);
+    return x >= 12 ? x - 12 : x;
+  }
+}
+
+// The logical chunk held by physical chunk p of row t.
+template <int D>
+__device__ __forceinline__ int tile_logical(int t, int p) {
+  if constexpr (D == 96) {
+    const int x = p - (t >> 2);
+    return x < 0 ? x + 12 : x;
+  } else {
+    return tile_phys<D>(t, p);  // an XOR is its own inverse
+  }
+}
+
+// Waits until at most `tiles` tiles of LOADS loads each are outstanding
+// (wave-uniform, at most 3).
+template <int LOADS>
+__device__ __forceinline__ void wait_tiles(int tiles) {
+  if (tiles >= 3) wait_vmcnt<3 * LOADS>();
+  else if (tiles == 2) wait_vmcnt<2 * LOADS>();
+  else if (tiles == 1) wait_vmcnt<LOADS>();
   else wait_vmcnt<0>();
 }
 
-template <typename T, int STAGES>
+typedef short tr_short4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) tr_short4 lds_tr_short4;
+
+template <typename T, int D, int STAGES>
 __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t* smem, uint32_t wg, int waves) {
+  constexpr int kTileBytes = kTileBytesOf<D>;
+  constexpr int kLoads = D / 32;  // 1 KiB loads per K (or V) tile
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;
@@ -145,28 +172,39 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
 
   const int G = a.group;
   const int hq = h * G + col;
-  short8_t qv[4];
+  short8_t qv[kLoads];
   {
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + qs * a.q_s0 +
                          static_cast<int64_t>(col < G ? hq : 0) * a.q_s1 + 8 * grp;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kLoads; ++i)
       qv[i] = (col < G) ? *reinterpret_cast<const short8_t*>(qp + 32 * i) : short8_t{0, 0, 0, 0, 0, 0, 0, 0};
   }
 
   uint8_t* wave_lds = smem + static_cast<size_t>(wave) * STAGES * 2 * kTileBytes;
   const uint32_t wave_lds_addr = lds_address(wave_lds);
   const uint16_t* cache = static_cast<const uint16_t*>(a.cache);
-  const int64_t head_elems = static_cast<int64_t>(h) * kDim;
+  const int64_t head_elems = static_cast<int64_t>(h) * D;
 
-  // Load-side mapping: instruction i, this lane -> token 4i + lane/16 of the
-  // tile, 16-byte chunk q (element offset from the tile's first row).
-  int64_t lane_off[4];
+  // Load-side mapping: instruction i, this lane -> 16-byte chunk 64i + lane of
+  // the tile's LDS slot (element offset of its data from the tile's first row).
+  int64_t lane_off[kLoads];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int t = 4 * i + (lane >> 4);
-    const int q = (lane & 15) ^ tile_swizzle(t);
-    lane_off[i] = t * a.c_s[2] + 8 * q;
+  for (int i = 0; i < kLoads; ++i) {
+    const int t = (64 * i + lane) / (D / 8);
+    const int p = (64 * i + lane) % (D / 8);
+    lane_off[i] = t * a.c_s[2] + 8 * tile_logical<D>(t, p);
+  }
+  // Read-side byte offsets within a tile: K row `col`, chunk 4i + grp; and the
+  // transposing V reads, in which lane 4k + c of a 16-lane group points at row
+  // 4grp + k, dims 16b + 4c .. +4.
+  int koff[kLoads], voff[D / 16];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) koff[i] = 2 * D * col + 16 * tile_phys<D>(col, 4 * i + grp);
+#pragma unroll
+  for (int b = 0; b < D / 16; ++b) {
+    const int t = 4 * grp + (col >> 2);
+    voff[b] = 2 * D * t + 16 * tile_phys<D>(t, 2 * b + ((col & 3) >> 1)) + 8 * (col & 1);
   }
 
   auto issue = [&](int tile, int stage) {
@@ -180,18 +218,16 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
                                       : cache;
     const int64_t plane = blk >= 0 ? a.c_s[0] : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
       const uint16_t* src = blk >= 0 ? tile_k + lane_off[i] : cache;
       lds_dma_load16_stream(src, kdst + i * 1024);
       lds_dma_load16_stream(src + plane, vdst + i * 1024);
     }
   };
 
-  float4_t acc[2][4];
+  float4_t acc[D / 16];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[j][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < D / 16; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
   // The block ids and Q must be in registers before the first tile address.
@@ -210,7 +246,7 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
       issue(ahead, ahead % STAGES);
     }
     const int later = (ntiles - 1 - k) < (STAGES - 1) ? (ntiles - 1 - k) : (STAGES - 1);
-    wait_vmcnt_dyn(8 * later);
+    wait_tiles<2 * kLoads>(later);
     __builtin_amdgcn_wave_barrier();
     compiler_fence();
 
@@ -224,13 +260,12 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
       okmask = (last_ok >= first_ok) ? ((0xFFFFu >> (15 - last_ok)) & (0xFFFFu << first_ok)) : 0u;
     }
     const uint8_t* kt = wave_lds + stage * 2 * kTileBytes;
-    const uint8_t* vt = kt + kTileBytes;
+    const uint32_t vt = wave_lds_addr + stage * 2 * kTileBytes + kTileBytes;
 
     float4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const short8_t kk = *reinterpret_cast<const short8_t*>(
-          kt + 16 * (16 * col + ((4 * i + grp) ^ tile_swizzle(col))));
+    for (int i = 0; i < kLoads; ++i) {
+      const short8_t kk = *reinterpret_cast<const short8_t*>(kt + koff[i]);
       sc = Mfma<T>::k32(kk, qv[i], sc);
     }
     float s[4];
@@ -247,9 +282,7 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
     l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     if (__ballot(alpha != 1.f)) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[j][c] *= alpha;
+      for (int b = 0; b < D / 16; ++b) acc[b] *= alpha;
     }
     m = mn;
 
@@ -262,24 +295,13 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
     const uint32_t mlo = ((okmask >> (4 * grp)) & 1u ? 0xFFFFu : 0u) | ((okmask >> (4 * grp + 1)) & 1u ? 0xFFFF0000u : 0u);
     const uint32_t mhi = ((okmask >> (4 * grp + 2)) & 1u ? 0xFFFFu : 0u) | ((okmask >> (4 * grp + 3)) & 1u ? 0xFFFF0000u : 0u);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      uint2 rv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 4 * grp + e;
-        const int q = 8 * j + (col >> 1);
-        rv[e] = *reinterpret_cast<const uint2*>(vt + 16 * (16 * t + (q ^ tile_swizzle(t))) + 8 * (col & 1));
-      }
-      short4_t av[4];
-      av[0] = __builtin_bit_cast(short4_t, uint2{pack_lo16(rv[0].x, rv[1].x) & mlo, pack_lo16(rv[2].x, rv[3].x) & mhi});
-      av[1] = __builtin_bit_cast(short4_t, uint2{pack_hi16(rv[0].x, rv[1].x) & mlo, pack_hi16(rv[2].x, rv[3].x) & mhi});
-      av[2] = __builtin_bit_cast(short4_t, uint2{pack_lo16(rv[0].y, rv[1].y) & mlo, pack_lo16(rv[2].y, rv[3].y) & mhi});
-      av[3] = __builtin_bit_cast(short4_t, uint2{pack_hi16(rv[0].y, rv[1].y) & mlo, pack_hi16(rv[2].y, rv[3].y) & mhi});
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        acc[j][c] = Mfma<T>::k16(av[c], pb_hi, acc[j][c]);
-        acc[j][c] = Mfma<T>::k16(av[c], pb_lo, acc[j][c]);
-      }
+    for (int b = 0; b < D / 16; ++b) {
+      // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
+      const uint2 rv = __builtin_bit_cast(
+          uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(vt + voff[b]))));
+      const short4_t av = __builtin_bit_cast(short4_t, uint2{rv.x & mlo, rv.y & mhi});
+      acc[b] = Mfma<T>::k16(av, pb_hi, acc[b]);
+      acc[b] = Mfma<T>::k16(av, pb_lo, acc[b]);
     }
     // All LDS reads of this stage must retire before a later issue refills it.
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -288,7 +310,7 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
   if (col >= G) return;
-  write_decode_result<T>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
+  write_decode_result<T, D>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
 }
 
 }  // namespace dec
