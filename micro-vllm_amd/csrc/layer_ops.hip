@@ -542,33 +542,86 @@ struct ArgmaxLane {
 
 __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// One workgroup per row: 16-byte loads, four in flight per lane, then a
-// 64-bit maximum over the workgroup.
+// max(a, b, c) in one instruction; a NaN operand is passed over.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// One workgroup per row. Eight vectors of 16 bytes in flight per lane: the
+// next four are loaded while four are searched.
+//
+// The search is two-level, which takes a third of the vector instructions of
+// an element-by-element one: per vector only its maximum is formed (v_max3)
+// and compared with the lane's best, which remembers the vector; the element
+// is looked up in that one vector at the end. Indices grow along a lane's
+// walk and a strictly greater value is needed to replace the best, so the
+// first of equal values stays. NaN (the maximum, by torch's rule) is passed
+// over by v_max3 and only noted; a row that holds one is searched again
+// element by element. Vectors past the row's end re-read its last one, which
+// changes nothing: the smaller index of equal candidates wins. The bound is
+// HBM: 256 bf16 rows of 151,936 (78 MB) took 18.6 us element by element with
+// four vectors in flight, 13.0 us now (6.0 TB/s).
 template <typename T>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(ArgmaxArgs a) {
   const int64_t row = blockIdx.x;
   const uint8_t* base = a.logits + row * a.row_stride * a.esize;
   ArgmaxLane lane_state;
   const int tid = threadIdx.x;
-  if (a.vec) {
-    constexpr int P = Logit<T>::kPerVec;
-    const int64_t nvec = a.cols / P;
+  constexpr int P = Logit<T>::kPerVec;
+  const int64_t nvec = a.vec ? a.cols / P : 0;
+  if (nvec > 0) {
     const uint4* vp = reinterpret_cast<const uint4*>(base);
+    typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+    auto load = [&](int64_t v) {
+      const uint4v w = __builtin_nontemporal_load(reinterpret_cast<const uint4v*>(vp + (v < nvec ? v : nvec - 1)));
+      return uint4{w[0], w[1], w[2], w[3]};
+    };
+    float best = -INFINITY;
+    int64_t best_v = tid < nvec ? tid : nvec - 1;
+    bool nan = false;
+    uint4 cur[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) cur[u] = load(tid + static_cast<int64_t>(u) * kArgmaxThreads);
     for (int64_t v0 = tid; v0 < nvec; v0 += 4LL * kArgmaxThreads) {
-      uint4 buf[4];
+      uint4 nxt[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) nxt[u] = load(v0 + static_cast<int64_t>(u + 4) * kArgmaxThreads);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int64_t v = v0 + static_cast<int64_t>(u) * kArgmaxThreads;
-        buf[u] = v < nvec ? vp[v] : uint4{0u, 0u, 0u, 0u};
-      }
+        float x[P];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t v = v0 + static_cast<int64_t>(u) * kArgmaxThreads;
-        if (v < nvec) {
-#pragma unroll
-          for (int e = 0; e < P; ++e) lane_state.see(Logit<T>::get(buf[u], e), static_cast<uint32_t>(v * P + e));
+        for (int e = 0; e < P; ++e) x[e] = Logit<T>::get(cur[u], e);
+        float m = max3(x[0], x[1], x[2]);
+        if constexpr (P == 8) {
+          m = max3(m, x[3], x[4]);
+          m = max3(m, x[5], x[6]);
+          m = max3(m, x[7], x[7]);
+        } else {
+          m = max3(m, x[3], x[3]);
         }
+#pragma unroll
+        for (int e = 0; e < P; e += 2) nan |= __builtin_isunordered(x[e], x[e + 1]);
+        const int64_t v = v0 + static_cast<int64_t>(u) * kArgmaxThreads;
+        const bool more = m > best;
+        best = more ? m : best;
+        best_v = more ? v : best_v;
       }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) cur[u] = nxt[u];
+    }
+    if (best_v >= nvec) best_v = nvec - 1;
+    const uint4 w = vp[best_v];
+    uint32_t first = 0;
+#pragma unroll
+    for (int e = P - 1; e >= 0; --e) first = Logit<T>::get(w, e) == best ? e : first;
+    lane_state.best = best;
+    lane_state.best_idx = static_cast<uint32_t>(best_v * P + first);
+    if (__syncthreads_or(nan)) {
+      lane_state = ArgmaxLane();
+      for (int64_t c = tid; c < nvec * P; c += kArgmaxThreads)
+        lane_state.see(Logit<T>::get1(base + c * a.esize), static_cast<uint32_t>(c));
     }
     // The tail past the last whole vector, by the first lanes.
     const int64_t tail = nvec * P + tid;
