@@ -6,13 +6,20 @@
 namespace mvllm {
 
 // One decode work-list record: split `split` (of `ns`) of request `r`, whose
-// single query is token `qs` with visible keys [lo, hi]; the split streams
-// keys [begin, end]. Positions fit in int32 (the launcher checks the block
-// table's reach). r = -1 marks an empty slot.
+// single query is token `qs` with visible keys from `lo`; the split streams
+// keys [begin, end], and its partial goes to row `base` + `split` of the
+// partials. Positions fit in int32 (the launcher checks the block table's
+// reach). r = -1 marks an empty slot.
 struct DecodeItem {
   int32_t r, split, qs, ns;
-  int32_t lo, hi, begin, end;
+  int32_t lo, base, begin, end;
 };
+
+// Longest split that the pipelined decode kernel takes: it reads a split's
+// block ids once, two 16-token tiles per lane. (The general kernel, which has
+// no such limit, streams ~15% slower: 1,097 against 916 us on 64 contexts of
+// 8k-33k tokens.)
+constexpr int32_t kMaxSplit = 2048;
 
 // One prefill work-list record: query tokens [t0, t1) of request `r` (whose
 // first query is token `qs`); lo is the first visible key of row t0 and hi
@@ -45,29 +52,36 @@ struct AttnArgs {
   // quotient is a power of two (16-key pages are then found with shifts),
   // else -1.
   int32_t page_shift = -1;
-  // Split-KV decode partials: acc [R][max_splits][Hq][D], (max, sum) [R][max_splits][Hq].
+  // Split-KV decode partials: acc [item_capacity][Hq][D], (max, sum)
+  // [item_capacity][Hq]; a request's splits take consecutive rows.
   float* ws_acc;
   float2* ws_ml;
-  int32_t split_tokens, max_splits;
+  int64_t item_capacity;  // slots of the decode work list
+  int32_t split_tokens;   // bound on the length of a split
+  int32_t split_fixed;    // the length of every split, or 0: chosen with the work list
+  int32_t num_cus;
   int32_t mode;  // generic kernel: 0 = every token; 1 = only requests with > 1 query
   // Prefill work list: one record per (request, query block) slot, heaviest
   // first; r = -1 marks an empty slot. Written by the item kernel before the
   // prefill kernel reads it.
   PrefillItem* items;
-  // Decode work list: one record per (request, split) slot, full splits
-  // first, then the partial last splits from the largest; r = -1 marks an
+  // Decode work list: one record per (request, split), full splits first, then the partial last splits from the largest; r = -1 marks an
   // empty slot.
   DecodeItem* decode_items;
   // Per request, written with the decode work list: (query token, number of
   // splits), or (0, -1) for a request that is not a single-query decode. The
-  // combine kernel reads it instead of re-deriving the visible range.
+  // rows that no split writes are found from it.
   int2* decode_req;
+  // Per (request, group of KV heads that share a workgroup): splits finished
+  // so far in this launch. Zeroed with the work list; the workgroup that
+  // completes a request zeroes its counter again.
+  int32_t* done;
   // Host side only: the work lists and the per-request table are already in
   // the workspace (planned once for a step), so the launches skip the
   // work-list kernels.
   int32_t lists_ready;
-  // The caller's max_query_len hint said 1 (no prefill launch): the combine
-  // kernel makes the rows of any request with another query count NaN.
+  // The caller's max_query_len hint said 1 (no prefill launch): the rows of
+  // any request with another query count are made NaN (tidy_rows).
   int32_t decode_only;
 };
 
@@ -95,13 +109,6 @@ __device__ __forceinline__ int64_t block_of(const AttnArgs& a, int64_t r, int64_
   return (b >= 0 && b < a.num_blocks) ? b : -1;
 }
 
-// Number of split-KV partitions of a decode query with visible range [lo, hi].
-__device__ __forceinline__ int64_t decode_num_splits(int64_t lo, int64_t hi, int32_t split) {
-  if (hi < lo) return 0;
-  const int64_t base = lo & ~int64_t(15);
-  return (hi - base + split) / split;
-}
-
 // Host-side launchers (one per kernel family).
 // Launchers; `start`/`stop` (may be null) bracket the main kernel's launch.
 int launch_generic(const AttnArgs& a, int32_t dtype, hipStream_t s);
@@ -123,7 +130,6 @@ bool decode_step_eligible(const AttnArgs& a);
 // split length (128 always; 64 and 96 with the pipelined kernel only).
 bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens);
 int64_t decode_step_blocks(const AttnArgs& a);  // decode workgroups of the step grid
-int launch_decode_combine(const AttnArgs& a, int32_t dtype, hipStream_t s);
 // `prefill_first`: the prefill workgroups lead the grid (else the decode ones).
 int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_t s, hipEvent_t start,
                 hipEvent_t stop);

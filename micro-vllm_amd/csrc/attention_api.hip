@@ -27,56 +27,59 @@ int device_cu_count() {
 
 namespace {
 
-// Split size (tokens) of the split-KV decode partition. It depends only on
-// shapes so that the workspace can be sized before a graph is captured.
-int32_t decode_split_tokens(int64_t num_requests, int64_t max_context) {
+// The split length that MVLLM_DECODE_SPLIT asks for (0: none), for every
+// split of a call.
+int32_t decode_split_override() {
   if (const char* env = std::getenv("MVLLM_DECODE_SPLIT")) {
     const long v = std::strtol(env, nullptr, 10);
     if (v >= 16 && v % 16 == 0 && v <= (1 << 20)) return static_cast<int32_t>(v);
   }
-  // Aim for roughly 2 (request, split) items per CU when every request
-  // reaches half of the table's reach; never below 64 tokens per split.
-  // (The sorted decode work list balances the grid; fewer, longer items
-  // spend less on dispatch and per-item setup: 1,024-token splits on the
-  // 256-sequence Qwen3 batch ran at 357-361 us against 371 us for 512.)
+  return 0;
+}
+
+// Split length that sizes the workspace. It depends only on shapes, so that
+// the workspace can be sized before a graph is captured: two (request, split)
+// items per CU when every request reaches half of the table's reach, at least
+// 64 tokens. The actual lengths are chosen on the device from the visible
+// tokens (choose_split), within the slots that this gives.
+int32_t decode_layout_split(int64_t num_requests, int64_t max_context) {
+  if (const int32_t fixed = decode_split_override()) return fixed;
   const int64_t target_items = 2LL * device_cu_count();
   const int64_t est_tokens = num_requests * (max_context / 2 > 16 ? max_context / 2 : 16);
   int64_t split = (est_tokens + target_items - 1) / target_items;
   split = (split + 15) / 16 * 16;
   if (split < 64) split = 64;
-  // The pipelined decode kernel reads a split's block ids once, two 16-token
-  // tiles per lane, so it takes splits of up to 2048 tokens; longer splits
-  // would fall back to the general kernel, which streams ~15% slower
-  // (64 contexts of 8k-33k tokens: 916 vs 1097 us).
-  if (split > 2048) split = 2048;
+  if (split > kMaxSplit) split = kMaxSplit;
   return static_cast<int32_t>(split);
 }
 
 struct DecodeLayout {
-  int32_t split_tokens;
-  int32_t max_splits;
+  int64_t item_capacity;  // (request, split) slots
   int64_t acc_bytes;
   int64_t ml_bytes;
   int64_t items_bytes;  // prefill work list: one 32-byte record per slot, N / 8 + R slots at most
   int64_t decode_items_bytes;  // decode work list: one 32-byte record per (request, split)
-  int64_t decode_req_bytes;  // per request (query token, splits) for the combine kernel
-  int64_t total() const { return acc_bytes + ml_bytes + items_bytes + decode_items_bytes + decode_req_bytes; }
+  int64_t decode_req_bytes;  // per request (query token, splits)
+  int64_t done_bytes;  // per (request, group of KV heads) finished splits; there are at most Hq groups
+  int64_t results_and_lists() const { return acc_bytes + ml_bytes + items_bytes + decode_items_bytes + decode_req_bytes; }
+  int64_t total() const { return results_and_lists() + done_bytes; }
 };
 
 DecodeLayout decode_layout(const mvllm_batch* b, int64_t num_q_heads, int64_t head_dim) {
   DecodeLayout d;
   const int64_t reach = b->block_table_width * b->block_size;
-  d.split_tokens = decode_split_tokens(b->num_requests, reach);
+  const int64_t split = decode_layout_split(b->num_requests, reach);
   // Visible ranges start at a 16-aligned base at most 15 tokens early.
-  const int64_t splits = (reach + 15 + d.split_tokens) / d.split_tokens;
-  d.max_splits = static_cast<int32_t>(splits < 1 ? 1 : splits);
-  const int64_t items = b->num_requests * d.max_splits * num_q_heads;
+  const int64_t splits = (reach + 15 + split) / split;
+  d.item_capacity = b->num_requests * (splits < 1 ? 1 : splits);
+  const int64_t items = d.item_capacity * num_q_heads;
   d.acc_bytes = (items * head_dim * 4 + 255) / 256 * 256;
   d.ml_bytes = (items * 8 + 255) / 256 * 256;
   // Prefill query blocks hold T = 128 / G >= 8 tokens.
   d.items_bytes = ((b->num_tokens / 8 + b->num_requests) * static_cast<int64_t>(sizeof(PrefillItem)) + 255) / 256 * 256;
-  d.decode_items_bytes = (b->num_requests * d.max_splits * static_cast<int64_t>(sizeof(DecodeItem)) + 255) / 256 * 256;
+  d.decode_items_bytes = (d.item_capacity * static_cast<int64_t>(sizeof(DecodeItem)) + 255) / 256 * 256;
   d.decode_req_bytes = (b->num_requests * 8 + 255) / 256 * 256;
+  d.done_bytes = (b->num_requests * num_q_heads * 4 + 255) / 256 * 256;
   return d;
 }
 
@@ -251,12 +254,12 @@ void fill_batch_args(AttnArgs& a, const mvllm_batch* batch, const mvllm_kv_cache
 
 // The cache-side conditions of the MFMA kernels (the query and output add
 // their own): a plan is built whenever a planned call can take that path.
-bool fast_cache(const mvllm_kv_cache* cache, const mvllm_batch* batch, int64_t group) {
+bool fast_cache(const mvllm_kv_cache* cache, int64_t group) {
   const int32_t dtype = cache->dtype;
   const int64_t es = dtype_bytes(dtype);
   return (dtype == MVLLM_DTYPE_BF16 || dtype == MVLLM_DTYPE_F16) && group <= 16 &&
-         decode_supported(cache->head_dim, cache->block_size,
-                          decode_split_tokens(batch->num_requests, batch->block_table_width * batch->block_size)) &&
+         decode_supported(cache->head_dim, cache->block_size, decode_split_override()) &&
+         32 * cache->stride[2] < (int64_t{1} << 32) &&  // 16 rows within a 32-bit byte offset
          cache->stride[4] == 1 && cache->stride[3] == cache->head_dim && vec16(cache->stride[0], es) &&
          vec16(cache->stride[1], es) && vec16(cache->stride[2], es) && aligned16(cache->data);
 }
@@ -275,7 +278,7 @@ bool takes_lists(const mvllm_batch* batch, const mvllm_kv_cache* cache, int64_t 
   const DecodeLayout d = decode_layout(batch, Hq, cache->head_dim);
   return workspace && aligned16(workspace) && workspace_bytes >= d.total() &&
          batch->block_table_width * batch->block_size < kMost && batch->num_tokens < kMost &&
-         batch->num_requests * d.max_splits * cache->num_kv_heads < kMost &&
+         d.item_capacity * cache->num_kv_heads < kMost &&
          (batch->num_tokens / 8 + batch->num_requests) * cache->num_kv_heads < kMost &&
          batch->num_requests * Hq < kMost;
 }
@@ -289,7 +292,7 @@ bool attention_fast_path(const mvllm_tensor3* query, const mvllm_kv_cache* cache
   const int64_t Hkv = cache->num_kv_heads;
   if (Hkv <= 0 || query->size[1] % Hkv != 0) return false;
   const int64_t es = dtype_bytes(query->dtype);
-  return fast_cache(cache, batch, query->size[1] / Hkv) &&
+  return fast_cache(cache, query->size[1] / Hkv) &&
          takes_lists(batch, cache, query->size[1], workspace, workspace_bytes) && query->stride[2] == 1 && vec16(query->stride[0], es) &&
          vec16(query->stride[1], es) && aligned16(query->data) && out->stride[2] == 1 &&
          vec16(out->stride[0], es) && vec16(out->stride[1], es) && aligned16(out->data);
@@ -304,14 +307,19 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
                 (long long)workspace_bytes, (long long)d.total());
   if (!aligned16(workspace)) return fail(MVLLM_ERR_INVALID, "workspace must be 16-byte aligned");
   char* const w = static_cast<char*>(workspace);
-  a.split_tokens = d.split_tokens;
-  a.max_splits = d.max_splits;
+  a.split_fixed = decode_split_override();
+  a.split_tokens = a.split_fixed ? a.split_fixed : kMaxSplit;
+  a.num_cus = device_cu_count();
+  a.item_capacity = a.split_fixed ? d.item_capacity
+                                  : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
+                                               d.item_capacity, a.num_cus, D);
   a.decode_only = batch->max_query_len == 1 ? 1 : 0;
   a.ws_acc = reinterpret_cast<float*>(w);
   a.ws_ml = reinterpret_cast<float2*>(w + d.acc_bytes);
   a.items = reinterpret_cast<PrefillItem*>(w + d.acc_bytes + d.ml_bytes);
   a.decode_items = reinterpret_cast<DecodeItem*>(w + d.acc_bytes + d.ml_bytes + d.items_bytes);
   a.decode_req = reinterpret_cast<int2*>(w + d.acc_bytes + d.ml_bytes + d.items_bytes + d.decode_items_bytes);
+  a.done = reinterpret_cast<int32_t*>(w + d.results_and_lists());
   return MVLLM_OK;
 }
 
@@ -323,7 +331,7 @@ int attention_plan(const mvllm_batch* batch, int64_t Hq, const mvllm_kv_cache* c
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0)
     return fail(MVLLM_ERR_INVALID, "query heads %lld not a multiple of KV heads %lld", (long long)Hq,
                 (long long)Hkv);
-  if (batch->num_tokens == 0 || batch->num_requests == 0 || !fast_cache(cache, batch, Hq / Hkv)) return MVLLM_OK;
+  if (batch->num_tokens == 0 || batch->num_requests == 0 || !fast_cache(cache, Hq / Hkv)) return MVLLM_OK;
   AttnArgs a = {};
   fill_batch_args(a, batch, cache, Hq);
   if (!takes_lists(batch, cache, Hq, workspace, workspace_bytes)) return MVLLM_OK;
@@ -480,7 +488,11 @@ int attention_forward(const mvllm_tensor3* query, const mvllm_tensor3* key,
 // it until the process ends. In host code `scratch` names a host-side
 // stand-in, never the device memory: its device address comes from
 // hipGetSymbolAddress, once per device, and only that address is passed on.
-static __device__ __align__(256) unsigned char scratch[MVLLM_NOALLOC_SCRATCH_BYTES];
+// The partial results and work lists may fill MVLLM_NOALLOC_SCRATCH_BYTES; the
+// counters of finished splits (4 bytes per request and query head, against at
+// least 256 bytes of partials) lie behind them.
+static constexpr int64_t kScratchBytes = MVLLM_NOALLOC_SCRATCH_BYTES + MVLLM_NOALLOC_SCRATCH_BYTES / 64 + 256;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace mvllm {
 namespace {
@@ -584,7 +596,7 @@ extern "C" int mvllm_attention_forward_noalloc(const mvllm_tensor3* query,
   clear_error();
   if (!query || !batch || !cache) return fail(MVLLM_ERR_INVALID, "query, batch or cache is null");
   const int64_t need = mvllm_attention_workspace_bytes(batch, query->size[1], query->size[2]);
-  if (need > MVLLM_NOALLOC_SCRATCH_BYTES)
+  if (need > 0 && decode_layout(batch, query->size[1], query->size[2]).results_and_lists() > MVLLM_NOALLOC_SCRATCH_BYTES)
     return fail(MVLLM_ERR_WORKSPACE,
                 "batch needs %lld bytes of workspace; mvllm_attention_forward_noalloc holds at most %lld "
                 "(use mvllm_attention_forward with a caller workspace)",
@@ -593,6 +605,6 @@ extern "C" int mvllm_attention_forward_noalloc(const mvllm_tensor3* query,
   void* ws = nullptr;
   if (int rc = scratch_address(s, &ws)) return rc;
   // Everything stays on the caller's stream: no side stream is created.
-  return attention_forward(query, key, value, cache, batch, out, scale, ws, MVLLM_NOALLOC_SCRATCH_BYTES,
+  return attention_forward(query, key, value, cache, batch, out, scale, ws, kScratchBytes,
                            nullptr, stream, true);
 }

@@ -23,11 +23,10 @@
 // MFMAs are free).
 //
 // Each split writes (max, sum, unnormalised acc) partials; a request whose
-// context fits one split writes its output directly. The combine kernel
-// merges partials with the standard log-sum-exp rescaling (FlashAttention-2,
-// Dao 2023; flash-decoding, Dao et al. 2023) and zero-fills tokens that
-// belong to no request. It learns each request's query token and split count
-// from a table that the work-list kernel writes, one load per workgroup.
+// context fits one split writes its output directly. The workgroup that
+// completes a request merges its partials with the standard log-sum-exp
+// rescaling (FlashAttention-2, Dao 2023; flash-decoding, Dao et al. 2023).
+// The grid's last workgroups fill the rows that no split writes.
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -95,19 +94,25 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
   // 1-D grid: workgroup b takes head group b % groups of work-list slot b / groups.
   const int groups = (a.num_kv_heads + waves - 1) / waves;
   const int h = static_cast<int>(blockIdx.x % groups) * waves + wave;
-  const DecodeItem item = a.decode_items[blockIdx.x / groups];
+  const int64_t slot = blockIdx.x / groups;
+  if (slot >= a.item_capacity) {  // past the work list's capacity
+    tidy_rows<T>(a, static_cast<int64_t>(blockIdx.x) - a.item_capacity * groups);
+    return;
+  }
+  const DecodeItem item = a.decode_items[slot];
   if (item.r < 0 || item.r >= a.num_requests) return;
   const int split = item.split;
   const int64_t r = item.r;
-  if (h >= a.num_kv_heads) return;
+  const bool live = h < a.num_kv_heads;  // a spare wave only joins the epilogue's barriers
   const int64_t qs = item.qs;
   const int64_t lo = item.lo;
   const int64_t begin = item.begin;
-  const int64_t end = item.end;
+  const int64_t end = live ? item.end : item.begin - 1;
   // Records index the query, the table and the partials: out-of-range
   // fields (never written by the work-list kernel) end the workgroup.
-  if (begin < 0 || begin > end || end - begin >= a.split_tokens || end >= a.width * a.block_size ||
-      qs < 0 || qs >= a.num_tokens || split < 0 || split >= a.max_splits)
+  if (begin < 0 || begin > item.end || end - begin >= a.split_tokens || end >= a.width * a.block_size ||
+      qs < 0 || qs >= a.num_tokens || split < 0 || split >= item.ns || item.base < 0 ||
+      static_cast<int64_t>(item.base) + item.ns > a.item_capacity)
     return;
 
   // Q^T as the B operand: lane (col, grp) holds head col, dims 32i + 8grp .. +8.
@@ -116,10 +121,10 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
   short8_t qv[4];
   {
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + qs * a.q_s0 +
-                         static_cast<int64_t>(col < G ? hq : 0) * a.q_s1 + 8 * grp;
+                         static_cast<int64_t>(live && col < G ? hq : 0) * a.q_s1 + 8 * grp;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      qv[i] = (col < G) ? *reinterpret_cast<const short8_t*>(qp + 32 * i) : short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      qv[i] = (live && col < G) ? *reinterpret_cast<const short8_t*>(qp + 32 * i) : short8_t{0, 0, 0, 0, 0, 0, 0, 0};
     }
   }
 
@@ -192,166 +197,16 @@ __global__ __launch_bounds__(512) void decode_split_kernel(AttnArgs a) {
   }
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
-  if (col >= G) return;
-  write_decode_result<T, kDim>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
+  finish_split<T, kDim>(a, item, h, live, static_cast<int>(blockIdx.x % groups), groups, m, lt, acc,
+                        reinterpret_cast<int32_t*>(&lds[0][0]));
 }
 
 // The pipelined kernel (decode_split_lds_body) for block sizes that are
 // multiples of 16: K and V tiles go straight from HBM to LDS.
 template <typename T, int D, int STAGES>
-__global__ __launch_bounds__(256) void decode_split_lds_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 2) void decode_split_lds_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   decode_split_lds_body<T, D, STAGES>(a, smem, blockIdx.x, blockDim.x >> 6);
-}
-
-
-// Blocks [0, R * head_groups): merge split partials of multi-split
-// decode requests, kCombineHeads query heads per block, 32 lanes per head
-// (4 dims each; at head_dim 64 and 96 the last lanes only merge statistics). Up to CAP splits are merged from one round of loads (the
-// launch picks CAP >= the layout's split count when it is at most 32).
-// Blocks after that: zero tokens outside every request, kZeroTokens each.
-constexpr int kZeroTokens = 16;
-constexpr int kCombineHeads = 8;
-
-template <typename T, int D, int CAP>
-__global__ __launch_bounds__(256) void decode_combine_kernel(AttnArgs a, int32_t head_groups) {
-  const int64_t R = a.num_requests;
-  const int64_t combine_blocks = R * head_groups;
-  if (static_cast<int64_t>(blockIdx.x) >= combine_blocks) {
-    const int64_t first = a.qsl[0], last = a.qsl[R];
-    const int64_t t0 = (blockIdx.x - combine_blocks) * kZeroTokens;
-    const int64_t row = static_cast<int64_t>(a.num_q_heads) * a.head_dim;
-    // Contiguous, 16-byte aligned token rows (the usual output): 16-byte
-    // stores of zero bits (+0 in every dtype); otherwise element stores.
-    const bool vec = a.o_s2 == 1 && a.o_s1 == a.head_dim && (row * static_cast<int64_t>(sizeof(T))) % 16 == 0 &&
-                     (a.o_s0 * static_cast<int64_t>(sizeof(T))) % 16 == 0 &&
-                     (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
-    for (int64_t t = t0; t < t0 + kZeroTokens && t < a.num_tokens; ++t) {
-      if (t >= first && t < last) continue;
-      T* op = static_cast<T*>(a.out) + t * a.o_s0;
-      if (vec) {
-        const int64_t chunks = row * static_cast<int64_t>(sizeof(T)) / 16;
-        for (int64_t i = threadIdx.x; i < chunks; i += blockDim.x)
-          reinterpret_cast<uint4*>(op)[i] = uint4{0u, 0u, 0u, 0u};
-      } else {
-        for (int64_t i = threadIdx.x; i < row; i += blockDim.x) {
-          const int64_t hq = i / a.head_dim, d = i - hq * a.head_dim;
-          Elem<T>::store(op + hq * a.o_s1 + d * a.o_s2, 0.f);
-        }
-      }
-    }
-    return;
-  }
-  const int64_t r = blockIdx.x / head_groups;
-  const int hq = static_cast<int>(blockIdx.x % head_groups) * kCombineHeads + (threadIdx.x >> 5);
-  if (hq >= a.num_q_heads) return;
-  // (query token, splits) from the work-list kernel: -1 is not a decode
-  // request, and a single split has written its output itself.
-  const int2 req = a.decode_req[r];
-  const int64_t qs = req.x, ns = req.y;
-  const bool has_dims = 4 * (threadIdx.x & 31) < D;
-  const int d0 = has_dims ? 4 * (threadIdx.x & 31) : 0;
-  if (ns < 0 && a.decode_only) {
-    // A request with another query count in a batch whose hint promised
-    // single-query requests only: no kernel computes its rows, so they are
-    // made NaN rather than left holding whatever the output memory held.
-    const int64_t q0 = a.qsl[r], q1 = a.qsl[r + 1];
-    if (q0 < 0 || q1 > a.num_tokens) return;
-    const uint32_t nan_bits = Elem<T>::to_bits(NAN);
-    const uint32_t nan2 = nan_bits | (nan_bits << 16);
-    for (int64_t t = q0; t < q1; ++t) {
-      uint16_t* op = static_cast<uint16_t*>(a.out) + t * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
-      if (has_dims) *reinterpret_cast<uint2*>(op + d0) = uint2{nan2, nan2};
-    }
-    return;
-  }
-  if (ns < 0 || ns == 1 || ns > a.max_splits || qs < 0 || qs >= a.num_tokens) return;
-  uint32_t w[2];
-  if (ns == 0) {
-    // Nothing visible: softmax over no keys is NaN in the reference.
-    const uint32_t nan_bits = Elem<T>::to_bits(NAN);
-    w[0] = w[1] = nan_bits | (nan_bits << 16);
-  } else if (ns <= CAP) {
-    // Up to CAP splits (the common case): every split's (max, sum) and
-    // accumulator slice are loaded at once, one round trip after the table.
-    const int sub = threadIdx.x & 31;
-    const int64_t first_item = r * a.max_splits * a.num_q_heads + hq;
-    const int cnt = static_cast<int>(ns);
-    float2 ml = make_float2(-INFINITY, 0.f);
-    if (sub < cnt) ml = a.ws_ml[first_item + sub * a.num_q_heads];
-    const float* accp = a.ws_acc + first_item * D + d0;
-    float4_t v[CAP];
-#pragma unroll
-    for (int j = 0; j < CAP; ++j) {
-      const int k = j < cnt ? j : cnt - 1;  // indices past the last split re-read it, unused
-      v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * D);
-    }
-    float mx = ml.x;  // lanes past the last split hold -inf and a zero sum
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 32));
-    // A split with no visible key (m = -inf) weighs 0; so does every split
-    // when none has one, and the output is then NaN (0 / 0).
-    const float wgt = ml.x == -INFINITY ? 0.f : exp2f(ml.x - mx);
-    float sum = wgt * ml.y;
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 32);
-    float4_t o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < CAP; ++j) {
-      const float wj = __shfl(wgt, j, 32);
-      if (j < cnt) o += v[j] * wj;
-    }
-    const float inv = 1.f / sum;
-    w[0] = Elem<T>::to_bits(o[0] * inv) | (Elem<T>::to_bits(o[1] * inv) << 16);
-    w[1] = Elem<T>::to_bits(o[2] * inv) | (Elem<T>::to_bits(o[3] * inv) << 16);
-  } else {
-    // Two passes over the head's splits, 32 lanes wide: the maximum first,
-    // then every split's weight exp2(m_s - max) from its own lane, so the
-    // accumulator loads do not wait on a running maximum.
-    const int sub = threadIdx.x & 31;
-    const int64_t first_item = r * a.max_splits * a.num_q_heads + hq;
-    float mx = -INFINITY;
-    for (int64_t s0 = 0; s0 < ns; s0 += 32)
-      if (s0 + sub < ns) mx = fmaxf(mx, a.ws_ml[first_item + (s0 + sub) * a.num_q_heads].x);
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 32));
-    float sum = 0.f;
-    float4_t o = {0.f, 0.f, 0.f, 0.f};
-    for (int64_t s0 = 0; s0 < ns; s0 += 32) {
-      float w = 0.f;
-      if (s0 + sub < ns) {
-        const float2 ml = a.ws_ml[first_item + (s0 + sub) * a.num_q_heads];
-        // A split with no visible key (m = -inf) weighs 0; so does every
-        // split when none has one, and the output is then NaN (0 / 0).
-        w = ml.x == -INFINITY ? 0.f : exp2f(ml.x - mx);
-        sum += w * ml.y;
-      }
-      const int cnt = ns - s0 < 32 ? static_cast<int>(ns - s0) : 32;
-      const float* accp = a.ws_acc + (first_item + s0 * a.num_q_heads) * D + d0;
-      // Eight splits per pass, their loads issued together (indices past
-      // the last split re-read it and are not added).
-      for (int k0 = 0; k0 < cnt; k0 += 8) {
-        float4_t v[8];
-        float wk[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int k = k0 + j < cnt ? k0 + j : cnt - 1;
-          wk[j] = __shfl(w, k, 32);
-          v[j] = *reinterpret_cast<const float4_t*>(accp + static_cast<int64_t>(k) * a.num_q_heads * D);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (k0 + j < cnt) o += v[j] * wk[j];
-      }
-    }
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 32);
-    const float inv = 1.f / sum;
-    w[0] = Elem<T>::to_bits(o[0] * inv) | (Elem<T>::to_bits(o[1] * inv) << 16);
-    w[1] = Elem<T>::to_bits(o[2] * inv) | (Elem<T>::to_bits(o[3] * inv) << 16);
-  }
-  uint16_t* op = static_cast<uint16_t*>(a.out) + qs * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
-  if (has_dims) *reinterpret_cast<uint2*>(op + d0) = uint2{w[0], w[1]};
 }
 
 
@@ -367,7 +222,7 @@ struct DecodeTuning {
 
 DecodeTuning decode_tuning(const AttnArgs& a) {
   DecodeTuning t;
-  t.lds_pipeline = a.block_size % 16 == 0 && a.split_tokens <= 2048;
+  t.lds_pipeline = a.block_size % 16 == 0 && a.split_tokens <= kMaxSplit;
   t.waves = 4;
   t.stages = a.head_dim == 64 ? kStages<64> : a.head_dim == 96 ? kStages<96> : kStages<128>;
   t.prefetch = false;
@@ -411,30 +266,13 @@ int launch_lds_kernel(const AttnArgs& a, dim3 grid, int waves, hipStream_t s, hi
 }
 
 template <typename T, int D>
-int launch_combine_t(const AttnArgs& a, hipStream_t s) {
-  const int32_t head_groups = (a.num_q_heads + kCombineHeads - 1) / kCombineHeads;
-  const int64_t blocks = a.num_requests * head_groups + (a.num_tokens + kZeroTokens - 1) / kZeroTokens;
-  if (blocks > 0) {
-    if (blocks > INT32_MAX) return fail(MVLLM_ERR_INVALID, "combine grid too large");
-    // Short splits on small batches give requests up to ~20 splits; they
-    // still merge in one round of loads.
-    const dim3 grid(static_cast<unsigned>(blocks)), block(32 * kCombineHeads);
-    if (a.max_splits <= 8) hipLaunchKernelGGL((decode_combine_kernel<T, D, 8>), grid, block, 0, s, a, head_groups);
-    else if (a.max_splits <= 16) hipLaunchKernelGGL((decode_combine_kernel<T, D, 16>), grid, block, 0, s, a, head_groups);
-    else hipLaunchKernelGGL((decode_combine_kernel<T, D, 32>), grid, block, 0, s, a, head_groups);
-    MVLLM_LAUNCH_CHECK("decode_combine_kernel");
-  }
-  return MVLLM_OK;
-}
-
-template <typename T, int D>
 int launch_decode_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
   const DecodeTuning tune = decode_tuning(a);
   const int waves = tune.waves;
   const int groups = (a.num_kv_heads + waves - 1) / waves;
 
   if (a.num_requests > 0) {
-    const int64_t blocks = a.num_requests * a.max_splits * groups;
+    const int64_t blocks = a.item_capacity * groups + tidy_blocks(a);
     if (blocks > INT32_MAX) return fail(MVLLM_ERR_INVALID, "decode grid too large (%lld workgroups)", (long long)blocks);
     if (!a.lists_ready) {
       if (int rc = launch_decode_lists(a, s)) return rc;
@@ -465,7 +303,7 @@ int launch_decode_t(const AttnArgs& a, hipStream_t s, hipEvent_t start, hipEvent
       MVLLM_LAUNCH_CHECK("decode_split_kernel");
     }
   }
-  return launch_combine_t<T, D>(a, s);
+  return MVLLM_OK;
 }
 
 // Calls f(T{}, integral_constant D) for the decode kernels' types and head
@@ -504,7 +342,7 @@ int launch_decode(const AttnArgs& a, int32_t dtype, hipStream_t s, hipEvent_t st
 }
 
 bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens) {
-  return head_dim == 128 || ((head_dim == 64 || head_dim == 96) && block_size % 16 == 0 && split_tokens <= 2048);
+  return head_dim == 128 || ((head_dim == 64 || head_dim == 96) && block_size % 16 == 0 && split_tokens <= kMaxSplit);
 }
 
 bool decode_step_eligible(const AttnArgs& a) {
@@ -517,13 +355,7 @@ bool decode_step_eligible(const AttnArgs& a) {
 }
 
 int64_t decode_step_blocks(const AttnArgs& a) {
-  return a.num_requests * a.max_splits * ((a.num_kv_heads + kStepDecodeWaves - 1) / kStepDecodeWaves);
-}
-
-int launch_decode_combine(const AttnArgs& a, int32_t dtype, hipStream_t s) {
-  return for_decode_types(a, dtype, [&](auto t, auto d) {
-    return launch_combine_t<decltype(t), decltype(d)::value>(a, s);
-  });
+  return a.item_capacity * ((a.num_kv_heads + kStepDecodeWaves - 1) / kStepDecodeWaves) + tidy_blocks(a);
 }
 
 }  // namespace mvllm

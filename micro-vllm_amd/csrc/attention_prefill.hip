@@ -115,21 +115,6 @@ template <> struct Mma32<f16_t> {
   }
 };
 
-// Minimum / maximum over the wave, in every lane, with no LDS round trip:
-// DPP quad permutes [1,0,3,2] and [2,3,0,1], then the 8- and 16-lane mirrors,
-// then the 16- and 32-lane swaps.
-template <typename Op>
-__device__ __forceinline__ int32_t wave_reduce_i(int32_t v, Op op) {
-  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
-  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
-  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
-  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
-  const auto r16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
-  v = op(static_cast<int32_t>(r16[0]), static_cast<int32_t>(r16[1]));
-  const auto r32 = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
-  return op(static_cast<int32_t>(r32[0]), static_cast<int32_t>(r32[1]));
-}
-
 __device__ __forceinline__ int32_t wave_min_i(int32_t v) {
   return wave_reduce_i(v, [](int32_t x, int32_t y) { return x < y ? x : y; });
 }
@@ -258,8 +243,7 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   constexpr int kSteps = D / 16;              // 16-dim MFMA steps of a score
   constexpr int kBlocks = D / 32;             // 32-dim blocks of O^T; also the 1 KiB loads of a page
   constexpr bool kSplitP = D != 128;
-  uint8_t* const kbuf = smem;                   // K stages 0, 1 (16 KiB each)
-  uint8_t* const vbuf = smem + 2 * kTileBytes;  // V stages 0, 1
+  uint8_t* const vbuf = smem + 2 * kTileBytes;  // V stages 0, 1 (K stages 0, 1 lie before them)
   int32_t* const page_tbl = reinterpret_cast<int32_t*>(smem + 4 * kTileBytes);
   int32_t* const red = page_tbl + kTableInts;
   uint8_t* const dummy = reinterpret_cast<uint8_t*>(red + 16);
@@ -918,11 +902,9 @@ int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_
     return fail(MVLLM_ERR_UNSUPPORTED, "the attention step kernel does not support this geometry");
   if (a.width * a.block_size > INT32_MAX || a.num_tokens > INT32_MAX)
     return fail(MVLLM_ERR_UNSUPPORTED, "decode positions beyond 2^31 are not supported");
-  if (int rc = for_prefill_types(a, dtype, [&](auto t, auto d) {
-        return launch_step_t<decltype(t), decltype(d)::value>(a, prefill_first, s, start, stop);
-      }))
-    return rc;
-  return launch_decode_combine(a, dtype, s);
+  return for_prefill_types(a, dtype, [&](auto t, auto d) {
+    return launch_step_t<decltype(t), decltype(d)::value>(a, prefill_first, s, start, stop);
+  });
 }
 
 }  // namespace mvllm

@@ -146,6 +146,22 @@ __device__ __forceinline__ float sum_xor32_f(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Reduction over the wave (minimum, maximum, sum), in every lane, with no LDS
+// round trip:
+// DPP quad permutes [1,0,3,2] and [2,3,0,1], then the 8- and 16-lane mirrors,
+// then the 16- and 32-lane swaps.
+template <typename Op>
+__device__ __forceinline__ int32_t wave_reduce_i(int32_t v, Op op) {
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
+  const auto r16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
+  v = op(static_cast<int32_t>(r16[0]), static_cast<int32_t>(r16[1]));
+  const auto r32 = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(v), static_cast<uint32_t>(v), false, false);
+  return op(static_cast<int32_t>(r32[0]), static_cast<int32_t>(r32[1]));
+}
+
 // Orders this wave's LDS writes before its later LDS reads (and vice versa)
 // without a workgroup barrier: the waves of one workgroup never share LDS
 // rows in the decode kernel.
@@ -173,16 +189,19 @@ __device__ __forceinline__ void lds_dma_load16(const void* global_ptr, uint32_t 
 }
 
 // lds_dma_load16 for data read exactly once (the decode kernel's K/V
-// stream): the non-temporal hint lets the lines leave the caches first
-// instead of displacing data that is reused.
-__device__ __forceinline__ void lds_dma_load16_stream(const void* global_ptr, uint32_t lds_base) {
+// stream), from a wave-uniform 64-bit base in SGPRs and a per-lane 32-bit byte
+// offset, to a wave-uniform LDS base plus an immediate added straight into M0
+// (s_add_u32 also writes SCC). The non-temporal hint lets the lines leave the
+// caches first instead of displacing data that is reused.
+template <int OFF>
+__device__ __forceinline__ void lds_dma_load16_stream(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile(
-      "s_mov_b32 m0, %1\n\t"
+      "s_add_u32 m0, %1, %3\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off nt"
+      "global_load_lds_dwordx4 %0, %2 nt"
       :
-      : "v"(global_ptr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
-      : "memory", "m0");
+      : "v"(offset), "s"(lds_base), "s"(base), "i"(OFF)
+      : "memory", "m0", "scc");
 }
 
 // lds_dma_load16 with a wave-uniform 64-bit base in SGPRs and a per-lane

@@ -28,18 +28,137 @@ __device__ __forceinline__ void split_hi_lo(float p, uint32_t& hi, uint32_t& lo)
   lo = Elem<T>::to_bits(p - Elem<T>::from_bits(hi));
 }
 
-// Epilogue shared by the decode kernels. acc[b][e] is
-// O[head hq][dim 16b + 4grp + e] (unnormalised), m / lt the running
+// ---------------------------------------------------------------------------
+// Partials of a request with several splits, and their merge.
+//
+// The workgroup that finishes a request's last open split merges the partials
+// in the same launch. Workgroups of one request run on different XCDs, whose
+// L2 caches are not coherent with each other, so the partials are written and
+// read past them (sc1: agent-scope stores and loads, the same bits that
+// relaxed agent-scope atomics carry): each workgroup's stores are complete
+// (vmcnt 0) before it counts itself done, and the one that counts last reads
+// only after that. No cache-wide write-back or invalidation is involved (with
+// a device-scope fence per workgroup the 256-sequence Qwen3 batch's kernel had
+// taken 590 us instead of 372). A merge kernel of its own cost 4-9 us per
+// forward: the launch, then two or three dependent rounds of loads.
+
+typedef uint32_t uint4_ext __attribute__((ext_vector_type(4)));
+constexpr int kAgentScope = 16;  // sc1 in a buffer instruction's cache-policy operand
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);
+}
+
+// Merges `ns` partials (rows base, base + 1, ...) of query token `qs` for the G
+// query heads of KV head `h`, one wave: 32 lanes per query head, 4 dims each
+// (at head_dim 64 and 96 the last lanes only merge statistics), with the
+// log-sum-exp rule. A round takes up to CAP splits (MANY: several rounds) of
+// PAIRS pairs of heads, about 32 rows, whose loads are issued together.
+template <typename T, int D, int CAP, bool MANY>
+__device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t base, int64_t qs, int h, int ns) {
+  static_assert(CAP <= 32, "one lane per split of a round");
+  constexpr int PAIRS = CAP <= 8 ? 4 : CAP <= 16 ? 2 : 1;
+  const int sub = threadIdx.x & 31;
+  const int half = (threadIdx.x >> 5) & 1;
+  const bool has_dims = 4 * sub < D;
+  const int d0 = has_dims ? 4 * sub : 0;
+  const int64_t row0 = base * a.num_q_heads;  // partial row of (split 0, head 0)
+  for (int g0 = 0; g0 < a.group; g0 += 2 * PAIRS) {
+    auto pair_live = [&](int p) { return g0 + 2 * p < a.group; };  // wave-uniform
+    auto head_live = [&](int p) { return g0 + 2 * p + half < a.group; };
+    auto head = [&](int p) { return h * a.group + g0 + 2 * p + (head_live(p) ? half : 0); };
+    // This lane's split of a round: its (max, sum), or (-inf, 0) past the end.
+    auto round_stats = [&](int s0, int p) {
+      const bool own = sub < CAP && s0 + sub < ns;
+      int s = own ? s0 + sub : 0;
+      asm volatile("" : "+v"(s));  // one load for all lanes, not one per side of the condition
+      const uint64_t w = __hip_atomic_load(
+          reinterpret_cast<const uint64_t*>(a.ws_ml) + row0 + head(p) + static_cast<int64_t>(s) * a.num_q_heads,
+          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return own ? make_float2(__uint_as_float(static_cast<uint32_t>(w)), __uint_as_float(static_cast<uint32_t>(w >> 32)))
+                 : make_float2(-INFINITY, 0.f);
+    };
+    float mx[PAIRS], sum[PAIRS];
+    float4_t o[PAIRS];
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      mx[p] = -INFINITY;
+      sum[p] = 0.f;
+      o[p] = float4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (MANY) {
+        for (int s0 = CAP; s0 < ns; s0 += CAP) mx[p] = fmaxf(mx[p], round_stats(s0, p).x);
+      }
+    }
+    for (int s0 = 0; s0 < (MANY ? ns : 1); s0 += CAP) {
+      float2 ml[PAIRS];
+      float4_t v[PAIRS][CAP];
+      const __amdgpu_buffer_rsrc_t rows = buffer_at(a.ws_acc + (row0 + static_cast<int64_t>(s0) * a.num_q_heads) * D);
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p) {
+        if (!pair_live(p)) continue;
+        ml[p] = round_stats(s0, p);
+#pragma unroll
+        for (int j = 0; j < CAP; ++j) {
+          const int k = s0 + j < ns ? j : ns - 1 - s0;  // past the last split: re-read, unused
+          v[p][j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     rows, 4 * ((k * a.num_q_heads + head(p)) * D + d0), 0, kAgentScope));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // every load before the first use
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p) {
+        if (!pair_live(p)) continue;
+        if (s0 == 0) {
+          mx[p] = fmaxf(mx[p], ml[p].x);
+#pragma unroll
+          for (int m = 16; m >= 1; m >>= 1) mx[p] = fmaxf(mx[p], __shfl_xor(mx[p], m, 32));
+        }
+        // A split with no visible key (m = -inf) weighs 0; so does every split
+        // when none has one, and the output is then NaN (0 / 0).
+        const float w = ml[p].x == -INFINITY ? 0.f : exp2f(ml[p].x - mx[p]);
+        sum[p] += w * ml[p].y;
+#pragma unroll
+        for (int j = 0; j < CAP; ++j) {
+          const float wj = __shfl(w, j, 32);
+          if (s0 + j < ns) o[p] += v[p][j] * wj;
+        }
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      if (!pair_live(p)) continue;
+#pragma unroll
+      for (int m = 16; m >= 1; m >>= 1) sum[p] += __shfl_xor(sum[p], m, 32);
+      const float inv = 1.f / sum[p];
+      if (head_live(p) && has_dims) {
+        uint16_t* op = static_cast<uint16_t*>(a.out) + qs * a.o_s0 + static_cast<int64_t>(head(p)) * a.o_s1;
+        *reinterpret_cast<uint2*>(op + d0) =
+            uint2{Elem<T>::to_bits(o[p][0] * inv) | (Elem<T>::to_bits(o[p][1] * inv) << 16),
+                  Elem<T>::to_bits(o[p][2] * inv) | (Elem<T>::to_bits(o[p][3] * inv) << 16)};
+      }
+    }
+  }
+}
+
+// Epilogue shared by the decode kernels, entered by every wave of the
+// workgroup (`live`: the wave has a KV head). acc[b][e] is
+// O[head h*G + col][dim 16b + 4grp + e] (unnormalised), m / lt the running
 // max (exp2 domain) and the complete softmax denominator of this split. A
 // request with one split gets its output directly; otherwise the partial goes
-// to the workspace for the combine kernel.
+// to the workspace, and the workgroup that completes the request (for its
+// group of KV heads, `head_group`) merges the partials. `flag`: an LDS word
+// that no wave uses any more once all have entered.
 template <typename T, int D>
-__device__ __forceinline__ void write_decode_result(const AttnArgs& a, int64_t r, int64_t qs, int hq,
-                                                    int split, int64_t ns, float m, float lt,
-                                                    const float4_t (&acc)[D / 16], int grp) {
-  if (ns == 1) {
+__device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem& item, int h, bool live, int head_group,
+                                             int head_groups, float m, float lt, const float4_t (&acc)[D / 16],
+                                             int32_t* flag) {
+  const int col = threadIdx.x & 15;
+  const int grp = (threadIdx.x >> 4) & 3;
+  const int G = a.group;
+  if (item.ns == 1) {
+    if (!live || col >= G) return;
     const float inv = 1.f / lt;
-    uint16_t* op = static_cast<uint16_t*>(a.out) + qs * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
+    uint16_t* op = static_cast<uint16_t*>(a.out) + item.qs * a.o_s0 + static_cast<int64_t>(h * G + col) * a.o_s1;
 #pragma unroll
     for (int b = 0; b < D / 16; ++b) {
       const uint32_t w0 = Elem<T>::to_bits(acc[b][0] * inv) | (Elem<T>::to_bits(acc[b][1] * inv) << 16);
@@ -48,11 +167,81 @@ __device__ __forceinline__ void write_decode_result(const AttnArgs& a, int64_t r
     }
     return;
   }
-  const int64_t item = (r * a.max_splits + split) * a.num_q_heads + hq;
-  float* wp = a.ws_acc + item * D;
+  if (live && col < G) {
+    // Partial row of (this split, head h * G); the lanes' heads follow it.
+    const int64_t row = (static_cast<int64_t>(item.base) + item.split) * a.num_q_heads +
+                        static_cast<int64_t>(__builtin_amdgcn_readfirstlane(h)) * G;
+    const __amdgpu_buffer_rsrc_t rows = buffer_at(a.ws_acc + row * D);
 #pragma unroll
-  for (int b = 0; b < D / 16; ++b) *reinterpret_cast<float4_t*>(wp + 16 * b + 4 * grp) = acc[b];
-  if (grp == 0) a.ws_ml[item] = float2{m, lt};
+    for (int b = 0; b < D / 16; ++b)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_ext, acc[b]), rows, 4 * (col * D + 16 * b + 4 * grp), 0,
+                                             kAgentScope);
+    if (grp == 0)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(a.ws_ml) + row + col,
+                         static_cast<uint64_t>(__float_as_uint(m)) | (static_cast<uint64_t>(__float_as_uint(lt)) << 32),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // This wave's partials have reached the point all XCDs read from.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  int32_t* const counter = a.done + static_cast<int64_t>(item.r) * head_groups + head_group;
+  if (threadIdx.x == 0) {
+    const int32_t before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The last one leaves the counter at zero for the next launch.
+    if (before + 1 == item.ns) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = before + 1 == item.ns;
+  }
+  __syncthreads();
+  if (!*flag || !live) return;
+  const int hu = __builtin_amdgcn_readfirstlane(h);
+  if (item.ns <= 2) merge_splits<T, D, 2, false>(a, item.base, item.qs, hu, item.ns);
+  else if (item.ns <= 4) merge_splits<T, D, 4, false>(a, item.base, item.qs, hu, item.ns);
+  else if (item.ns <= 8) merge_splits<T, D, 8, false>(a, item.base, item.qs, hu, item.ns);
+  else if (item.ns <= 16) merge_splits<T, D, 16, false>(a, item.base, item.qs, hu, item.ns);
+  else if (item.ns <= 24) merge_splits<T, D, 24, false>(a, item.base, item.qs, hu, item.ns);
+  else merge_splits<T, D, 32, true>(a, item.base, item.qs, hu, item.ns);
+}
+
+// Output rows that no split writes, kTidyTokens tokens and as many requests
+// per workgroup `wg`: zeros for tokens outside every request (the reference's
+// zeros_like output), and NaN for a decode request with no visible key
+// (softmax over no keys) and, in a batch whose hint promised single-query
+// requests only, for the rows of any other request, which no kernel computes.
+constexpr int kTidyTokens = 16;
+
+inline int64_t tidy_blocks(const AttnArgs& a) {
+  const int64_t most = a.num_tokens > a.num_requests ? a.num_tokens : a.num_requests;
+  return (most + kTidyTokens - 1) / kTidyTokens;
+}
+
+template <typename T>
+__device__ inline void tidy_rows(const AttnArgs& a, int64_t wg) {
+  const int64_t R = a.num_requests;
+  const int64_t first = a.qsl[0], last = a.qsl[R];
+  // Rows are contiguous (16-byte aligned, head_dim a multiple of 8).
+  auto fill_row = [&](int64_t t, uint32_t bits2) {
+    uint16_t* op = static_cast<uint16_t*>(a.out) + t * a.o_s0;
+    const int chunks = a.head_dim / 8;
+    for (int i = threadIdx.x; i < a.num_q_heads * chunks; i += blockDim.x) {
+      const int hq = i / chunks, c = i - hq * chunks;
+      *reinterpret_cast<uint4*>(op + hq * a.o_s1 + 8 * c) = uint4{bits2, bits2, bits2, bits2};
+    }
+  };
+  const int64_t t0 = wg * kTidyTokens;
+  if (t0 < first || t0 + kTidyTokens > last) {
+    for (int64_t t = t0; t < t0 + kTidyTokens && t < a.num_tokens; ++t)
+      if (t < first || t >= last) fill_row(t, 0u);
+  }
+  const uint32_t nan_bits = Elem<T>::to_bits(NAN);
+  const uint32_t nan2 = nan_bits | (nan_bits << 16);
+  for (int64_t r = t0; r < t0 + kTidyTokens && r < R; ++r) {
+    const int2 req = a.decode_req[r];  // (query token, splits; -1: not a decode request)
+    if (req.y == 0 && req.x >= 0 && req.x < a.num_tokens) fill_row(req.x, nan2);
+    if (req.y >= 0 || !a.decode_only) continue;
+    const int64_t q0 = a.qsl[r], q1 = a.qsl[r + 1];
+    if (q0 < 0 || q1 > a.num_tokens) continue;
+    for (int64_t t = q0; t < q1; ++t) fill_row(t, nan2);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -68,7 +257,13 @@ __device__ __forceinline__ void write_decode_result(const AttnArgs& a, int64_t r
 // transposing V reads (8 rows, two neighbouring chunks). STAGES tiles per wave
 // are in flight; waits are explicit vmcnt counts because the only
 // vector-memory instructions in the loop are these tile loads (the split's
-// block ids are fetched once, up front). The loads carry the non-temporal
+// block ids are fetched once, up front).
+//
+// A lone wave's tile took 2,650 cycles when the loads of tile k + 1 were issued
+// from 64-bit lane addresses before tile k was read (issue 820, S 465, softmax
+// 440, P.V 800 behind its LDS reads); scalar load addresses, the tile read to
+// registers first and the refill issued behind those reads shorten it, and
+// keep a tile more in flight where HBM is the bound. The loads carry the non-temporal
 // hint: every K/V byte is read exactly once, and keeping the stream from
 // displacing other cached lines raised the measured bandwidth from 5.5 to
 // 6.0 TB/s on the Qwen3 decode batch.
@@ -119,12 +314,13 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
 
 typedef short tr_short4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) tr_short4 lds_tr_short4;
+typedef __attribute__((address_space(3))) const short8_t lds_short8;
 
 template <typename T, int D, int STAGES>
 __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t* smem, uint32_t wg, int waves) {
   constexpr int kTileBytes = kTileBytesOf<D>;
   constexpr int kLoads = D / 32;  // 1 KiB loads per K (or V) tile
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;
   const int grp = lane >> 4;
@@ -134,9 +330,14 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   // The work-list record carries the request's query token, visible range
   // and this split's key range, so the first tile loads wait on two
   // dependent loads (the record, then the block ids) rather than four.
-  const DecodeItem item = a.decode_items[wg / groups];
+  const int64_t slot = wg / groups;
+  if (slot >= a.item_capacity) {  // past the work list's capacity
+    tidy_rows<T>(a, static_cast<int64_t>(wg) - a.item_capacity * groups);
+    return;
+  }
+  const DecodeItem item = a.decode_items[slot];
   if (item.r < 0 || item.r >= a.num_requests) return;
-  if (h >= a.num_kv_heads) return;
+  const bool live = h < a.num_kv_heads;  // a spare wave only joins the epilogue's barriers
   const int split = item.split;
   const int64_t r = item.r;
   const int64_t qs = item.qs;
@@ -146,20 +347,36 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   // Records index the query, the table and the partials: out-of-range
   // fields (never written by the work-list kernel) end the workgroup.
   if (begin < 0 || begin > end || end - begin >= a.split_tokens || end >= a.width * a.block_size ||
-      qs < 0 || qs >= a.num_tokens || split < 0 || split >= a.max_splits)
+      qs < 0 || qs >= a.num_tokens || split < 0 || split >= item.ns || item.base < 0 ||
+      static_cast<int64_t>(item.base) + item.ns > a.item_capacity)
     return;
-  const int ntiles = static_cast<int>((end - begin) / 16 + 1);  // <= 128 (split <= 2048)
+  const int ntiles = live ? static_cast<int>((end - begin) / 16 + 1) : 0;  // <= 128 (split <= 2048)
 
   // Block id and in-block row of tiles `lane` and `lane + 64` of this split,
   // fetched once (block ids are < 2^31; a 16-aligned tile never straddles a
   // block).
   int32_t my_block[2] = {-1, -1}, my_row[2] = {0, 0};
+  if (a.page_shift >= 0) {
+    // A power-of-two number of 16-token pages per block: shifts instead of
+    // 64-bit divisions.
+    const int64_t* const table_row = a.table + r * a.t_s0;
+    int64_t id[2] = {-1, -1};
 #pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    if (lane + 64 * x < ntiles) {
-      const int64_t p = begin + 16 * (lane + 64 * x);
-      my_block[x] = static_cast<int32_t>(block_of(a, r, p));
-      my_row[x] = static_cast<int32_t>(p % a.block_size);
+    for (int x = 0; x < 2; ++x) {
+      const uint32_t page = (static_cast<uint32_t>(begin) >> 4) + lane + 64 * x;
+      my_row[x] = static_cast<int32_t>((page & ((1u << a.page_shift) - 1u)) << 4);
+      if (lane + 64 * x < ntiles) id[x] = table_row[static_cast<int64_t>(page >> a.page_shift) * a.t_s1];
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) my_block[x] = id[x] >= 0 && id[x] < a.num_blocks ? static_cast<int32_t>(id[x]) : -1;
+  } else {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      if (lane + 64 * x < ntiles) {
+        const int64_t p = begin + 16 * (lane + 64 * x);
+        my_block[x] = static_cast<int32_t>(block_of(a, r, p));
+        my_row[x] = static_cast<int32_t>(p % a.block_size);
+      }
     }
   }
   // Tile t's block id and row (t wave-uniform).
@@ -175,25 +392,26 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   short8_t qv[kLoads];
   {
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + qs * a.q_s0 +
-                         static_cast<int64_t>(col < G ? hq : 0) * a.q_s1 + 8 * grp;
+                         static_cast<int64_t>(live && col < G ? hq : 0) * a.q_s1 + 8 * grp;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
-      qv[i] = (col < G) ? *reinterpret_cast<const short8_t*>(qp + 32 * i) : short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      qv[i] = (live && col < G) ? *reinterpret_cast<const short8_t*>(qp + 32 * i) : short8_t{0, 0, 0, 0, 0, 0, 0, 0};
   }
 
   uint8_t* wave_lds = smem + static_cast<size_t>(wave) * STAGES * 2 * kTileBytes;
-  const uint32_t wave_lds_addr = lds_address(wave_lds);
+  const uint32_t wave_lds_addr = __builtin_amdgcn_readfirstlane(lds_address(wave_lds));
   const uint16_t* cache = static_cast<const uint16_t*>(a.cache);
   const int64_t head_elems = static_cast<int64_t>(h) * D;
 
   // Load-side mapping: instruction i, this lane -> 16-byte chunk 64i + lane of
-  // the tile's LDS slot (element offset of its data from the tile's first row).
-  int64_t lane_off[kLoads];
+  // the tile's LDS slot (byte offset of its data from the tile's first row;
+  // decode_supported's callers keep 16 rows within 32 bits).
+  uint32_t lane_off[kLoads];
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) {
     const int t = (64 * i + lane) / (D / 8);
     const int p = (64 * i + lane) % (D / 8);
-    lane_off[i] = t * a.c_s[2] + 8 * tile_logical<D>(t, p);
+    lane_off[i] = static_cast<uint32_t>(2 * (t * a.c_s[2] + 8 * tile_logical<D>(t, p)));
   }
   // Read-side byte offsets within a tile: K row `col`, chunk 4i + grp; and the
   // transposing V reads, in which lane 4k + c of a 16-lane group points at row
@@ -210,18 +428,22 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   auto issue = [&](int tile, int stage) {
     const int32_t blk = tile_block(tile);
     const int32_t row = tile_row(tile);
-    const uint32_t kdst = wave_lds_addr + stage * 2 * kTileBytes;
-    const uint32_t vdst = kdst + kTileBytes;
-    // An invalid block id masks the whole tile: read a valid dummy line instead.
-    const uint16_t* tile_k = blk >= 0 ? cache + static_cast<int64_t>(blk) * a.c_s[1] +
-                                            static_cast<int64_t>(row) * a.c_s[2] + head_elems
-                                      : cache;
-    const int64_t plane = blk >= 0 ? a.c_s[0] : 0;
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const uint16_t* src = blk >= 0 ? tile_k + lane_off[i] : cache;
-      lds_dma_load16_stream(src, kdst + i * 1024);
-      lds_dma_load16_stream(src + plane, vdst + i * 1024);
+    const uint32_t dst = wave_lds_addr + stage * 2 * kTileBytes;
+    // An invalid block id masks the whole tile: block 0 is read instead.
+    const int64_t at = blk >= 0 ? static_cast<int64_t>(blk) * a.c_s[1] + static_cast<int64_t>(row) * a.c_s[2] : 0;
+    const uint16_t* const tile_k = cache + at + head_elems;
+    const uint16_t* const tile_v = tile_k + a.c_s[0];
+    lds_dma_load16_stream<0>(tile_k, lane_off[0], dst);
+    lds_dma_load16_stream<kTileBytes>(tile_v, lane_off[0], dst);
+    lds_dma_load16_stream<1024>(tile_k, lane_off[1], dst);
+    lds_dma_load16_stream<kTileBytes + 1024>(tile_v, lane_off[1], dst);
+    if constexpr (kLoads > 2) {
+      lds_dma_load16_stream<2048>(tile_k, lane_off[2], dst);
+      lds_dma_load16_stream<kTileBytes + 2048>(tile_v, lane_off[2], dst);
+    }
+    if constexpr (kLoads > 3) {
+      lds_dma_load16_stream<3072>(tile_k, lane_off[3], dst);
+      lds_dma_load16_stream<kTileBytes + 3072>(tile_v, lane_off[3], dst);
     }
   };
 
@@ -233,41 +455,50 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   // The block ids and Q must be in registers before the first tile address.
   __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
+  for (int s = 0; s < STAGES; ++s)
     if (s < ntiles) issue(s, s);
 
   for (int k = 0; k < ntiles; ++k) {
     const int stage = k % STAGES;
-    const int ahead = k + STAGES - 1;
-    if (ahead < ntiles) {
-      // The stage being refilled, (k - 1) % STAGES, was read in the previous
-      // iteration. Its LDS reads have retired only because that iteration
-      // ended with an lgkmcnt(0) wait; that wait is what makes the refill safe.
-      issue(ahead, ahead % STAGES);
-    }
     const int later = (ntiles - 1 - k) < (STAGES - 1) ? (ntiles - 1 - k) : (STAGES - 1);
     wait_tiles<2 * kLoads>(later);
     __builtin_amdgcn_wave_barrier();
     compiler_fence();
 
-    const int64_t tb = begin + 16 * static_cast<int64_t>(k);
-    const int64_t blk = tile_block(k);
+    // The whole tile goes to registers first, so that its stage refills while
+    // it is computed (STAGES tiles in flight throughout) and the V reads do
+    // not wait behind the softmax.
+    const uint32_t kt = wave_lds_addr + stage * 2 * kTileBytes;
+    const uint32_t vt = kt + kTileBytes;
+    short8_t kf[kLoads];
+    uint2 vf[D / 16];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      kf[i] = *reinterpret_cast<lds_short8*>(static_cast<uintptr_t>(kt + koff[i]));
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) {
+      // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
+      vf[b] = __builtin_bit_cast(
+          uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(vt + voff[b]))));
+    }
+    // All LDS reads of this stage retire before the refill is issued.
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    compiler_fence();
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + STAGES < ntiles) issue(k + STAGES, stage);
+
+    const int32_t tb = static_cast<int32_t>(begin) + 16 * k;
     // Token j of the tile is visible iff its position is in [lo, end] and the block is valid.
     uint32_t okmask = 0;
-    if (blk >= 0) {
-      const int64_t first_ok = lo > tb ? lo - tb : 0;
-      const int64_t last_ok = end - tb < 15 ? end - tb : 15;
+    if (tile_block(k) >= 0) {
+      const int32_t first_ok = lo > tb ? static_cast<int32_t>(lo) - tb : 0;
+      const int32_t last_ok = end - tb < 15 ? static_cast<int32_t>(end) - tb : 15;
       okmask = (last_ok >= first_ok) ? ((0xFFFFu >> (15 - last_ok)) & (0xFFFFu << first_ok)) : 0u;
     }
-    const uint8_t* kt = wave_lds + stage * 2 * kTileBytes;
-    const uint32_t vt = wave_lds_addr + stage * 2 * kTileBytes + kTileBytes;
 
     float4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const short8_t kk = *reinterpret_cast<const short8_t*>(kt + koff[i]);
-      sc = Mfma<T>::k32(kk, qv[i], sc);
-    }
+    for (int i = 0; i < kLoads; ++i) sc = Mfma<T>::k32(kf[i], qv[i], sc);
     float s[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -275,10 +506,12 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
     float bm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
     bm = max_xor32_f(max_xor16_f(bm));
     const float mn = fmaxf(m, bm);
-    const float alpha = (mn == -INFINITY) ? 1.f : exp2f(m - mn);
+    // v_exp_f32 flushes results below 2^-126 to zero: nothing beside the
+    // row's maximum of 1.
+    const float alpha = (mn == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m - mn);
     float p[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = (s[e] == -INFINITY) ? 0.f : exp2f(s[e] - mn);
+    for (int e = 0; e < 4; ++e) p[e] = (s[e] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s[e] - mn);
     l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     if (__ballot(alpha != 1.f)) {
 #pragma unroll
@@ -291,26 +524,24 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
     for (int e = 0; e < 4; ++e) split_hi_lo<T>(p[e], ph[e], pl[e]);
     const short4_t pb_hi = __builtin_bit_cast(short4_t, uint2{ph[0] | (ph[1] << 16), ph[2] | (ph[3] << 16)});
     const short4_t pb_lo = __builtin_bit_cast(short4_t, uint2{pl[0] | (pl[1] << 16), pl[2] | (pl[3] << 16)});
-    // Rows of masked tokens may hold stale or non-finite data: zero them in V.
-    const uint32_t mlo = ((okmask >> (4 * grp)) & 1u ? 0xFFFFu : 0u) | ((okmask >> (4 * grp + 1)) & 1u ? 0xFFFF0000u : 0u);
-    const uint32_t mhi = ((okmask >> (4 * grp + 2)) & 1u ? 0xFFFFu : 0u) | ((okmask >> (4 * grp + 3)) & 1u ? 0xFFFF0000u : 0u);
+    if (okmask != 0xFFFFu) {
+      // Rows of masked tokens may hold stale or non-finite data: zero them in V.
+      const uint32_t ok4 = okmask >> (4 * grp);
+      const uint32_t mlo = (ok4 & 1u ? 0xFFFFu : 0u) | (ok4 & 2u ? 0xFFFF0000u : 0u);
+      const uint32_t mhi = (ok4 & 4u ? 0xFFFFu : 0u) | (ok4 & 8u ? 0xFFFF0000u : 0u);
 #pragma unroll
-    for (int b = 0; b < D / 16; ++b) {
-      // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
-      const uint2 rv = __builtin_bit_cast(
-          uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(vt + voff[b]))));
-      const short4_t av = __builtin_bit_cast(short4_t, uint2{rv.x & mlo, rv.y & mhi});
-      acc[b] = Mfma<T>::k16(av, pb_hi, acc[b]);
-      acc[b] = Mfma<T>::k16(av, pb_lo, acc[b]);
+      for (int b = 0; b < D / 16; ++b) vf[b] = uint2{vf[b].x & mlo, vf[b].y & mhi};
     }
-    // All LDS reads of this stage must retire before a later issue refills it.
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    compiler_fence();
+    // Both products of a block depend on each other, the blocks do not.
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_hi, acc[b]);
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_lo, acc[b]);
   }
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
-  if (col >= G) return;
-  write_decode_result<T, D>(a, r, qs, hq, split, item.ns, m, lt, acc, grp);
+  // The flag lies in the first wave's K tile: written after every wave's loop.
+  finish_split<T, D>(a, item, h, live, static_cast<int>(wg % groups), groups, m, lt, acc, reinterpret_cast<int32_t*>(smem));
 }
 
 }  // namespace dec

@@ -84,78 +84,154 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 // One workgroup lists the (request, split) items of the single-query
 // requests: every full split first (in any order), then the partial last
 // splits from the largest down, so the in-order dispatch of the decode grid
-// ends on the shortest items. Empty slots (up to R * max_splits) get
-// request -1.
+// ends on the shortest items. Empty slots (up to the capacity) get request -1.
+//
+// The split length follows from the visible tokens, which only the device
+// knows. A split costs a workgroup ~5 us besides its tiles (metadata, the
+// pipeline's start, the partial and its merge), and a tile of a workgroup that
+// has a CU to itself ~0.65 us. So (times per forward, captured back to back):
+// * while the work does not fill the chip, as many items as the CUs take at
+//   one workgroup each (96 items: two workgroups of four KV heads per item at
+//   8 KV heads), of 64 to 256 tokens. 8 contexts of 128 .. 4,096: 36.1 us with
+//   64-token splits, 23.3 with 192, 34.1 with 512; one context of 1,024: 13.7
+//   with 64, 21.0 with 256;
+// * beyond that, about two items per CU of up to 1,024 tokens (64 contexts of
+//   8k .. 33k: 868 us, 907 with 2,048; 256 of 128 .. 4,096: 361, 379 with
+//   256), or, beside prefill work, whose workgroups fill the chip as well,
+//   half an item per CU of up to 2,048 (248 decodes and 8 chunks of 512: 736
+//   us with 2,048, 781 with 512);
+// * at most 32 splits per request up to 512 tokens each: the merge loads 32
+//   at a time (one context of 32k: 143 us with 64-token splits, 47 with 512).
+// At least total / (capacity - R), so that the items fit the list: a request
+// of v tokens has at most v / split + 1 splits. (2,048-token splits always fit:
+// see item_slots.)
 constexpr int kDecodeListThreads = 1024;
 constexpr int kSizeBuckets = 64;  // sizes of a partial split, split / 64 tokens (rounded up to a power of two) each
 
+// (The figures are for head_dim 128; narrower tokens count by their bytes.)
+constexpr int32_t kSmallItems = 96, kSmallSplit = 64, kFullSplit = 256, kMostSplit = 1024;
+
+// Slots of the decode work list and of the decode grid, from shapes alone: at
+// most `capacity` (the workspace's) and no more than choose_split can fill. A
+// slot that stays empty still costs a workgroup's dispatch (~4 ns: 1,500 of
+// them took 6 of the 37 us of 30 decodes and two chunks at head_dim 64).
+// Splits of 2,048 tokens fit every one of the bounds.
+inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int64_t cus, int64_t head_dim) {
+  auto least = [](int64_t x, int64_t y) { return x < y ? x : y; };
+  auto larger = [](int64_t x, int64_t y) { return x > y ? x : y; };
+  const int64_t tokens = requests * reach;
+  const int64_t small = kSmallItems * 128 / head_dim + 1;
+  const int64_t full = least(2 * cus * 128 / head_dim, tokens / kFullSplit) + 1;
+  const int64_t slots = requests + larger(larger(small, full), tokens / kMostSplit + 1);
+  return least(least(slots, requests * ((reach + kSmallSplit - 1) / kSmallSplit)), capacity);
+}
+
+__device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t requests, int64_t capacity,
+                                       int32_t cus, int32_t head_dim, bool beside_prefill) {
+  // Quotients in float (a 64-bit division takes longer than the rest of the
+  // rule), raised by more than their error; lengths past 2^20 mean the same.
+  auto up16 = [](float v) { return (static_cast<int32_t>(fminf(v * 1.000001f, 1048576.f)) + 16) & ~15; };
+  const float tokens = static_cast<float>(total);
+  const float wide = tokens * head_dim / 128.f;
+  const int32_t most = beside_prefill ? kMaxSplit : kMostSplit;
+  int32_t split = up16(wide / (beside_prefill ? 0.5f * cus : 2.f * cus));
+  int32_t least = up16(wide / kSmallItems);
+  least = least < kSmallSplit ? kSmallSplit : least > kFullSplit ? kFullSplit : least;
+  split = split < least ? least : split > most ? most : split;
+  const int32_t by_merge = (longest / 32 + 16) & ~15;
+  if (split < by_merge) split = by_merge < 512 ? by_merge : split < 512 ? 512 : split;
+  const int32_t fits = capacity > requests ? up16(tokens / static_cast<float>(capacity - requests)) : kMaxSplit;
+  if (split < fits) split = fits;
+  return split < kMaxSplit ? split : kMaxSplit;
+}
+
 __device__ inline void build_decode_list(const AttnArgs& a) {
-  __shared__ int32_t full_count, full_pos;
+  __shared__ int32_t full_count, full_pos, base_pos, longest, others;
+  __shared__ unsigned long long pages;
   __shared__ int32_t bucket[kSizeBuckets];
   const int tid = threadIdx.x;
   const int64_t R = a.num_requests;
-  const int64_t capacity = R * a.max_splits;
-  // 64 buckets of 2^bucket_shift sizes span every split length: the
-  // smallest shift with 64 << shift >= split_tokens (a partial split holds
-  // 1 .. split_tokens - 1 keys, so its bucket index stays below 64).
-  int bucket_shift = 0;
-  while ((kSizeBuckets << bucket_shift) < a.split_tokens) ++bucket_shift;
-  if (tid == 0) full_count = full_pos = 0;
+  const int64_t capacity = a.item_capacity;
+  if (tid == 0) {
+    full_count = full_pos = base_pos = longest = others = 0;
+    pages = 0;
+  }
   if (tid < kSizeBuckets) bucket[tid] = 0;
-  // A decode request: its query token, visible keys, split count and the
-  // size of its last split (ns = 0: not a decode request, or no visible key;
+  // A decode request: its query token, visible keys and their number from the
+  // 16-aligned position below the first (0: none, or not a decode request;
   // dec = 1 marks a decode request).
   struct Desc {
-    int32_t qs, lo, hi, ns, last, dec;
+    int32_t qs, lo, hi, tokens, dec;
   };
+  const Desc none = {0, 0, -1, 0, 0};
   auto describe = [&](int64_t r) {
-    Desc d = {0, 0, -1, 0, 0, 0};
+    Desc d = none;
     const int64_t qs = a.qsl[r];
     if (qs < 0 || qs >= a.num_tokens || a.qsl[r + 1] - qs != 1) return d;
     d.qs = static_cast<int32_t>(qs);
     d.dec = 1;
     int64_t lo, hi;
     visible_range(a, r, qs, qs, lo, hi);
-    const int64_t n = decode_num_splits(lo, hi, a.split_tokens);
-    if (n <= 0) return d;
+    if (hi < lo) return d;
     d.lo = static_cast<int32_t>(lo);
     d.hi = static_cast<int32_t>(hi);
-    d.ns = static_cast<int32_t>(n);
-    d.last = static_cast<int32_t>((hi - (lo & ~int64_t(15)) + 1) - (n - 1) * a.split_tokens);
+    d.tokens = static_cast<int32_t>(hi - (lo & ~int64_t(15)) + 1);
     return d;
   };
-  auto record = [&](int64_t r, const Desc& d, int32_t sp) {
-    const int32_t begin = (d.lo & ~15) + sp * a.split_tokens;
-    const int32_t end = begin + a.split_tokens - 1 < d.hi ? begin + a.split_tokens - 1 : d.hi;
-    return DecodeItem{static_cast<int32_t>(r), sp, d.qs, d.ns, d.lo, d.hi, begin, end};
-  };
   // The thread's first request stays in registers between the passes.
-  Desc d0 = {0, 0, -1, 0, 0, 0};
-  if (tid < R) d0 = describe(tid);
+  const Desc d0 = tid < R ? describe(tid) : none;
+  auto desc_of = [&](int64_t r) { return r >= R ? none : r == tid ? d0 : describe(r); };
   __syncthreads();
   const int lane = tid & 63;
   // Exclusive prefix of v over the wave and the wave's total.
-  auto wave_scan = [&](int32_t v, int32_t& total) {
+  auto wave_scan = [&](int32_t v, int32_t& sum) {
     int32_t incl = v;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const int32_t y = __shfl_up(incl, d, 64);
       if (lane >= d) incl += y;
     }
-    total = __shfl(incl, 63, 64);
+    sum = __shfl(incl, 63, 64);
     return incl - v;
   };
+  // Pass 0: visible 16-token pages in all, the longest range, and whether any
+  // request is not a decode. The loop bounds are uniform per wave. A wave sums
+  // the low 16 bits of its page counts and the rest apart, so neither
+  // overflows.
+  const auto add = [](int32_t x, int32_t y) { return x + y; };
+  const auto larger = [](int32_t x, int32_t y) { return x > y ? x : y; };
+  int32_t split = a.split_fixed;
+  if (split == 0) {
+    for (int64_t r0 = tid - lane; r0 < R; r0 += kDecodeListThreads) {
+      const Desc d = desc_of(r0 + lane);
+      const int32_t count = (d.tokens >> 4) + ((d.tokens & 15) != 0);
+      const int32_t low = wave_reduce_i(count & 0xFFFF, add);
+      const int32_t high = wave_reduce_i(count >> 16, add);
+      const int32_t most = wave_reduce_i(d.tokens, larger);
+      const bool other = __ballot(r0 + lane < R && !d.dec) != 0;
+      if (lane == 0) {
+        atomicAdd(&pages, (static_cast<unsigned long long>(high) << 16) + low);
+        atomicMax(&longest, most);
+        if (other) others = 1;
+      }
+    }
+    __syncthreads();
+    split = choose_split(16 * static_cast<int64_t>(pages), longest, R, capacity, a.num_cus, a.head_dim, others && !a.decode_only);
+  }
+  // 64 buckets of 2^bucket_shift sizes span every split length: the smallest
+  // shift with 64 << shift >= split (a partial split holds 1 .. split - 1
+  // keys, so its bucket index stays below 64).
+  const int bucket_shift = split <= kSizeBuckets ? 0 : 32 - __builtin_clz((split - 1) / kSizeBuckets);
+  auto splits_of = [&](const Desc& d) { return (d.tokens + split - 1) / split; };
   // Pass 1: count full splits (one LDS atomic per wave), histogram the
-  // partial ones by size. The loop bound is uniform per wave.
+  // partial ones by size.
   for (int64_t r0 = tid - lane; r0 < R; r0 += kDecodeListThreads) {
-    const int64_t r = r0 + lane;
-    Desc d = {0, 0, -1, 0, 0, 0};
-    if (r < R) d = r == tid ? d0 : describe(r);
-    const int32_t ns = d.ns, last = d.last;
-    const bool partial = ns > 0 && last < a.split_tokens;
-    int32_t total;
-    wave_scan(partial ? ns - 1 : ns, total);
-    if (lane == 0 && total) atomicAdd(&full_count, total);
+    const Desc d = desc_of(r0 + lane);
+    const int32_t ns = splits_of(d);
+    const int32_t last = d.tokens - (ns - 1) * split;
+    const bool partial = ns > 0 && last < split;
+    const int32_t sum = wave_reduce_i(partial ? ns - 1 : ns, add);
+    if (lane == 0 && sum) atomicAdd(&full_count, sum);
     if (partial) atomicAdd(&bucket[(last - 1) >> bucket_shift], 1);
   }
   __syncthreads();
@@ -164,36 +240,46 @@ __device__ inline void build_decode_list(const AttnArgs& a) {
   static_assert(kSizeBuckets == 64, "one wave scans the buckets");
   if (tid < 64) {
     const int32_t c = bucket[63 - tid];
-    int32_t incl = c;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int32_t y = __shfl_up(incl, d, 64);
-      if (tid >= d) incl += y;
-    }
+    int32_t sum;
+    const int32_t excl = wave_scan(c, sum);
     const int32_t fulls = full_count;
-    bucket[63 - tid] = fulls + incl - c;
-    if (tid == 63) full_count = fulls + incl;  // total number of items
+    bucket[63 - tid] = fulls + excl;
+    if (tid == 63) full_count = fulls + sum;  // total number of items
   }
   __syncthreads();
-  // Pass 2: place the items (one LDS atomic per wave for the full splits).
+  // Pass 2: place the items (one LDS atomic per wave for the full splits and
+  // one for the requests' partial rows).
   for (int64_t r0 = tid - lane; r0 < R; r0 += kDecodeListThreads) {
     const int64_t r = r0 + lane;
-    Desc d = {0, 0, -1, 0, 0, 0};
-    if (r < R) d = r == tid ? d0 : describe(r);
-    const int32_t ns = d.ns, last = d.last;
-    const bool partial = ns > 0 && last < a.split_tokens;
+    const Desc d = desc_of(r);
+    const int32_t ns = splits_of(d);
+    const int32_t last = d.tokens - (ns - 1) * split;
+    const bool partial = ns > 0 && last < split;
     const int32_t nfull = partial ? ns - 1 : ns;
-    int32_t total;
-    const int32_t excl = wave_scan(nfull, total);
-    int32_t at = 0;
-    if (lane == 0 && total) at = atomicAdd(&full_pos, total);
-    at = __shfl(at, 0, 64) + excl;
-    for (int32_t sp = 0; sp < nfull; ++sp) a.decode_items[at + sp] = record(r, d, sp);
-    if (partial) a.decode_items[atomicAdd(&bucket[(last - 1) >> bucket_shift], 1)] = record(r, d, ns - 1);
+    int32_t rows;
+    const int32_t row_excl = wave_scan(ns, rows);
+    const uint64_t partials = __ballot(partial);
+    const int32_t before = __popcll(partials & ((uint64_t{1} << lane) - 1));  // partial splits of lower lanes
+    int32_t at = 0, base = 0;
+    if (lane == 0 && rows) {
+      at = atomicAdd(&full_pos, rows - static_cast<int32_t>(__popcll(partials)));
+      base = atomicAdd(&base_pos, rows);
+    }
+    at = __builtin_amdgcn_readfirstlane(at) + row_excl - before;
+    base = __builtin_amdgcn_readfirstlane(base) + row_excl;
+    auto place = [&](int32_t slot, int32_t sp) {
+      const int32_t begin = (d.lo & ~15) + sp * split;
+      const int32_t end = begin + split - 1 < d.hi ? begin + split - 1 : d.hi;
+      if (slot < capacity) a.decode_items[slot] = DecodeItem{static_cast<int32_t>(r), sp, d.qs, ns, d.lo, base, begin, end};
+    };
+    for (int32_t sp = 0; sp < nfull; ++sp) place(at + sp, sp);
+    if (partial) place(atomicAdd(&bucket[(last - 1) >> bucket_shift], 1), ns - 1);
     if (r < R) a.decode_req[r] = int2{d.qs, d.dec ? ns : -1};
   }
+  // At most one counter per (request, KV head).
+  for (int64_t j = tid; j < R * a.num_kv_heads; j += kDecodeListThreads) a.done[j] = 0;
   for (int64_t j = full_count + tid; j < capacity; j += kDecodeListThreads)
-    a.decode_items[j] = DecodeItem{-1, -1, 0, 0, 0, -1, 0, -1};
+    a.decode_items[j] = DecodeItem{-1, -1, 0, 0, 0, 0, 0, -1};
 }
 
 
