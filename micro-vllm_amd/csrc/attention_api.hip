@@ -312,7 +312,7 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
   a.num_cus = device_cu_count();
   a.item_capacity = a.split_fixed ? d.item_capacity
                                   : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
-                                               d.item_capacity, a.num_cus, D);
+                                               d.item_capacity, a.num_cus, D, a.num_kv_heads);
   a.decode_only = batch->max_query_len == 1 ? 1 : 0;
   a.ws_acc = reinterpret_cast<float*>(w);
   a.ws_ml = reinterpret_cast<float2*>(w + d.acc_bytes);

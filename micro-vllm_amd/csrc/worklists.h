@@ -95,6 +95,8 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 //   8 KV heads), of 64 to 256 tokens. 8 contexts of 128 .. 4,096: 36.1 us with
 //   64-token splits, 23.3 with 192, 34.1 with 512; one context of 1,024: 13.7
 //   with 64, 21.0 with 256;
+//   (With one KV head an item is one wave: up to 128 tokens then; 209 decodes
+//   of 55 .. 542 with 16 heads on one: 23.4 us with 128, 27.0 with 256.)
 // * beyond that, about two items per CU of up to 1,024 tokens (64 contexts of
 //   8k .. 33k: 868 us, 907 with 2,048; 256 of 128 .. 4,096: 361, 379 with
 //   256), or, beside prefill work, whose workgroups fill the chip as well,
@@ -109,25 +111,27 @@ constexpr int kDecodeListThreads = 1024;
 constexpr int kSizeBuckets = 64;  // sizes of a partial split, split / 64 tokens (rounded up to a power of two) each
 
 // (The figures are for head_dim 128; narrower tokens count by their bytes.)
-constexpr int32_t kSmallItems = 96, kSmallSplit = 64, kFullSplit = 256, kMostSplit = 1024;
+constexpr int32_t kSmallItems = 96, kSmallSplit = 64, kMostSplit = 1024;
+__host__ __device__ inline int32_t full_split(int32_t num_kv_heads) { return num_kv_heads == 1 ? 128 : 256; }
 
 // Slots of the decode work list and of the decode grid, from shapes alone: at
 // most `capacity` (the workspace's) and no more than choose_split can fill. A
 // slot that stays empty still costs a workgroup's dispatch (~4 ns: 1,500 of
 // them took 6 of the 37 us of 30 decodes and two chunks at head_dim 64).
 // Splits of 2,048 tokens fit every one of the bounds.
-inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int64_t cus, int64_t head_dim) {
+inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int64_t cus, int64_t head_dim,
+                          int32_t num_kv_heads) {
   auto least = [](int64_t x, int64_t y) { return x < y ? x : y; };
   auto larger = [](int64_t x, int64_t y) { return x > y ? x : y; };
   const int64_t tokens = requests * reach;
   const int64_t small = kSmallItems * 128 / head_dim + 1;
-  const int64_t full = least(2 * cus * 128 / head_dim, tokens / kFullSplit) + 1;
+  const int64_t full = least(2 * cus * 128 / head_dim, tokens / full_split(num_kv_heads)) + 1;
   const int64_t slots = requests + larger(larger(small, full), tokens / kMostSplit + 1);
   return least(least(slots, requests * ((reach + kSmallSplit - 1) / kSmallSplit)), capacity);
 }
 
 __device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t requests, int64_t capacity,
-                                       int32_t cus, int32_t head_dim, bool beside_prefill) {
+                                       int32_t cus, int32_t head_dim, int32_t num_kv_heads, bool beside_prefill) {
   // Quotients in float (a 64-bit division takes longer than the rest of the
   // rule), raised by more than their error; lengths past 2^20 mean the same.
   auto up16 = [](float v) { return (static_cast<int32_t>(fminf(v * 1.000001f, 1048576.f)) + 16) & ~15; };
@@ -136,7 +140,8 @@ __device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t r
   const int32_t most = beside_prefill ? kMaxSplit : kMostSplit;
   int32_t split = up16(wide / (beside_prefill ? 0.5f * cus : 2.f * cus));
   int32_t least = up16(wide / kSmallItems);
-  least = least < kSmallSplit ? kSmallSplit : least > kFullSplit ? kFullSplit : least;
+  const int32_t full = full_split(num_kv_heads);
+  least = least < kSmallSplit ? kSmallSplit : least > full ? full : least;
   split = split < least ? least : split > most ? most : split;
   const int32_t by_merge = (longest / 32 + 16) & ~15;
   if (split < by_merge) split = by_merge < 512 ? by_merge : split < 512 ? 512 : split;
@@ -216,7 +221,8 @@ __device__ inline void build_decode_list(const AttnArgs& a) {
       }
     }
     __syncthreads();
-    split = choose_split(16 * static_cast<int64_t>(pages), longest, R, capacity, a.num_cus, a.head_dim, others && !a.decode_only);
+    split = choose_split(16 * static_cast<int64_t>(pages), longest, R, capacity, a.num_cus, a.head_dim,
+                         a.num_kv_heads, others && !a.decode_only);
   }
   // 64 buckets of 2^bucket_shift sizes span every split length: the smallest
   // shift with 64 << shift >= split (a partial split holds 1 .. split - 1
