@@ -9,6 +9,7 @@ entry point raises ``NativeLibraryError``.
 from __future__ import annotations
 
 import ctypes
+import struct
 import threading
 from pathlib import Path
 
@@ -308,4 +309,79 @@ def kv_cache(cache: torch.Tensor, block_size: int | None = None) -> KVCache:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on ``device``."""
+
+    index = device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+# ---- packed descriptors -------------------------------------------------------
+#
+# The per-layer calls take their descriptors as packed bytes of the same
+# layout as the structures above: one struct.pack per descriptor instead of a
+# ctypes object filled field by field (an attention call's six descriptors
+# took two thirds of its ~22 us of host time that way, more than its kernels
+# run on a small batch). The library only reads them.
+
+_PACK_TENSOR3 = struct.Struct("=Qii3q3q")
+_PACK_KV_CACHE = struct.Struct("=Qii4q5q")
+_PACK_BATCH = struct.Struct("=6Q3q2q2q")
+assert _PACK_TENSOR3.size == ctypes.sizeof(Tensor3)
+assert _PACK_KV_CACHE.size == ctypes.sizeof(KVCache)
+assert _PACK_BATCH.size == ctypes.sizeof(Batch)
+
+_PACKED_ARGTYPES = {
+    "mvllm_attention_workspace_bytes": [ctypes.c_char_p, _i64, _i64],
+    "mvllm_attention_forward": [ctypes.c_char_p] * 6 + [ctypes.c_float, _ptr, _i64, _ptr],
+    "mvllm_qk_norm_rope_kv_write": [ctypes.c_char_p] * 3
+    + [_ptr, _ptr, _ptr, _ptr, _ptr, _i64, ctypes.c_float, _ptr, ctypes.c_char_p, _ptr, _ptr],
+}
+_packed: dict = {}
+
+
+def packed(name: str):
+    """The library's function ``name`` with packed-descriptor arguments."""
+
+    function = _packed.get(name)
+    if function is None:
+        lib = load()
+        function = lib[name]  # a function object of its own, beside the attribute
+        function.argtypes = _PACKED_ARGTYPES[name]
+        function.restype = getattr(lib, name).restype
+        _packed[name] = function
+    return function
+
+
+def pack_tensor3(t: torch.Tensor) -> bytes:
+    """``tensor3`` as packed bytes."""
+
+    shape = t.shape
+    if len(shape) != 3:
+        raise ValueError(f"expected a 3-D [tokens, heads, dim] tensor, got shape {tuple(shape)}")
+    code = _TORCH_DTYPES.get(t.dtype)
+    if code is None:
+        code = dtype_code(t.dtype)
+    return _PACK_TENSOR3.pack(0 if 0 in shape else t.data_ptr(), code, 0, *shape, *t.stride())
+
+
+def pack_kv_cache(cache: torch.Tensor) -> bytes:
+    """``kv_cache`` as packed bytes."""
+
+    shape = cache.shape
+    if len(shape) != 5 or shape[0] != 2:
+        raise ValueError(
+            "layer_kv_cache must be shaped (2, num_blocks, block_size, num_kv_heads, head_dim), "
+            f"got {tuple(shape)}"
+        )
+    _, blocks, block_size, heads, dim = shape
+    return _PACK_KV_CACHE.pack(
+        cache.data_ptr(), dtype_code(cache.dtype), 0, blocks, block_size, heads, dim, *cache.stride()
+    )
+
+
+def pack_batch(pointers: tuple, counts: tuple, table_stride: tuple, block_size: int, max_query_len: int) -> bytes:
+    """A ``Batch``: six pointers (0: none), (tokens, requests, table width)."""
+
+    return _PACK_BATCH.pack(*pointers, *counts, *table_stride, block_size, max_query_len)

@@ -24,18 +24,22 @@ from micro_vllm_amd.attention.operators.base import AttentionOperator
 SUPPORTED_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 
+_INT64 = torch.int64
+
+
 def _index(t: torch.Tensor, name: str, device: torch.device) -> torch.Tensor:
-    if t.dtype != torch.int64:
+    if t.dtype is not _INT64:
         raise ValueError(f"metadata.{name} must be int64, got {t.dtype}")
     if t.device != device:
         raise RuntimeError(f"metadata.{name} is on {t.device}, expected {device}")
-    return t if t.dim() != 1 or t.is_contiguous() else t.contiguous()
+    return t if t.is_contiguous() or t.dim() != 1 else t.contiguous()
 
 
-def batch_descriptor(metadata: AttentionMetadata, device: torch.device) -> tuple[_native.Batch, list]:
-    """C-ABI view of ``metadata``; the list keeps any made-contiguous copies alive."""
+def _batch_fields(metadata: AttentionMetadata, device: torch.device) -> tuple[tuple, tuple, tuple, int, int, tuple]:
+    """(pointers, (tokens, requests, table width), table strides, block size,
+    max_query_len) of ``metadata`` in ``Batch`` order, checked; and the tensors
+    whose memory the pointers name (made contiguous where they were not)."""
 
-    keep = []
     positions = _index(metadata.query_positions, "query_positions", device)
     starts = _index(metadata.query_context_start_positions, "query_context_start_positions", device)
     qsl = _index(metadata.query_start_locations, "query_start_locations", device)
@@ -49,28 +53,35 @@ def batch_descriptor(metadata: AttentionMetadata, device: torch.device) -> tuple
         raise ValueError(
             f"query_start_locations has {qsl.numel()} entries for {num_requests} requests"
         )
-    if table.shape[0] < num_requests:
-        raise ValueError(f"block_table has {table.shape[0]} rows for {num_requests} requests")
+    rows, width = table.shape
+    if rows < num_requests:
+        raise ValueError(f"block_table has {rows} rows for {num_requests} requests")
     num_tokens = positions.numel()
     if starts.numel() != num_tokens or slots.numel() != num_tokens:
         raise ValueError("query positions, context starts and slot_mapping differ in length")
-    keep.extend((positions, starts, qsl, lengths, slots, table))
-    b = _native.Batch()
-    b.query_positions = positions.data_ptr() if num_tokens else None
-    b.query_context_start_positions = starts.data_ptr() if num_tokens else None
-    b.query_start_locations = qsl.data_ptr()
-    b.context_lengths = lengths.data_ptr() if num_requests else None
-    b.block_table = table.data_ptr() if table.numel() else None
-    b.slot_mapping = slots.data_ptr() if num_tokens else None
-    b.num_tokens = num_tokens
-    b.num_requests = num_requests
-    b.block_table_width = table.shape[1]
-    b.block_table_stride[0] = table.stride(0)
-    b.block_table_stride[1] = table.stride(1)
-    b.block_size = metadata.block_size
     hint = getattr(metadata, "max_query_len", None)
-    b.max_query_len = hint if hint is not None else -1
-    return b, keep
+    return (
+        (
+            positions.data_ptr() if num_tokens else 0,
+            starts.data_ptr() if num_tokens else 0,
+            qsl.data_ptr(),
+            lengths.data_ptr() if num_requests else 0,
+            table.data_ptr() if rows and width else 0,
+            slots.data_ptr() if num_tokens else 0,
+        ),
+        (num_tokens, num_requests, width),
+        table.stride(),
+        metadata.block_size,
+        hint if hint is not None else -1,
+        (positions, starts, qsl, lengths, slots, table),
+    )
+
+
+def batch_descriptor(metadata: AttentionMetadata, device: torch.device) -> tuple[_native.Batch, list]:
+    """C-ABI view of ``metadata``; the list keeps any made-contiguous copies alive."""
+
+    *fields, keep = _batch_fields(metadata, device)
+    return _native.Batch.from_buffer_copy(_native.pack_batch(*fields)), list(keep)
 
 
 def _check_inputs(
@@ -87,11 +98,12 @@ def _check_inputs(
             "mi355x_paged attention supports torch.bfloat16, torch.float16 and torch.float32, "
             f"got {query.dtype}"
         )
+    device, dtype = query.device, query.dtype
     for name, t in (("key", key), ("value", value), ("layer_kv_cache", layer_kv_cache)):
-        if t.device != query.device:
-            raise RuntimeError(f"{name} is on {t.device}, query on {query.device}")
-        if t.dtype != query.dtype:
-            raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {query.dtype}")
+        if t.device != device:
+            raise RuntimeError(f"{name} is on {t.device}, query on {device}")
+        if t.dtype != dtype:
+            raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {dtype}")
     if layer_kv_cache.dim() != 5 or layer_kv_cache.shape[2] != metadata.block_size:
         raise ValueError(
             f"layer_kv_cache shape {tuple(layer_kv_cache.shape)} does not match block_size "
@@ -148,27 +160,41 @@ def hip_paged_attention(
 
     _check_inputs(query, key, value, layer_kv_cache, metadata)
     device = query.device
-    batch, keep = batch_descriptor(metadata, device)
+    *fields, keep = _batch_fields(metadata, device)
+    batch = _native.pack_batch(*fields)
     output = torch.empty_like(query)
-    lib = _native.load()
-    workspace_bytes = lib.mvllm_attention_workspace_bytes(batch, query.shape[1], query.shape[2])
+    _, num_heads, head_dim = query.shape
+    workspace_bytes = _native.packed("mvllm_attention_workspace_bytes")(batch, num_heads, head_dim)
     workspace = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=device)
-    args = (
-        _native.tensor3(query),
-        _native.tensor3(key),
-        _native.tensor3(value),
-        _native.kv_cache(layer_kv_cache),
-        batch,
-        _native.tensor3(output),
-        1.0 / math.sqrt(query.shape[-1]),
-        workspace.data_ptr(),
-        workspace.numel(),
-    )
+    scale = 1.0 / math.sqrt(head_dim)
     stream = _native.stream_handle(device)
     if timing is None:
-        status = lib.mvllm_attention_forward(*args, stream)
+        status = _native.packed("mvllm_attention_forward")(
+            _native.pack_tensor3(query),
+            _native.pack_tensor3(key),
+            _native.pack_tensor3(value),
+            _native.pack_kv_cache(layer_kv_cache),
+            batch,
+            _native.pack_tensor3(output),
+            scale,
+            workspace.data_ptr(),
+            max(workspace_bytes, 1),
+            stream,
+        )
     else:
-        status = lib.mvllm_attention_forward_timed(*args, timing, stream)
+        status = _native.load().mvllm_attention_forward_timed(
+            _native.tensor3(query),
+            _native.tensor3(key),
+            _native.tensor3(value),
+            _native.kv_cache(layer_kv_cache),
+            _native.Batch.from_buffer_copy(batch),
+            _native.tensor3(output),
+            scale,
+            workspace.data_ptr(),
+            workspace.numel(),
+            timing,
+            stream,
+        )
     _native.check(status, "mvllm_attention_forward")
     del keep
     return output

@@ -93,10 +93,10 @@ def qk_norm_rope_kv_write(
         raise ValueError("slot_mapping must be int64 with one entry per token")
     q_out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     _native.check(
-        _native.load().mvllm_qk_norm_rope_kv_write(
-            _native.tensor3(query),
-            _native.tensor3(key),
-            _native.tensor3(value),
+        _native.packed("mvllm_qk_norm_rope_kv_write")(
+            _native.pack_tensor3(query),
+            _native.pack_tensor3(key),
+            _native.pack_tensor3(value),
             q_weight.contiguous().data_ptr() if q_weight is not None else None,
             k_weight.contiguous().data_ptr() if k_weight is not None else None,
             cos.data_ptr() if cos is not None else None,
@@ -105,7 +105,7 @@ def qk_norm_rope_kv_write(
             rows if positions is not None else 0,
             eps,
             q_out.data_ptr(),
-            _native.kv_cache(layer_kv_cache),
+            _native.pack_kv_cache(layer_kv_cache),
             slot_mapping.contiguous().data_ptr(),
             _native.stream_handle(query.device),
         ),
