@@ -102,6 +102,13 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 //   256), or, beside prefill work, whose workgroups fill the chip as well,
 //   half an item per CU of up to 2,048 (248 decodes and 8 chunks of 512: 736
 //   us with 2,048, 781 with 512);
+// * no splits at all where the requests alone fill the chip (workgroups for
+//   three quarters of the CUs), are about even or short, and the longest one's
+//   tiles take no longer than the whole batch takes at the HBM's rate (0.04 us
+//   per token against ~6.2 TB/s): the partials and their merge are then pure
+//   cost. 201 decodes that see 484 keys each: 70 us whole, 77-81 in two or
+//   three splits; 256 of 505: 85.5 and 93; 128 of 20 .. 300: 23.0 and 26.1
+//   (uneven ones of up to 965 keys are better off split: 83.0 whole, 80.6);
 // * at most 32 splits per request up to 512 tokens each: the merge loads 32
 //   at a time (one context of 32k: 143 us with 64-token splits, 47 with 512).
 // At least total / (capacity - R), so that the items fit the list: a request
@@ -131,12 +138,18 @@ inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int
 }
 
 __device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t requests, int64_t capacity,
-                                       int32_t cus, int32_t head_dim, int32_t num_kv_heads, bool beside_prefill) {
+                                       int32_t cus, int32_t head_dim, int32_t num_kv_heads, int32_t decodes,
+                                       bool beside_prefill) {
   // Quotients in float (a 64-bit division takes longer than the rest of the
   // rule), raised by more than their error; lengths past 2^20 mean the same.
   auto up16 = [](float v) { return (static_cast<int32_t>(fminf(v * 1.000001f, 1048576.f)) + 16) & ~15; };
   const float tokens = static_cast<float>(total);
   const float wide = tokens * head_dim / 128.f;
+  const int32_t groups = (num_kv_heads + 3) / 4;
+  if (!beside_prefill && longest <= kMostSplit && 4.f * decodes * groups >= 3.f * cus &&
+      (longest <= 320 || tokens >= 0.75f * longest * decodes) &&
+      0.04f * longest <= tokens * num_kv_heads * head_dim / 1.55e6f)
+    return (longest + 15) & ~15;
   const int32_t most = beside_prefill ? kMaxSplit : kMostSplit;
   int32_t split = up16(wide / (beside_prefill ? 0.5f * cus : 2.f * cus));
   int32_t least = up16(wide / kSmallItems);
@@ -151,14 +164,14 @@ __device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t r
 }
 
 __device__ inline void build_decode_list(const AttnArgs& a) {
-  __shared__ int32_t full_count, full_pos, base_pos, longest, others;
+  __shared__ int32_t full_count, full_pos, base_pos, longest, others, decodes;
   __shared__ unsigned long long pages;
   __shared__ int32_t bucket[kSizeBuckets];
   const int tid = threadIdx.x;
   const int64_t R = a.num_requests;
   const int64_t capacity = a.item_capacity;
   if (tid == 0) {
-    full_count = full_pos = base_pos = longest = others = 0;
+    full_count = full_pos = base_pos = longest = others = decodes = 0;
     pages = 0;
   }
   if (tid < kSizeBuckets) bucket[tid] = 0;
@@ -214,15 +227,17 @@ __device__ inline void build_decode_list(const AttnArgs& a) {
       const int32_t high = wave_reduce_i(count >> 16, add);
       const int32_t most = wave_reduce_i(d.tokens, larger);
       const bool other = __ballot(r0 + lane < R && !d.dec) != 0;
+      const int32_t seen = static_cast<int32_t>(__popcll(__ballot(d.tokens > 0)));
       if (lane == 0) {
         atomicAdd(&pages, (static_cast<unsigned long long>(high) << 16) + low);
         atomicMax(&longest, most);
         if (other) others = 1;
+        atomicAdd(&decodes, seen);
       }
     }
     __syncthreads();
     split = choose_split(16 * static_cast<int64_t>(pages), longest, R, capacity, a.num_cus, a.head_dim,
-                         a.num_kv_heads, others && !a.decode_only);
+                         a.num_kv_heads, decodes, others && !a.decode_only);
   }
   // 64 buckets of 2^bucket_shift sizes span every split length: the smallest
   // shift with 64 << shift >= split (a partial split holds 1 .. split - 1

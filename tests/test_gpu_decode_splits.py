@@ -29,6 +29,8 @@ BATCHES = {
     "around-the-shortest-split": [191, 192, 193, 207, 208, 209, 383, 384, 385],
     "merge-rounds": [300, 700, 1500, 3000, 4500, 6100, 12_000],
     "single": [6145],
+    "whole-even": [1000 + r % 20 for r in range(110)],
+    "whole-short": [1 + (r * 7) % 320 for r in range(200)],
 }
 
 
