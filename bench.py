@@ -1,8 +1,8 @@
 """Benchmark of the ragged paged-attention path on one MI355X.
 
 A step is one pass of the hot path over one synthetic batch: the
-``mi355x_paged`` operator's forward (KV-cache write + split-KV decode +
-combine; + MFMA prefill for multi-query requests). The default workload is
+``mi355x_paged`` operator's forward (KV-cache write + split-KV decode with
+its merge; + MFMA prefill for multi-query requests). The default workload is
 the Qwen3-0.6B-head decode batch: 256 sequences, contexts U[128, 4096]
 (seed 0), 16 query / 8 KV heads, head_dim 128, block 16, bf16, blocks drawn
 from a shuffled 70,000-block pool, values N(0,1)*0.5.

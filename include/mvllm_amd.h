@@ -122,8 +122,8 @@ int mvllm_kv_write(const mvllm_tensor3* key, const mvllm_tensor3* value,
 /*
  * Bytes of device workspace mvllm_paged_attention / mvllm_attention_forward
  * need for this batch geometry: the split-KV partial results of the decode
- * kernel and the decode and prefill work lists, which the library writes
- * before it reads them (the caller need not initialise the workspace).
+ * kernel, the decode and prefill work lists and the counters of finished
+ * splits, which the library writes before it reads them (the caller need not initialise the workspace).
  * Decode positions must stay below 2^31 (block-table width * block size).
  * Depends only on
  * shapes, never on device data, so it can be sized before graph capture.
@@ -193,8 +193,9 @@ int mvllm_attention_forward(const mvllm_tensor3* query,
                             int64_t workspace_bytes, void* stream);
 
 /*
- * Device workspace held by mvllm_attention_forward_noalloc: 32 MiB per device.
- * It covers the split-KV partials and work lists of batches such as 256
+ * Device workspace held by mvllm_attention_forward_noalloc: 32 MiB per device
+ * (and 1/64 of that for the decode kernel's counters of finished splits, which
+ * do not count against it). It covers the split-KV partials and work lists of batches such as 256
  * decodes over a 512-block table with 32 query heads (about 21 MB).
  */
 #define MVLLM_NOALLOC_SCRATCH_BYTES (32LL * 1024 * 1024)
