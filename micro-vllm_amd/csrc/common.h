@@ -173,26 +173,27 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // Direct HBM -> LDS load of 16 bytes per lane (global_load_lds_dwordx4):
 // lane l's 16 bytes land at LDS byte address lds_base + 16 * l (lds_base is
-// wave-uniform). Issued through inline assembly so that the compiler does not
+// wave-uniform); the source is a wave-uniform 64-bit base in SGPRs plus a
+// per-lane 32-bit byte offset, which saves the 64-bit vector address
+// arithmetic. Issued through inline assembly so that the compiler does not
 // track the LDS write; callers order it with explicit s_waitcnt vmcnt counts.
 // The assembly sets M0, which the compiler treats as reserved (it warns about
 // the clobber): the kernels that use these loads contain no compiler-generated
 // M0 use, which their assembly shows.
-__device__ __forceinline__ void lds_dma_load16(const void* global_ptr, uint32_t lds_base) {
+__device__ __forceinline__ void lds_dma_load16_sbase(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile(
       "s_mov_b32 m0, %1\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
+      "global_load_lds_dwordx4 %0, %2"
       :
-      : "v"(global_ptr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
+      : "v"(offset), "s"(__builtin_amdgcn_readfirstlane(lds_base)), "s"(base)
       : "memory", "m0");
 }
 
-// lds_dma_load16 for data read exactly once (the decode kernel's K/V
-// stream), from a wave-uniform 64-bit base in SGPRs and a per-lane 32-bit byte
-// offset, to a wave-uniform LDS base plus an immediate added straight into M0
-// (s_add_u32 also writes SCC). The non-temporal hint lets the lines leave the
-// caches first instead of displacing data that is reused.
+// The same for data read exactly once (the decode kernel's K/V stream), to a
+// wave-uniform LDS base plus an immediate added straight into M0 (s_add_u32
+// also writes SCC). The non-temporal hint lets the lines leave the caches
+// first instead of displacing data that is reused.
 template <int OFF>
 __device__ __forceinline__ void lds_dma_load16_stream(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile(
@@ -204,18 +205,6 @@ __device__ __forceinline__ void lds_dma_load16_stream(const void* base, uint32_t
       : "memory", "m0", "scc");
 }
 
-// lds_dma_load16 with a wave-uniform 64-bit base in SGPRs and a per-lane
-// 32-bit byte offset, which saves the 64-bit vector address arithmetic.
-__device__ __forceinline__ void lds_dma_load16_sbase(const void* base, uint32_t offset, uint32_t lds_base) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %2"
-      :
-      : "v"(offset), "s"(__builtin_amdgcn_readfirstlane(lds_base)), "s"(base)
-      : "memory", "m0");
-}
-
 // s_waitcnt with vmcnt <= N (N < 64), other counters unconstrained (gfx9 encoding).
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -223,7 +212,7 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-// Byte address of an LDS location, for lds_dma_load16.
+// Byte address of an LDS location, for the loads above.
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return static_cast<uint32_t>(
       reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
@@ -269,18 +258,5 @@ template <> struct Mfma<f16_t> {
         0, 0);
   }
 };
-
-// Byte permute (v_perm_b32): result byte i = byte sel_i of {hi:lo}.
-__device__ __forceinline__ uint32_t perm_b32(uint32_t hi, uint32_t lo, uint32_t sel) {
-  return __builtin_amdgcn_perm(hi, lo, sel);
-}
-// Low 16 bits of a and b -> (a.lo | b.lo << 16).
-__device__ __forceinline__ uint32_t pack_lo16(uint32_t a, uint32_t b) {
-  return perm_b32(b, a, 0x05040100u);
-}
-// High 16 bits of a and b -> (a.hi | b.hi << 16).
-__device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) {
-  return perm_b32(b, a, 0x07060302u);
-}
 
 }  // namespace mvllm
