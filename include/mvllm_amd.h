@@ -155,7 +155,9 @@ int mvllm_paged_attention(const mvllm_tensor3* query,
  * cache's head_dim. No counterpart in the reference, whose operator runs per
  * layer (qwen.py:89-99): its callers are models whose layers share one batch
  * and one cache geometry, which then plan once per step instead of once per
- * layer (the lists depend only on the batch). Graph-capturable.
+ * layer. The lists depend on the batch, num_q_heads and the cache's geometry
+ * (element type, KV heads, head_dim, strides, alignment), not on its contents.
+ * Graph-capturable.
  */
 int mvllm_attention_plan(const mvllm_batch* batch, int64_t num_q_heads,
                          const mvllm_kv_cache* cache, void* workspace,
@@ -165,10 +167,13 @@ int mvllm_attention_plan(const mvllm_batch* batch, int64_t num_q_heads,
  * mvllm_paged_attention over the work lists that mvllm_attention_plan wrote
  * into the same workspace. The caller guarantees that the plan was made for
  * this batch, head count and cache geometry, and that nothing overwrote the
- * workspace since (calls in one stream may share it: each rewrites only the
- * split-KV partials). This is not checked; a mismatched plan gives wrong
- * results but every record field is range-checked before it is used as an
- * index.
+ * workspace since. Calls in one stream may share it: each rewrites the
+ * split-KV partials and counts its finished splits in it, and leaves the
+ * counters at zero for the next. So two calls that share a workspace must not
+ * overlap. None of this is checked: a mismatched plan, or an overlap, gives
+ * wrong results, and may leave a counter off, which spoils every later call on
+ * that workspace until mvllm_attention_plan has written it again. Every record
+ * field is range-checked before it is used as an index.
  */
 int mvllm_paged_attention_planned(const mvllm_tensor3* query,
                                   const mvllm_kv_cache* cache,

@@ -200,15 +200,33 @@ def hip_paged_attention(
     return output
 
 
+def plan_geometry(layer_kv_cache: torch.Tensor) -> tuple:
+    """What a plan takes from the cache: the element type, block size, KV heads,
+    head_dim, strides within a block and alignment decide which kernels run and
+    how the decode splits, their counters and the query blocks are laid out.
+    The block count and the memory itself do not matter."""
+
+    return (
+        layer_kv_cache.dtype,
+        *layer_kv_cache.shape[2:],
+        *layer_kv_cache.stride()[1:],
+        layer_kv_cache.stride(0) * layer_kv_cache.element_size() % 16,
+        layer_kv_cache.data_ptr() % 16,
+    )
+
+
 class AttentionPlan:
     """Work lists of one batch, built once and shared by every layer of a step.
 
     The reference's operator runs per layer (qwen.py:89-99); the lists depend
-    only on the batch, so a model whose layers share one metadata bundle and
-    one cache geometry plans once per step (``mvllm_attention_plan``) and
-    each layer's ``hip_attention_over_cache(..., plan=plan)`` skips the
-    list kernels. The plan owns the workspace, which every planned call on
-    the same stream reuses for its split-KV partials.
+    only on the batch, the query heads and the cache's geometry, so a model
+    whose layers share one metadata bundle and one geometry plans once per step
+    (``mvllm_attention_plan``) and each layer's
+    ``hip_attention_over_cache(..., plan=plan)`` skips the list kernels. A
+    layer whose cache differs (``plan_geometry``) is answered through lists of
+    its own. The plan owns the workspace, which every planned call reuses for
+    its split-KV partials and the counters of its finished splits: planned
+    calls of one plan run in one stream and never overlap.
     """
 
     def __init__(self, metadata: AttentionMetadata, num_q_heads: int, layer_kv_cache: torch.Tensor):
@@ -217,6 +235,7 @@ class AttentionPlan:
             raise RuntimeError("mi355x_paged attention plans require a GPU cache")
         self.metadata = metadata
         self.num_q_heads = num_q_heads
+        self.geometry = plan_geometry(layer_kv_cache)
         self.batch, self._keep = batch_descriptor(metadata, device)
         lib = _native.load()
         head_dim = layer_kv_cache.shape[-1]
@@ -244,7 +263,8 @@ def hip_attention_over_cache(
     """Ragged causal attention over a cache that already holds the step's
     K/V (written by ``layers.qk_norm_rope_kv_write``): the attention part of
     ``hip_paged_attention``, without the cache write. With ``plan`` (made for
-    this metadata and head count) the work lists are not rebuilt."""
+    this metadata and head count) the work lists are not rebuilt, unless the
+    cache's geometry is not the one that the plan was made for."""
 
     if query.device.type != "cuda" or layer_kv_cache.device != query.device:
         raise RuntimeError("mi355x_paged attention requires GPU tensors on one device")
@@ -256,6 +276,9 @@ def hip_attention_over_cache(
     if plan is not None:
         if plan.metadata is not metadata or plan.num_q_heads != query.shape[1]:
             raise ValueError("attention plan was made for other metadata or another head count")
+        if plan.geometry != plan_geometry(layer_kv_cache):
+            plan = None
+    if plan is not None:
         batch, keep, workspace, entry = plan.batch, None, plan.workspace, "mvllm_paged_attention_planned"
     else:
         batch, keep = batch_descriptor(metadata, device)
