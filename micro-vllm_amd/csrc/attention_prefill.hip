@@ -230,6 +230,70 @@ __device__ __forceinline__ void fill_tile_record(int32_t* tbl, const AttnArgs& a
   rec[1] = int4{e[2], static_cast<int32_t>(mask), e[3], static_cast<int32_t>(mask)};
 }
 
+// One output row, answered by one wave over the keys that the row sees and no
+// others, with fp32 scores and probabilities: a lane scores one key of 64, then
+// holds dims `lane` and `lane + 64`. For rows whose tiles gave something that is
+// not finite, so its time does not count.
+template <typename T, int D>
+__device__ __forceinline__ void answer_row(const AttnArgs& a, int64_t r, int64_t tok, int hq, int h, int32_t lo,
+                                           int32_t hi) {
+  constexpr int J = (D + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const uint16_t* const q = static_cast<const uint16_t*>(a.q) + tok * a.q_s0 + static_cast<int64_t>(hq) * a.q_s1;
+  const uint16_t* const cache = static_cast<const uint16_t*>(a.cache) + static_cast<int64_t>(h) * D;
+  float acc[J] = {};
+  float m = -INFINITY, l = 0.f;
+  for (int32_t base = lo; base <= hi; base += 64) {
+    const int32_t count = hi - base < 63 ? hi - base + 1 : 64;
+    int64_t row = -1;  // element offset of this lane's key row
+    if (lane < count) {
+      const int64_t b = block_of(a, r, base + lane);
+      if (b >= 0) row = b * a.c_s[1] + ((base + lane) % a.block_size) * a.c_s[2];
+    }
+    float s = -INFINITY;
+    if (row >= 0) {
+      float sum[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int d = 0; d < D; d += 4) {
+        const uint2 kw = *reinterpret_cast<const uint2*>(cache + row + d);
+        const uint2 qw = *reinterpret_cast<const uint2*>(q + d);
+        const uint32_t k[4] = {kw.x & 0xFFFFu, kw.x >> 16, kw.y & 0xFFFFu, kw.y >> 16};
+        const uint32_t x[4] = {qw.x & 0xFFFFu, qw.x >> 16, qw.y & 0xFFFFu, qw.y >> 16};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sum[e] = __builtin_fmaf(Elem<T>::from_bits(x[e]) * a.scale_log2, Elem<T>::from_bits(k[e]), sum[e]);
+      }
+      s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    }
+    float most = s;
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) most = fmaxf(most, __shfl_xor(most, x, 64));
+    const float mn = fmaxf(m, most);
+    const float alpha = mn == -INFINITY ? 1.f : exp2f(m - mn);
+    const float p = s == -INFINITY ? 0.f : exp2f(s - mn);
+    float sum = p;
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) sum += __shfl_xor(sum, x, 64);
+    l = l * alpha + sum;
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[j] *= alpha;
+    for (int k = 0; k < count; ++k) {
+      const int64_t vrow = __shfl(row, k, 64);
+      const float pk = __shfl(p, k, 64);
+      if (vrow < 0) continue;
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (lane + 64 * j < D)
+          acc[j] = __builtin_fmaf(pk, Elem<T>::from_bits(cache[a.c_s[0] + vrow + lane + 64 * j]), acc[j]);
+    }
+    m = mn;
+  }
+  uint16_t* const out = static_cast<uint16_t*>(a.out) + tok * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (lane + 64 * j < D) out[lane + 64 * j] = static_cast<uint16_t>(Elem<T>::to_bits(acc[j] * inv));
+}
+
 // At head_dim 64 and 96 Q is not rescaled (the scale multiplies the fp32
 // scores) and P enters the P.V product as a hi/lo pair of 16-bit values that
 // keeps ~16 bits of its mantissa, the row sum being taken over the fp32
@@ -729,6 +793,22 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   // v_permlane32_swap per word gives lane hh the whole group q = 2 p + hh,
   // so every lane writes 16-byte pieces.
   const float inv = nonempty ? 1.f / lt : NAN;  // an empty visible range is NaN, as in the reference
+  // At head_dim 64 and 96 a value of V that is not finite reaches only the rows
+  // that see its key (and an infinity stays one), as in the any-shape kernel.
+  // In the tiles it reaches every row of the workgroup, as 0 * inf and inf * lo;
+  // it never leaves an accumulator again, so it is looked for once, here: such
+  // rows are answered one by one below.
+  uint32_t redo = 0;  // bit n: row n of this wave
+  if constexpr (kSplitP) {
+    float zero = 0.f;
+#pragma unroll
+    for (int c = 0; c < kBlocks; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) zero = __builtin_fmaf(oacc[c][i], 0.f, zero);
+    const uint64_t bad = __ballot(zero != zero && row_ok && nonempty);
+    redo = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
+  }
+  const bool store_row = row_ok && !((redo >> n) & 1u);
   uint16_t* op = static_cast<uint16_t*>(a.out) + tok * a.o_s0 + static_cast<int64_t>(hq) * a.o_s1;
 #pragma unroll
   for (int c = 0; c < kBlocks; ++c)
@@ -751,8 +831,16 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         got[k] = hh ? r2[0] : r2[1];
       }
       const uint4 piece = hh ? uint4{got[0], got[1], w[1][0], w[1][1]} : uint4{w[0][0], w[0][1], got[0], got[1]};
-      if (row_ok) *reinterpret_cast<uint4*>(op + 32 * c + 8 * (2 * p + hh)) = piece;
+      if (store_row) *reinterpret_cast<uint4*>(op + 32 * c + 8 * (2 * p + hh)) = piece;
     }
+  if constexpr (kSplitP) {
+    for (; redo; redo &= redo - 1) {
+      const int x = __builtin_ctz(redo);
+      const int fx = wave * 32 + x;
+      answer_row<T, D>(a, r, t0 + (fx & (tpb - 1)), h * G + (fx >> lg_tok), h, __builtin_amdgcn_readlane(lo_n, x),
+                       __builtin_amdgcn_readlane(hi_n, x));
+    }
+  }
 }
 
 template <typename T, int D>

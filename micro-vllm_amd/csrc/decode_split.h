@@ -15,6 +15,7 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "worklists.h"
 
@@ -448,95 +449,128 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   };
 
   float4_t acc[D / 16];
+  float m, l;
+  // One walk over the split's tiles; EXACT: with P in fp32
+  // (v_mfma_f32_16x16x4_f32; as the only walk it took 31.1 us instead of 24.6 for
+  // 8 decodes of 4,000 keys at head_dim 96 and 2 KV heads).
+  auto walk = [&](auto exact_c) {
+    constexpr bool EXACT = decltype(exact_c)::value;
 #pragma unroll
-  for (int b = 0; b < D / 16; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
+    for (int b = 0; b < D / 16; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s)
+      if (s < ntiles) issue(s, s);
 
+    for (int k = 0; k < ntiles; ++k) {
+      const int stage = k % STAGES;
+      const int later = (ntiles - 1 - k) < (STAGES - 1) ? (ntiles - 1 - k) : (STAGES - 1);
+      wait_tiles<2 * kLoads>(later);
+      __builtin_amdgcn_wave_barrier();
+      compiler_fence();
+
+      // The whole tile goes to registers first, so that its stage refills while
+      // it is computed (STAGES tiles in flight throughout) and the V reads do
+      // not wait behind the softmax.
+      const uint32_t kt = wave_lds_addr + stage * 2 * kTileBytes;
+      const uint32_t vt = kt + kTileBytes;
+      short8_t kf[kLoads];
+      uint2 vf[D / 16];
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        kf[i] = *reinterpret_cast<lds_short8*>(static_cast<uintptr_t>(kt + koff[i]));
+#pragma unroll
+      for (int b = 0; b < D / 16; ++b) {
+        // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
+        vf[b] = __builtin_bit_cast(
+            uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(vt + voff[b]))));
+      }
+      // All LDS reads of this stage retire before the refill is issued.
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      compiler_fence();
+      __builtin_amdgcn_sched_barrier(0);
+      if (k + STAGES < ntiles) issue(k + STAGES, stage);
+
+      const int32_t tb = static_cast<int32_t>(begin) + 16 * k;
+      // Token j of the tile is visible iff its position is in [lo, end] and the block is valid.
+      uint32_t okmask = 0;
+      if (tile_block(k) >= 0) {
+        const int32_t first_ok = lo > tb ? static_cast<int32_t>(lo) - tb : 0;
+        const int32_t last_ok = end - tb < 15 ? static_cast<int32_t>(end) - tb : 15;
+        okmask = (last_ok >= first_ok) ? ((0xFFFFu >> (15 - last_ok)) & (0xFFFFu << first_ok)) : 0u;
+      }
+
+      float4_t sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) sc = Mfma<T>::k32(kf[i], qv[i], sc);
+      float s[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s[e] = ((okmask >> (4 * grp + e)) & 1u) ? sc[e] * a.scale_log2 : -INFINITY;
+      float bm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+      bm = max_xor32_f(max_xor16_f(bm));
+      const float mn = fmaxf(m, bm);
+      // v_exp_f32 flushes results below 2^-126 to zero: nothing beside the
+      // row's maximum of 1.
+      const float alpha = (mn == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+      float p[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[e] = (s[e] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s[e] - mn);
+      l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+      if (__ballot(alpha != 1.f)) {
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) acc[b] *= alpha;
+      }
+      m = mn;
+
+      if (okmask != 0xFFFFu) {
+        // Rows of masked tokens may hold stale or non-finite data: zero them in V.
+        const uint32_t ok4 = okmask >> (4 * grp);
+        const uint32_t mlo = (ok4 & 1u ? 0xFFFFu : 0u) | (ok4 & 2u ? 0xFFFF0000u : 0u);
+        const uint32_t mhi = (ok4 & 4u ? 0xFFFFu : 0u) | (ok4 & 8u ? 0xFFFF0000u : 0u);
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) vf[b] = uint2{vf[b].x & mlo, vf[b].y & mhi};
+      }
+      if constexpr (!EXACT) {
+        uint32_t ph[4], pl[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split_hi_lo<T>(p[e], ph[e], pl[e]);
+        const short4_t pb_hi = __builtin_bit_cast(short4_t, uint2{ph[0] | (ph[1] << 16), ph[2] | (ph[3] << 16)});
+        const short4_t pb_lo = __builtin_bit_cast(short4_t, uint2{pl[0] | (pl[1] << 16), pl[2] | (pl[3] << 16)});
+        // Both products of a block depend on each other, the blocks do not.
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_hi, acc[b]);
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_lo, acc[b]);
+      } else {
+        // Step x: k index grp stands for token 4grp + x, whose probability and V
+        // row the lane holds already.
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int b = 0; b < D / 16; ++b) {
+            const uint32_t w = x < 2 ? vf[b].x : vf[b].y;
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<T>::from_bits(x & 1 ? w >> 16 : w & 0xFFFFu), p[x], acc[b],
+                                                          0, 0, 0);
+          }
+      }
+    }
+  };
   // The block ids and Q must be in registers before the first tile address.
   __builtin_amdgcn_s_waitcnt(0);
+  walk(std::false_type{});
+  // At head_dim 64 and 96 an infinity in V stays one, as in the any-shape kernel:
+  // times a low half that is zero or negative it is NaN, which no later tile
+  // takes out of the accumulators again. Such a wave answers its split with P in
+  // fp32.
+  if constexpr (D != 128) {
+    float zero = 0.f;
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s)
-    if (s < ntiles) issue(s, s);
-
-  for (int k = 0; k < ntiles; ++k) {
-    const int stage = k % STAGES;
-    const int later = (ntiles - 1 - k) < (STAGES - 1) ? (ntiles - 1 - k) : (STAGES - 1);
-    wait_tiles<2 * kLoads>(later);
-    __builtin_amdgcn_wave_barrier();
-    compiler_fence();
-
-    // The whole tile goes to registers first, so that its stage refills while
-    // it is computed (STAGES tiles in flight throughout) and the V reads do
-    // not wait behind the softmax.
-    const uint32_t kt = wave_lds_addr + stage * 2 * kTileBytes;
-    const uint32_t vt = kt + kTileBytes;
-    short8_t kf[kLoads];
-    uint2 vf[D / 16];
+    for (int b = 0; b < D / 16; ++b)
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-      kf[i] = *reinterpret_cast<lds_short8*>(static_cast<uintptr_t>(kt + koff[i]));
-#pragma unroll
-    for (int b = 0; b < D / 16; ++b) {
-      // A operand: lane (col, grp) receives V[token 4grp + e][dim 16b + col].
-      vf[b] = __builtin_bit_cast(
-          uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr_short4*>(static_cast<uintptr_t>(vt + voff[b]))));
-    }
-    // All LDS reads of this stage retire before the refill is issued.
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    compiler_fence();
-    __builtin_amdgcn_sched_barrier(0);
-    if (k + STAGES < ntiles) issue(k + STAGES, stage);
-
-    const int32_t tb = static_cast<int32_t>(begin) + 16 * k;
-    // Token j of the tile is visible iff its position is in [lo, end] and the block is valid.
-    uint32_t okmask = 0;
-    if (tile_block(k) >= 0) {
-      const int32_t first_ok = lo > tb ? static_cast<int32_t>(lo) - tb : 0;
-      const int32_t last_ok = end - tb < 15 ? static_cast<int32_t>(end) - tb : 15;
-      okmask = (last_ok >= first_ok) ? ((0xFFFFu >> (15 - last_ok)) & (0xFFFFu << first_ok)) : 0u;
-    }
-
-    float4_t sc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) sc = Mfma<T>::k32(kf[i], qv[i], sc);
-    float s[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      s[e] = ((okmask >> (4 * grp + e)) & 1u) ? sc[e] * a.scale_log2 : -INFINITY;
-    float bm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    bm = max_xor32_f(max_xor16_f(bm));
-    const float mn = fmaxf(m, bm);
-    // v_exp_f32 flushes results below 2^-126 to zero: nothing beside the
-    // row's maximum of 1.
-    const float alpha = (mn == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m - mn);
-    float p[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = (s[e] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s[e] - mn);
-    l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-    if (__ballot(alpha != 1.f)) {
-#pragma unroll
-      for (int b = 0; b < D / 16; ++b) acc[b] *= alpha;
-    }
-    m = mn;
-
-    uint32_t ph[4], pl[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) split_hi_lo<T>(p[e], ph[e], pl[e]);
-    const short4_t pb_hi = __builtin_bit_cast(short4_t, uint2{ph[0] | (ph[1] << 16), ph[2] | (ph[3] << 16)});
-    const short4_t pb_lo = __builtin_bit_cast(short4_t, uint2{pl[0] | (pl[1] << 16), pl[2] | (pl[3] << 16)});
-    if (okmask != 0xFFFFu) {
-      // Rows of masked tokens may hold stale or non-finite data: zero them in V.
-      const uint32_t ok4 = okmask >> (4 * grp);
-      const uint32_t mlo = (ok4 & 1u ? 0xFFFFu : 0u) | (ok4 & 2u ? 0xFFFF0000u : 0u);
-      const uint32_t mhi = (ok4 & 4u ? 0xFFFFu : 0u) | (ok4 & 8u ? 0xFFFF0000u : 0u);
-#pragma unroll
-      for (int b = 0; b < D / 16; ++b) vf[b] = uint2{vf[b].x & mlo, vf[b].y & mhi};
-    }
-    // Both products of a block depend on each other, the blocks do not.
-#pragma unroll
-    for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_hi, acc[b]);
-#pragma unroll
-    for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_lo, acc[b]);
+      for (int e = 0; e < 4; ++e) zero = __builtin_fmaf(acc[b][e], 0.f, zero);
+    if (__ballot(zero != zero)) walk(std::true_type{});
   }
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
