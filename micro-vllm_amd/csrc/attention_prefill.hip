@@ -90,6 +90,16 @@ template <> struct Mma32<bf16_t> {
   __device__ static float2v unpack2(uint32_t w) {
     return float2v{__uint_as_float(w << 16), __uint_as_float(w & 0xFFFF0000u)};
   }
+  // x and y less the low and the high bf16 value of w (w.lo * -1 + w.hi * 0 + x):
+  // one instruction each, where widening the value first takes two. The factors
+  // (-1, 0) and (0, -1) are opaque: the compiler would give the first one as the
+  // inline constant -1.0, which the instruction reads as the second.
+  __device__ static float2v less(float x, float y, uint32_t w) {
+    uint32_t lo = 0x0000BF80u, hi = 0xBF800000u;
+    asm("" : "+s"(lo), "+s"(hi));
+    return float2v{__builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, lo), x, false),
+                   __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, hi), y, false)};
+  }
   // acc + the two bf16 values of w.
   __device__ static float dot2_ones(uint32_t w, float acc) {
     const bf16x2_t one = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
@@ -107,6 +117,10 @@ template <> struct Mma32<f16_t> {
   }
   __device__ static float2v unpack2(uint32_t w) {
     return __builtin_convertvector(__builtin_bit_cast(f16x2_t, w), float2v);
+  }
+  __device__ static float2v less(float x, float y, uint32_t w) {
+    const float2v r = unpack2(w);
+    return float2v{x - r[0], y - r[1]};
   }
   // acc + the two fp16 values of w.
   __device__ static float dot2_ones(uint32_t w, float acc) {
@@ -295,11 +309,16 @@ __device__ __forceinline__ void answer_row(const AttnArgs& a, int64_t r, int64_t
 }
 
 // At head_dim 64 and 96 Q is not rescaled (the scale multiplies the fp32
-// scores) and P enters the P.V product as a hi/lo pair of 16-bit values that
-// keeps ~16 bits of its mantissa, the row sum being taken over the fp32
-// probabilities, as in the decode kernel: these rows' requests have always
-// been answered with fp32 probabilities. The narrower accumulators leave the
-// registers for it.
+// scores) and the row sum is taken over the fp32 probabilities, which enter the
+// P.V product in kParts 16-bit parts: these rows' requests have always been
+// answered with fp32 probabilities. Three parts of bf16 hold all 24 bits. Two of
+// fp16 hold 22: the second is scaled by 2^11, out of the subnormals, and summed
+// apart (kSumLow), and both are lifted by 2^7 (exponents that fp16's range leaves
+// over above the lazy offset's 2^8), so that a probability keeps its 22 bits down
+// to 2^-21 of the row's maximum. The narrower accumulators leave the registers
+// for it. Against a pair without lift: 2 chunks of 1,024 at 8,192 keys, 16/8 heads
+// of 64, 187 -> 247 us in bf16 (a third more P.V products), 190 -> 218 in fp16; 30
+// decodes and chunks of 200 and 256, 34.5 -> 36.7 and 34.8 -> 36.0.
 template <typename T, int D>
 __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, uint8_t* smem, uint32_t wg) {
   constexpr int kTileBytes = kKeyTileBytes<D>;
@@ -307,6 +326,11 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   constexpr int kSteps = D / 16;              // 16-dim MFMA steps of a score
   constexpr int kBlocks = D / 32;             // 32-dim blocks of O^T; also the 1 KiB loads of a page
   constexpr bool kSplitP = D != 128;
+  constexpr int kParts = !kSplitP ? 1 : std::is_same_v<T, bf16_t> ? 3 : 2;
+  constexpr bool kSumLow = kParts == 2;
+  constexpr float kLowScale = 2048.f;
+  constexpr float kLift = kSumLow ? 7.f : 0.f;  // a row's first maximum becomes 2^kLift
+  constexpr float kMostSum = kSumLow ? 32768.f : 4096.f;
   uint8_t* const vbuf = smem + 2 * kTileBytes;  // V stages 0, 1 (K stages 0, 1 lie before them)
   int32_t* const page_tbl = reinterpret_cast<int32_t*>(smem + 4 * kTileBytes);
   int32_t* const red = page_tbl + kTableInts;
@@ -422,6 +446,11 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
   float16v oacc[kBlocks];
 #pragma unroll
   for (int c = 0; c < kBlocks; ++c) oacc[c] = float16v{};
+  float16v olow[kBlocks];  // kSumLow: the product with the second parts, times kLowScale
+  if constexpr (kSumLow) {
+#pragma unroll
+    for (int c = 0; c < kBlocks; ++c) olow[c] = float16v{};
+  }
   // Softmax state of this lane's row, in the exp2 domain. m_c is the
   // running offset (-inf until the row has seen a visible key); the S MFMAs
   // start from the accumulator value -c_in, so they produce scores already
@@ -620,9 +649,9 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
           s[i] = vis ? s[i] : -INFINITY;
         }
       };
-      // P^T of a half's two 16-key steps as MFMA B operands (lo: kSplitP only).
+      // P^T of a half's two 16-key steps as MFMA B operands, in kParts parts.
       struct PBits {
-        short8_t hi[2], lo[2];
+        short8_t part[kParts][2];
       };
       // O^T += V^T . P^T over a half's two 16-key steps.
       auto pv_mma = [&](const short4v (&vf)[2][kSteps], const PBits& pb) {
@@ -632,8 +661,13 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
           for (int c = 0; c < kBlocks; ++c) {
             const short4v lo4 = vf[q][c], hi4 = vf[q][kBlocks + c];
             const short8_t av = short8_t{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
-            oacc[c] = Mma32<T>::mma(av, pb.hi[q], oacc[c]);
-            if constexpr (kSplitP) oacc[c] = Mma32<T>::mma(av, pb.lo[q], oacc[c]);
+            if constexpr (kSumLow) {
+              oacc[c] = Mma32<T>::mma(av, pb.part[0][q], oacc[c]);
+              olow[c] = Mma32<T>::mma(av, pb.part[1][q], olow[c]);
+            } else {
+#pragma unroll
+              for (int y = 0; y < kParts; ++y) oacc[c] = Mma32<T>::mma(av, pb.part[y][q], oacc[c]);
+            }
           }
       };
       // Probabilities exp2(s + shift) (P^T B operands in pb), the add
@@ -651,21 +685,24 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           // P^T B operand: keys 16 s2 + 8 u + 4 hh + e  <->  k = 8 hh + 4 u + e.
-          uint32_t ph[4], pl[4];
+          uint32_t pw[kParts][4];
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
-            const float p0 = p[8 * s2 + 2 * w], p1 = p[8 * s2 + 2 * w + 1];
-            ph[w] = Mma32<T>::pack2(p0, p1);
-            if constexpr (kSplitP) {
-              const float2v r = Mma32<T>::unpack2(ph[w]);
-              pl[w] = Mma32<T>::pack2(p0 - r[0], p1 - r[1]);
-              inc += p0 + p1;
-            } else {
-              inc = Mma32<T>::dot2_ones(ph[w], inc);
+            float p0 = p[8 * s2 + 2 * w], p1 = p[8 * s2 + 2 * w + 1];
+            if constexpr (kSplitP) inc += p0 + p1;
+#pragma unroll
+            for (int y = 0; y < kParts; ++y) {
+              pw[y][w] = Mma32<T>::pack2(p0, p1);
+              if (y + 1 == kParts) continue;
+              const float2v rest = Mma32<T>::less(p0, p1, pw[y][w]);
+              p0 = kSumLow ? rest[0] * kLowScale : rest[0];
+              p1 = kSumLow ? rest[1] * kLowScale : rest[1];
             }
+            if constexpr (!kSplitP) inc = Mma32<T>::dot2_ones(pw[0][w], inc);
           }
-          pb.hi[s2] = __builtin_bit_cast(short8_t, uint4{ph[0], ph[1], ph[2], ph[3]});
-          if constexpr (kSplitP) pb.lo[s2] = __builtin_bit_cast(short8_t, uint4{pl[0], pl[1], pl[2], pl[3]});
+#pragma unroll
+          for (int y = 0; y < kParts; ++y)
+            pb.part[y][s2] = __builtin_bit_cast(short8_t, uint4{pw[y][0], pw[y][1], pw[y][2], pw[y][3]});
         }
         return inc;
       };
@@ -678,13 +715,16 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
         mx = max_with_partner(mx);
         const float mx_c = mx + c_in;
-        const bool grow = mx_c > m_c + 8.f;
+        const bool grow = mx_c > m_c + (8.f + kLift);
         if (__ballot(grow)) {
-          const float m_new = grow ? mx_c : m_c;
+          const float m_new = grow ? mx_c - kLift : m_c;
           const float alpha = grow ? __builtin_amdgcn_exp2f(m_c - m_new) : 1.f;
           l *= alpha;
 #pragma unroll
-          for (int c = 0; c < kBlocks; ++c) oacc[c] *= alpha;
+          for (int c = 0; c < kBlocks; ++c) {
+            oacc[c] *= alpha;
+            if constexpr (kSumLow) olow[c] *= alpha;
+          }
           m_c = m_new;
         }
         const float m_eff = m_c == -INFINITY ? 0.f : m_c;
@@ -696,15 +736,15 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
       // A half's softmax with `work` (MFMAs of this wave that do not depend
       // on it) in the same block. A half first tries the current offset with
       // no row maximum (the scores already carry it): a lane's 16
-      // probabilities summing to at most 2^12 keep each below 2^12, which
-      // bf16 and fp16 P and the accumulators hold; otherwise (a maximum that
+      // probabilities summing to at most 2^12 (2^15 where they are lifted) keep
+      // each below that, which bf16 and fp16 P and the accumulators hold; otherwise (a maximum that
       // grew, an unset offset, NaN) the half is redone from its maximum.
       auto softmax_with = [&](float16v& s, PBits& pb, auto&& work) {
         work();
         // Speculative: the probabilities are formed in the same block as
         // `work`, and kept only when every lane has an offset.
         float inc = make_p(s, 0.f, std::false_type{}, pb);
-        const bool done = !__ballot(m_c == -INFINITY || !(inc <= 4096.f));
+        const bool done = !__ballot(m_c == -INFINITY || !(inc <= kMostSum));
         if (!done) inc = softmax_slow(s, pb);
         return inc;
       };
@@ -787,6 +827,10 @@ __device__ __forceinline__ void prefill_body(const AttnArgs& a, int32_t lg_tok, 
     if (tl < nt) step(tl, std::integral_constant<int, 0>{});
   }
 
+  if constexpr (kSumLow) {
+#pragma unroll
+    for (int c = 0; c < kBlocks; ++c) oacc[c] += olow[c] * (1.f / kLowScale);
+  }
   const float lt = sum_with_partner(l);
   // O^T block c, register 4 q + e of lane (n, hh): dim 32 c + 8 q + 4 hh + e.
   // Lanes n and n + 32 hold the two halves of each 8-dim group 8 q; one

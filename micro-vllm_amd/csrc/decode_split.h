@@ -11,7 +11,8 @@
 // of the KV head, padded to 16, K = head_dim: 64, 96 or 128); the softmax runs
 // on the accumulator layout, and P^T is the B operand of O^T += V^T . P^T
 // (v_mfma_f32_16x16x16), fed as a hi/lo pair so the product keeps ~16 mantissa
-// bits; the V^T operand comes from transposing LDS reads (ds_read_b64_tr_b16).
+// bits (more at head_dim 64 and 96: kSplitParts); the V^T operand comes from
+// transposing LDS reads (ds_read_b64_tr_b16).
 #pragma once
 
 #include <cmath>
@@ -269,6 +270,17 @@ __device__ inline void tidy_rows(const AttnArgs& a, int64_t wg) {
 // displacing other cached lines raised the measured bandwidth from 5.5 to
 // 6.0 TB/s on the Qwen3 decode batch.
 
+// P^T enters P.V in 16-bit parts. At head_dim 128: a hi/lo pair. At 64 and 96
+// requests have always been answered with fp32 probabilities, which three parts
+// of bf16 hold whole (256 decodes of 2,000 keys: 186 us, 185 with a pair); two of
+// fp16 hold 22 bits, down to 2^-29 of the maximum, with P lifted by 2^15 and the
+// second part by another 2^11 and summed apart, out of the subnormals.
+template <typename T, int D>
+constexpr int kSplitParts = D != 128 && std::is_same_v<T, bf16_t> ? 3 : 2;
+template <typename T, int D>
+constexpr bool kSumLow = D != 128 && !std::is_same_v<T, bf16_t>;
+constexpr float kLift = 32768.f, kLowScale = 2048.f;
+
 template <int D> constexpr int kTileBytesOf = 16 * 2 * D;  // one 16-token tile of one head, K or V
 
 // Tiles in flight per wave: 32 KiB of K and V per wave for the narrow heads
@@ -448,6 +460,8 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
     }
   };
 
+  constexpr int kParts = kSplitParts<T, D>;
+  constexpr bool kLow = kSumLow<T, D>;
   float4_t acc[D / 16];
   float m, l;
   // One walk over the split's tiles; EXACT: with P in fp32
@@ -455,8 +469,9 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
   // 8 decodes of 4,000 keys at head_dim 96 and 2 KV heads).
   auto walk = [&](auto exact_c) {
     constexpr bool EXACT = decltype(exact_c)::value;
+    float4_t low[D / 16];  // kLow: the product with the second parts
 #pragma unroll
-    for (int b = 0; b < D / 16; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < D / 16; ++b) acc[b] = low[b] = float4_t{0.f, 0.f, 0.f, 0.f};
     m = -INFINITY;
     l = 0.f;
 #pragma unroll
@@ -520,7 +535,10 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
       l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
       if (__ballot(alpha != 1.f)) {
 #pragma unroll
-        for (int b = 0; b < D / 16; ++b) acc[b] *= alpha;
+        for (int b = 0; b < D / 16; ++b) {
+          acc[b] *= alpha;
+          if constexpr (kLow && !EXACT) low[b] *= alpha;
+        }
       }
       m = mn;
 
@@ -533,16 +551,29 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
         for (int b = 0; b < D / 16; ++b) vf[b] = uint2{vf[b].x & mlo, vf[b].y & mhi};
       }
       if constexpr (!EXACT) {
-        uint32_t ph[4], pl[4];
+        short4_t part[kParts];
+        float rest[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) split_hi_lo<T>(p[e], ph[e], pl[e]);
-        const short4_t pb_hi = __builtin_bit_cast(short4_t, uint2{ph[0] | (ph[1] << 16), ph[2] | (ph[3] << 16)});
-        const short4_t pb_lo = __builtin_bit_cast(short4_t, uint2{pl[0] | (pl[1] << 16), pl[2] | (pl[3] << 16)});
-        // Both products of a block depend on each other, the blocks do not.
+        for (int e = 0; e < 4; ++e) rest[e] = kLow ? p[e] * kLift : p[e];
 #pragma unroll
-        for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_hi, acc[b]);
+        for (int y = 0; y < kParts; ++y) {
+          uint32_t w[4];
 #pragma unroll
-        for (int b = 0; b < D / 16; ++b) acc[b] = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), pb_lo, acc[b]);
+          for (int e = 0; e < 4; ++e) {
+            w[e] = Elem<T>::to_bits(rest[e]);
+            rest[e] -= Elem<T>::from_bits(w[e]);
+            if constexpr (kLow) rest[e] *= kLowScale;
+          }
+          part[y] = __builtin_bit_cast(short4_t, uint2{w[0] | (w[1] << 16), w[2] | (w[3] << 16)});
+        }
+        // The products of a block depend on each other, the blocks do not.
+#pragma unroll
+        for (int y = 0; y < kParts; ++y)
+#pragma unroll
+          for (int b = 0; b < D / 16; ++b) {
+            float4_t& to = kLow && y == 1 ? low[b] : acc[b];
+            to = Mfma<T>::k16(__builtin_bit_cast(short4_t, vf[b]), part[y], to);
+          }
       } else {
         // Step x: k index grp stands for token 4grp + x, whose probability and V
         // row the lane holds already.
@@ -556,12 +587,16 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
           }
       }
     }
+    if constexpr (kLow && !EXACT) {
+#pragma unroll
+      for (int b = 0; b < D / 16; ++b) acc[b] = (acc[b] + low[b] * (1.f / kLowScale)) * (1.f / kLift);
+    }
   };
   // The block ids and Q must be in registers before the first tile address.
   __builtin_amdgcn_s_waitcnt(0);
   walk(std::false_type{});
   // At head_dim 64 and 96 an infinity in V stays one, as in the any-shape kernel:
-  // times a low half that is zero or negative it is NaN, which no later tile
+  // times a part of P that is zero or negative it is NaN, which no later tile
   // takes out of the accumulators again. Such a wave answers its split with P in
   // fp32.
   if constexpr (D != 128) {
