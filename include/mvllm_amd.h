@@ -170,10 +170,11 @@ int mvllm_attention_plan(const mvllm_batch* batch, int64_t num_q_heads,
  * workspace since. Calls in one stream may share it: each rewrites the
  * split-KV partials and counts its finished splits in it, and leaves the
  * counters at zero for the next. So two calls that share a workspace must not
- * overlap. None of this is checked: a mismatched plan, or an overlap, gives
- * wrong results, and may leave a counter off, which spoils every later call on
- * that workspace until mvllm_attention_plan has written it again. Every record
- * field is range-checked before it is used as an index.
+ * overlap: both may give wrong results (later calls are not affected). None of
+ * this is checked: a mismatched plan gives wrong results, and may leave a
+ * counter off, which spoils every later call on that workspace until
+ * mvllm_attention_plan has written it again. Every record field is
+ * range-checked before it is used as an index.
  */
 int mvllm_paged_attention_planned(const mvllm_tensor3* query,
                                   const mvllm_kv_cache* cache,

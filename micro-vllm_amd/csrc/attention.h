@@ -73,8 +73,8 @@ struct AttnArgs {
   // rows that no split writes are found from it.
   int2* decode_req;
   // Per (request, group of KV heads that share a workgroup): splits finished
-  // so far in this launch. Zeroed with the work list; the workgroup that
-  // completes a request zeroes its counter again.
+  // so far in this launch. Zeroed with the work list; the count wraps to zero
+  // with the workgroup that completes a request.
   int32_t* done;
   // Host side only: the work lists and the per-request table are already in
   // the workspace (planned once for a step), so the launches skip the

@@ -188,10 +188,11 @@ __device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem
   __syncthreads();
   int32_t* const counter = a.done + static_cast<int64_t>(item.r) * head_groups + head_group;
   if (threadIdx.x == 0) {
-    const int32_t before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // The last one leaves the counter at zero for the next launch.
-    if (before + 1 == item.ns) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *flag = before + 1 == item.ns;
+    // Counts to ns and wraps to zero for the next launch, in one operation: a
+    // reset of its own would lose counts that another launch on this workspace
+    // added in between, and leave the counter off for every later one.
+    const uint32_t last = static_cast<uint32_t>(item.ns) - 1;
+    *flag = atomicInc(reinterpret_cast<unsigned int*>(counter), last) == last;
   }
   __syncthreads();
   if (!*flag || !live) return;
