@@ -76,6 +76,9 @@ struct AttnArgs {
   // so far in this launch. Zeroed with the work list; the count wraps to zero
   // with the workgroup that completes a request.
   int32_t* done;
+  // The partials are merged by a launch of their own (merge_apart in
+  // attention_api.hip); `done` then holds each request's first partial row.
+  int32_t merge_apart;
   // Host side only: the work lists and the per-request table are already in
   // the workspace (planned once for a step), so the launches skip the
   // work-list kernels.
@@ -114,6 +117,9 @@ __device__ __forceinline__ int64_t block_of(const AttnArgs& a, int64_t r, int64_
 int launch_generic(const AttnArgs& a, int32_t dtype, hipStream_t s);
 int launch_decode(const AttnArgs& a, int32_t dtype, hipStream_t s, hipEvent_t start,
                   hipEvent_t stop);
+// The decode partials' merge, where it is a launch of its own (launch_decode
+// includes it).
+int launch_merge(const AttnArgs& a, int32_t dtype, hipStream_t s);
 // The work-list kernels alone (decode list + per-request table; prefill list).
 int launch_decode_lists(const AttnArgs& a, hipStream_t s);
 int launch_prefill_lists(const AttnArgs& a, hipStream_t s);

@@ -298,6 +298,36 @@ bool attention_fast_path(const mvllm_tensor3* query, const mvllm_kv_cache* cache
          vec16(out->stride[0], es) && vec16(out->stride[1], es) && aligned16(out->data);
 }
 
+// Nothing but decodes, by the hint or, without one, as far as the counts tell.
+bool looks_like_decodes(const mvllm_batch* batch) {
+  return batch->max_query_len == 1 || (batch->max_query_len < 0 && batch->num_tokens <= batch->num_requests);
+}
+
+// Whether a launch of its own merges the decode partials, a wave per two query
+// heads, instead of the workgroup that finishes a request. That workgroup merges
+// G heads per wave, all through one CU, which tells once G is above two or so and
+// the request has many splits: one context of 2,000 takes 26.0 us with 16/1 heads,
+// 24.2 with 28/4, 20.3 with 32/8 and 17.9 with 16/8, and 18.2, 18.9, 18.8 and 18.6
+// with the launch; one of 300 18.8, 16.9, 15.2 and 14.3, and 14.9, 15.4, 15.5 and
+// 14.7. But the launch takes 3 us of the caller's ~16 us per call, 0.5-1.5 us of
+// the GPU where nothing is left to merge, and prefill workgroups hide the merge (a
+// context of 2,000 and a prompt of 500 with 32/4 heads: 27.5, 31.6 with the
+// launch). So, by what is known before the call:
+// * above eight heads per KV head always;
+// * above four for batches that look like decodes and tables of more than 512
+//   tokens (one context of 1,000 with 28/4: 20.0 and 16.7);
+// * above two for such batches, more than 1,024 tokens, and requests that do not
+//   fill the chip by themselves (128 contexts of 150 .. 300 with 32/8 heads, which
+//   are not split: 27.9 and 29.3).
+bool merge_apart(const AttnArgs& a, const mvllm_batch* batch) {
+  const int64_t reach = a.width * a.block_size;
+  if (reach <= kSmallSplit) return false;  // no splits
+  if (a.group > 8) return true;
+  const int64_t groups = (a.num_kv_heads + 3) / 4;
+  const bool few = 4 * a.num_requests * groups < 3 * a.num_cus;
+  return looks_like_decodes(batch) && ((a.group > 4 && reach > 512) || (a.group > 2 && reach > 1024 && few));
+}
+
 // Split-KV partials, work lists and the per-request table in the workspace.
 int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D, void* workspace,
                    int64_t workspace_bytes) {
@@ -314,6 +344,7 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
                                   : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
                                                d.item_capacity, a.num_cus, D, a.num_kv_heads);
   a.decode_only = batch->max_query_len == 1 ? 1 : 0;
+  a.merge_apart = merge_apart(a, batch) ? 1 : 0;
   a.ws_acc = reinterpret_cast<float*>(w);
   a.ws_ml = reinterpret_cast<float2*>(w + d.acc_bytes);
   a.items = reinterpret_cast<PrefillItem*>(w + d.acc_bytes + d.ml_bytes);

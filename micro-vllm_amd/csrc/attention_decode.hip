@@ -210,6 +210,23 @@ __global__ __launch_bounds__(256, 2) void decode_split_lds_kernel(AttnArgs a) {
 }
 
 
+// The merge as a launch of its own: a workgroup of four waves takes
+// kMergeHeads query heads of one request, two per wave.
+constexpr int kMergeHeads = 8;
+
+template <typename T, int D>
+__global__ __launch_bounds__(256) void decode_merge_kernel(AttnArgs a, int32_t head_blocks) {
+  const int64_t r = blockIdx.x / head_blocks;
+  const int2 req = a.decode_req[r];  // (query token, splits)
+  const int64_t base = a.done[r];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head0 = static_cast<int>(blockIdx.x % head_blocks) * kMergeHeads + 2 * wave;
+  if (req.y <= 1 || req.x < 0 || req.x >= a.num_tokens || base < 0 || base + req.y > a.item_capacity ||
+      head0 >= a.num_q_heads)
+    return;
+  merge_request<T, D>(a, base, req.x, head0, a.num_q_heads - head0 < 2 ? 1 : 2, req.y);
+}
+
 __global__ __launch_bounds__(kDecodeListThreads) void decode_items_kernel(AttnArgs a) { build_decode_list(a); }
 
 struct DecodeTuning {
@@ -262,6 +279,16 @@ int launch_lds_kernel(const AttnArgs& a, dim3 grid, int waves, hipStream_t s, hi
   hipExtLaunchKernelGGL((decode_split_lds_kernel<T, D, STAGES>), grid, dim3(64 * waves), lds, s, start, stop,
                         0, a);
   MVLLM_LAUNCH_CHECK("decode_split_lds_kernel");
+  return MVLLM_OK;
+}
+
+template <typename T, int D>
+int launch_merge_t(const AttnArgs& a, hipStream_t s) {
+  const int32_t head_blocks = (a.num_q_heads + kMergeHeads - 1) / kMergeHeads;
+  const int64_t blocks = a.num_requests * head_blocks;
+  if (blocks > INT32_MAX) return fail(MVLLM_ERR_INVALID, "merge grid too large (%lld workgroups)", (long long)blocks);
+  hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a, head_blocks);
+  MVLLM_LAUNCH_CHECK("decode_merge_kernel");
   return MVLLM_OK;
 }
 
@@ -336,9 +363,16 @@ int launch_decode_lists(const AttnArgs& a, hipStream_t s) {
 
 int launch_decode(const AttnArgs& a, int32_t dtype, hipStream_t s, hipEvent_t start,
                   hipEvent_t stop) {
-  return for_decode_types(a, dtype, [&](auto t, auto d) {
-    return launch_decode_t<decltype(t), decltype(d)::value>(a, s, start, stop);
-  });
+  if (int rc = for_decode_types(a, dtype, [&](auto t, auto d) {
+        return launch_decode_t<decltype(t), decltype(d)::value>(a, s, start, stop);
+      }))
+    return rc;
+  return launch_merge(a, dtype, s);
+}
+
+int launch_merge(const AttnArgs& a, int32_t dtype, hipStream_t s) {
+  if (!a.merge_apart || a.num_requests <= 0) return MVLLM_OK;
+  return for_decode_types(a, dtype, [&](auto t, auto d) { return launch_merge_t<decltype(t), decltype(d)::value>(a, s); });
 }
 
 bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens) {

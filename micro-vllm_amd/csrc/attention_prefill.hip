@@ -1034,9 +1034,11 @@ int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_
     return fail(MVLLM_ERR_UNSUPPORTED, "the attention step kernel does not support this geometry");
   if (a.width * a.block_size > INT32_MAX || a.num_tokens > INT32_MAX)
     return fail(MVLLM_ERR_UNSUPPORTED, "decode positions beyond 2^31 are not supported");
-  return for_prefill_types(a, dtype, [&](auto t, auto d) {
-    return launch_step_t<decltype(t), decltype(d)::value>(a, prefill_first, s, start, stop);
-  });
+  if (int rc = for_prefill_types(a, dtype, [&](auto t, auto d) {
+        return launch_step_t<decltype(t), decltype(d)::value>(a, prefill_first, s, start, stop);
+      }))
+    return rc;
+  return launch_merge(a, dtype, s);
 }
 
 }  // namespace mvllm

@@ -51,13 +51,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);
 }
 
-// Merges `ns` partials (rows base, base + 1, ...) of query token `qs` for the G
-// query heads of KV head `h`, one wave: 32 lanes per query head, 4 dims each
+// Merges `ns` partials (rows base, base + 1, ...) of query token `qs` for `heads`
+// query heads from `head0`, one wave: 32 lanes per query head, 4 dims each
 // (at head_dim 64 and 96 the last lanes only merge statistics), with the
 // log-sum-exp rule. A round takes up to CAP splits (MANY: several rounds) of
 // PAIRS pairs of heads, about 32 rows, whose loads are issued together.
 template <typename T, int D, int CAP, bool MANY>
-__device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t base, int64_t qs, int h, int ns) {
+__device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t base, int64_t qs, int head0, int heads, int ns) {
   static_assert(CAP <= 32, "one lane per split of a round");
   constexpr int PAIRS = CAP <= 8 ? 4 : CAP <= 16 ? 2 : 1;
   const int sub = threadIdx.x & 31;
@@ -65,10 +65,10 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t base, in
   const bool has_dims = 4 * sub < D;
   const int d0 = has_dims ? 4 * sub : 0;
   const int64_t row0 = base * a.num_q_heads;  // partial row of (split 0, head 0)
-  for (int g0 = 0; g0 < a.group; g0 += 2 * PAIRS) {
-    auto pair_live = [&](int p) { return g0 + 2 * p < a.group; };  // wave-uniform
-    auto head_live = [&](int p) { return g0 + 2 * p + half < a.group; };
-    auto head = [&](int p) { return h * a.group + g0 + 2 * p + (head_live(p) ? half : 0); };
+  for (int g0 = 0; g0 < heads; g0 += 2 * PAIRS) {
+    auto pair_live = [&](int p) { return g0 + 2 * p < heads; };  // wave-uniform
+    auto head_live = [&](int p) { return g0 + 2 * p + half < heads; };
+    auto head = [&](int p) { return head0 + g0 + 2 * p + (head_live(p) ? half : 0); };
     // This lane's split of a round: its (max, sum), or (-inf, 0) past the end.
     auto round_stats = [&](int s0, int p) {
       const bool own = sub < CAP && s0 + sub < ns;
@@ -142,6 +142,18 @@ __device__ __forceinline__ void merge_splits(const AttnArgs& a, int64_t base, in
   }
 }
 
+// merge_splits with the round that fits `ns`.
+template <typename T, int D>
+__device__ __forceinline__ void merge_request(const AttnArgs& a, int64_t base, int64_t qs, int head0, int heads, int ns) {
+  if (ns <= 2) merge_splits<T, D, 2, false>(a, base, qs, head0, heads, ns);
+  else if (ns <= 4) merge_splits<T, D, 4, false>(a, base, qs, head0, heads, ns);
+  else if (ns <= 8) merge_splits<T, D, 8, false>(a, base, qs, head0, heads, ns);
+  else if (ns <= 16) merge_splits<T, D, 16, false>(a, base, qs, head0, heads, ns);
+  else if (ns <= 24) merge_splits<T, D, 24, false>(a, base, qs, head0, heads, ns);
+  else if (ns <= 32) merge_splits<T, D, 32, false>(a, base, qs, head0, heads, ns);
+  else merge_splits<T, D, 32, true>(a, base, qs, head0, heads, ns);
+}
+
 // Epilogue shared by the decode kernels, entered by every wave of the
 // workgroup (`live`: the wave has a KV head). acc[b][e] is
 // O[head h*G + col][dim 16b + 4grp + e] (unnormalised), m / lt the running
@@ -183,6 +195,7 @@ __device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem
                          static_cast<uint64_t>(__float_as_uint(m)) | (static_cast<uint64_t>(__float_as_uint(lt)) << 32),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  if (a.merge_apart) return;
   // This wave's partials have reached the point all XCDs read from.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -196,13 +209,7 @@ __device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem
   }
   __syncthreads();
   if (!*flag || !live) return;
-  const int hu = __builtin_amdgcn_readfirstlane(h);
-  if (item.ns <= 2) merge_splits<T, D, 2, false>(a, item.base, item.qs, hu, item.ns);
-  else if (item.ns <= 4) merge_splits<T, D, 4, false>(a, item.base, item.qs, hu, item.ns);
-  else if (item.ns <= 8) merge_splits<T, D, 8, false>(a, item.base, item.qs, hu, item.ns);
-  else if (item.ns <= 16) merge_splits<T, D, 16, false>(a, item.base, item.qs, hu, item.ns);
-  else if (item.ns <= 24) merge_splits<T, D, 24, false>(a, item.base, item.qs, hu, item.ns);
-  else merge_splits<T, D, 32, true>(a, item.base, item.qs, hu, item.ns);
+  merge_request<T, D>(a, item.base, item.qs, __builtin_amdgcn_readfirstlane(h) * G, G, item.ns);
 }
 
 // Output rows that no split writes, kTidyTokens tokens and as many requests

@@ -295,10 +295,14 @@ __device__ inline void build_decode_list(const AttnArgs& a) {
     };
     for (int32_t sp = 0; sp < nfull; ++sp) place(at + sp, sp);
     if (partial) place(atomicAdd(&bucket[(last - 1) >> bucket_shift], 1), ns - 1);
-    if (r < R) a.decode_req[r] = int2{d.qs, d.dec ? ns : -1};
+    if (r < R) {
+      a.decode_req[r] = int2{d.qs, d.dec ? ns : -1};
+      if (a.merge_apart) a.done[r] = base;
+    }
   }
   // At most one counter per (request, KV head).
-  for (int64_t j = tid; j < R * a.num_kv_heads; j += kDecodeListThreads) a.done[j] = 0;
+  if (!a.merge_apart)
+    for (int64_t j = tid; j < R * a.num_kv_heads; j += kDecodeListThreads) a.done[j] = 0;
   for (int64_t j = full_count + tid; j < capacity; j += kDecodeListThreads)
     a.decode_items[j] = DecodeItem{-1, -1, 0, 0, 0, 0, 0, -1};
 }
