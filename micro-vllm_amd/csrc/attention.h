@@ -31,6 +31,21 @@ struct PrefillItem {
   int32_t lo, hi, pad0, pad1;
 };
 
+// How long the decode splits are (worklists.h): rates in split tokens per token
+// of the batch, and bounds.
+struct SplitRule {
+  float small, full;                // while the work does not fill the chip; when it does
+  float beside_small, beside_full;  // the same beside prefill work
+  float waves;                      // one wave per SIMD
+  float fits;                       // 1 / (slots beyond one per request), or 0
+  float whole;                      // longest request answered whole, per token of the batch
+  int32_t whole_decodes;            // requests that fill the chip by themselves
+  int32_t least;                    // a shorter split than this is only for few tokens
+  int32_t beside_most;              // longest split beside prefill work
+  int32_t merge_apart;              // the partials are merged by a launch of their own
+  int32_t beside_merge;             // splits per request beside prefill work, up to 128 tokens each (0: no bound)
+};
+
 // Everything a ragged paged-attention launch needs. Strides are in elements.
 struct AttnArgs {
   const void* q;
@@ -60,6 +75,7 @@ struct AttnArgs {
   int32_t split_tokens;   // bound on the length of a split
   int32_t split_fixed;    // the length of every split, or 0: chosen with the work list
   int32_t num_cus;
+  SplitRule rule;
   int32_t mode;  // generic kernel: 0 = every token; 1 = only requests with > 1 query
   // Prefill work list: one record per (request, query block) slot, heaviest
   // first; r = -1 marks an empty slot. Written by the item kernel before the

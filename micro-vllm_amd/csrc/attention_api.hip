@@ -342,9 +342,10 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
   a.num_cus = device_cu_count();
   a.item_capacity = a.split_fixed ? d.item_capacity
                                   : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
-                                               d.item_capacity, a.num_cus, D, a.num_kv_heads);
+                                               d.item_capacity, a.num_cus, D, a.num_kv_heads, looks_like_decodes(batch));
   a.decode_only = batch->max_query_len == 1 ? 1 : 0;
   a.merge_apart = merge_apart(a, batch) ? 1 : 0;
+  a.rule = split_rule(a);
   a.ws_acc = reinterpret_cast<float*>(w);
   a.ws_ml = reinterpret_cast<float2*>(w + d.acc_bytes);
   a.items = reinterpret_cast<PrefillItem*>(w + d.acc_bytes + d.ml_bytes);

@@ -87,21 +87,31 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 // ends on the shortest items. Empty slots (up to the capacity) get request -1.
 //
 // The split length follows from the visible tokens, which only the device
-// knows. A split costs a workgroup ~5 us besides its tiles (metadata, the
-// pipeline's start, the partial and its merge), and a tile of a workgroup that
-// has a CU to itself ~0.65 us. So (times per forward, captured back to back):
-// * while the work does not fill the chip, as many items as the CUs take at
-//   one workgroup each (96 items: two workgroups of four KV heads per item at
-//   8 KV heads), of 64 to 256 tokens. 8 contexts of 128 .. 4,096: 36.1 us with
-//   64-token splits, 23.3 with 192, 34.1 with 512; one context of 1,024: 13.7
-//   with 64, 21.0 with 256;
-//   (With one KV head an item is one wave: up to 128 tokens then; 209 decodes
-//   of 55 .. 542 with 16 heads on one: 23.4 us with 128, 27.0 with 256.)
+// knows; the numbers of items it aims at follow from the shape (split_rule). A
+// split costs a workgroup ~5 us besides its tiles (metadata, the pipeline's
+// start, the partial and its merge), and a tile of a workgroup that has a CU to
+// itself ~0.65 us. A workgroup holds up to four KV heads, one wave each, so an
+// item is ceil(heads / 4) workgroups, of fewer waves below four heads. So (us per
+// forward, captured back to back; head_dim 128, narrower tokens count by their
+// bytes):
+// * while the work does not fill the chip, one workgroup for three quarters of
+//   the CUs, of 64 to 256 tokens; with two or three KV heads, whose workgroups
+//   leave room, one per CU of up to 192, and with one head two of up to 128. 8
+//   contexts of 128 .. 4,096 with 8 heads: 36.1 with 64-token splits, 23.3 with
+//   192, 34.1 with 512; one context of 1,024: 13.7 with 64, 21.0 with 256. 96
+//   items whatever the heads, as for 8, had taken, for 32 contexts of 500 ..
+//   1,000 with 4 heads 23.5 (18.9 with 192 items) and with 2 23.1 (17.3 with
+//   256), and for 4 of 1,000 .. 2,000 with 16 heads 23.2 (20.9 with 48);
 // * beyond that, about two items per CU of up to 1,024 tokens (64 contexts of
-//   8k .. 33k: 868 us, 907 with 2,048; 256 of 128 .. 4,096: 361, 379 with
-//   256), or, beside prefill work, whose workgroups fill the chip as well,
-//   half an item per CU of up to 2,048 (248 decodes and 8 chunks of 512: 736
-//   us with 2,048, 781 with 512);
+//   8k .. 33k: 868, 907 with 2,048; 256 of 128 .. 4,096: 361, 379 with 256),
+//   four with fewer than four KV heads (128 contexts of 2,000 .. 4,000 with 14/2
+//   heads: 90 with two per CU, 82 with four);
+// * beside prefill work, whose workgroups fill the chip as well, half an item per
+//   CU of up to 2,048 (248 decodes and 8 chunks of 512: 736 with 2,048, 781 with
+//   512). One per CU of up to 768 with four KV heads (128 decodes of 3,000 ..
+//   6,000 and a chunk of 40 with 32/4: 230 with 2,048, 216 with 768), and one and
+//   a half per CU below four (128 of 1,000 .. 2,000 with one KV head: 84.5 with
+//   half an item per CU, 39 with one and a half);
 // * no splits at all where the requests alone fill the chip (workgroups for
 //   three quarters of the CUs), are about even or short, and the longest one's
 //   tiles take no longer than the whole batch takes at the HBM's rate (0.04 us
@@ -111,54 +121,95 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 //   (uneven ones of up to 965 keys are better off split: 83.0 whole, 80.6);
 // * at most 32 splits per request up to 512 tokens each: the merge loads 32
 //   at a time (one context of 32k: 143 us with 64-token splits, 47 with 512).
+//   Where a launch of its own merges, a wave per two heads: 32 up to 256, then 64
+//   while the work leaves SIMDs idle (one context of 16k with 28/4 heads: 39.6
+//   with 512, 33.0 with 256; four with 32/8: 49 with 512, 57 with 256). Beside
+//   prefill work 16 up to 128 tokens each where one wave merges more than four
+//   heads (a context of 2,000 and a chunk of 40 with 32/4 heads: 25.8 with 64,
+//   22.2 with 128).
 // At least total / (capacity - R), so that the items fit the list: a request
 // of v tokens has at most v / split + 1 splits. (2,048-token splits always fit:
 // see item_slots.)
 constexpr int kDecodeListThreads = 1024;
 constexpr int kSizeBuckets = 64;  // sizes of a partial split, split / 64 tokens (rounded up to a power of two) each
+constexpr int32_t kSmallSplit = 64, kMostSplit = 1024;
 
-// (The figures are for head_dim 128; narrower tokens count by their bytes.)
-constexpr int32_t kSmallItems = 96, kSmallSplit = 64, kMostSplit = 1024;
-__host__ __device__ inline int32_t full_split(int32_t num_kv_heads) { return num_kv_heads == 1 ? 128 : 256; }
+// Items (of 128-wide tokens) that a batch is split into, at most, by the rule above.
+inline int32_t small_items(int32_t cus, int32_t num_kv_heads) {
+  const int32_t items =
+      num_kv_heads == 1 ? 2 * cus : num_kv_heads < 4 ? cus : 3 * cus / (4 * ((num_kv_heads + 3) / 4));
+  return items > 1 ? items : 1;
+}
+inline int32_t full_items(int32_t cus, int32_t num_kv_heads) { return num_kv_heads < 4 ? 4 * cus : 2 * cus; }
+inline int32_t full_split(int32_t num_kv_heads) { return num_kv_heads == 1 ? 128 : num_kv_heads < 4 ? 192 : 256; }
+
+// The rule's numbers for a shape. Rates turn tokens into a split length.
+inline SplitRule split_rule(const AttnArgs& a) {
+  const int32_t heads = a.num_kv_heads, cus = a.num_cus;
+  const float width = a.head_dim / 128.f;
+  SplitRule r;
+  r.small = width / small_items(cus, heads);
+  r.full = width / full_items(cus, heads);
+  r.beside_small = width / 96.f;
+  r.beside_full = width / (heads < 4 ? 1.5f * cus : heads == 4 ? 1.f * cus : 0.5f * cus);
+  r.waves = width * heads / (4.f * cus);
+  r.fits = a.item_capacity > a.num_requests ? 1.f / static_cast<float>(a.item_capacity - a.num_requests) : 0.f;
+  r.whole = heads * a.head_dim / (0.04f * 1.55e6f);
+  r.whole_decodes = (3 * cus + 4 * ((heads + 3) / 4) - 1) / (4 * ((heads + 3) / 4));
+  r.least = full_split(heads);
+  r.beside_most = heads == 4 ? 768 : kMaxSplit;
+  r.merge_apart = a.merge_apart;
+  r.beside_merge = !a.merge_apart && a.group > 4 ? 16 : 0;
+  return r;
+}
 
 // Slots of the decode work list and of the decode grid, from shapes alone: at
 // most `capacity` (the workspace's) and no more than choose_split can fill. A
 // slot that stays empty still costs a workgroup's dispatch (~4 ns: 1,500 of
 // them took 6 of the 37 us of 30 decodes and two chunks at head_dim 64).
 // Splits of 2,048 tokens fit every one of the bounds.
+// `decodes`: the batch looks like decodes alone. Beside prefill work spare slots
+// cost more than their dispatch: the work is then spread over the CUs unevenly (8
+// decodes of 2,000 and a chunk of 500 with 32/4 heads: 27.5, 32.0 with 96 more).
 inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int64_t cus, int64_t head_dim,
-                          int32_t num_kv_heads) {
+                          int32_t num_kv_heads, bool decodes) {
   auto least = [](int64_t x, int64_t y) { return x < y ? x : y; };
   auto larger = [](int64_t x, int64_t y) { return x > y ? x : y; };
   const int64_t tokens = requests * reach;
-  const int64_t small = kSmallItems * 128 / head_dim + 1;
-  const int64_t full = least(2 * cus * 128 / head_dim, tokens / full_split(num_kv_heads)) + 1;
+  const int64_t small = (decodes ? small_items(static_cast<int32_t>(cus), num_kv_heads) : 96) * 128 / head_dim + 1;
+  const int64_t full = least(full_items(static_cast<int32_t>(cus), num_kv_heads) * 128LL / head_dim,
+                             tokens / full_split(num_kv_heads)) + 1;
   const int64_t slots = requests + larger(larger(small, full), tokens / kMostSplit + 1);
   return least(least(slots, requests * ((reach + kSmallSplit - 1) / kSmallSplit)), capacity);
 }
 
-__device__ inline int32_t choose_split(int64_t total, int32_t longest, int64_t requests, int64_t capacity,
-                                       int32_t cus, int32_t head_dim, int32_t num_kv_heads, int32_t decodes,
-                                       bool beside_prefill) {
-  // Quotients in float (a 64-bit division takes longer than the rest of the
+__host__ __device__ inline int32_t choose_split(int64_t total, int32_t longest, int32_t decodes, bool beside_prefill,
+                                       const SplitRule& rule) {
+  // Quotients as products in float (divisions take longer than the rest of the
   // rule), raised by more than their error; lengths past 2^20 mean the same.
   auto up16 = [](float v) { return (static_cast<int32_t>(fminf(v * 1.000001f, 1048576.f)) + 16) & ~15; };
   const float tokens = static_cast<float>(total);
-  const float wide = tokens * head_dim / 128.f;
-  const int32_t groups = (num_kv_heads + 3) / 4;
-  if (!beside_prefill && longest <= kMostSplit && 4.f * decodes * groups >= 3.f * cus &&
-      (longest <= 320 || tokens >= 0.75f * longest * decodes) &&
-      0.04f * longest <= tokens * num_kv_heads * head_dim / 1.55e6f)
+  if (!beside_prefill && longest <= kMostSplit && decodes >= rule.whole_decodes &&
+      (longest <= 320 || tokens >= 0.75f * longest * decodes) && longest <= tokens * rule.whole)
     return (longest + 15) & ~15;
-  const int32_t most = beside_prefill ? kMaxSplit : kMostSplit;
-  int32_t split = up16(wide / (beside_prefill ? 0.5f * cus : 2.f * cus));
-  int32_t least = up16(wide / kSmallItems);
-  const int32_t full = full_split(num_kv_heads);
-  least = least < kSmallSplit ? kSmallSplit : least > full ? full : least;
+  const int32_t most = beside_prefill ? rule.beside_most : kMostSplit;
+  int32_t split = up16(tokens * (beside_prefill ? rule.beside_full : rule.full));
+  int32_t least = up16(tokens * (beside_prefill ? rule.beside_small : rule.small));
+  least = least < kSmallSplit ? kSmallSplit : least > rule.least ? rule.least : least;
+  if (beside_prefill && rule.beside_merge > 0) {
+    const int32_t few = longest / rule.beside_merge < 112 ? (longest / rule.beside_merge + 16) & ~15 : 128;
+    least = least < few ? few : least;
+  }
   split = split < least ? least : split > most ? most : split;
-  const int32_t by_merge = (longest / 32 + 16) & ~15;
+  int32_t by_merge = (longest / 32 + 16) & ~15;
+  if (rule.merge_apart && by_merge > 256) {
+    const int32_t by_waves = up16(tokens * rule.waves);
+    const int32_t by_64 = (longest / 64 + 16) & ~15;
+    const int32_t more = by_64 > by_waves ? by_64 : by_waves;
+    by_merge = more < 256 ? 256 : more < by_merge ? more : by_merge;
+  }
   if (split < by_merge) split = by_merge < 512 ? by_merge : split < 512 ? 512 : split;
-  const int32_t fits = capacity > requests ? up16(tokens / static_cast<float>(capacity - requests)) : kMaxSplit;
+  const int32_t fits = rule.fits > 0.f ? up16(tokens * rule.fits) : kMaxSplit;
   if (split < fits) split = fits;
   return split < kMaxSplit ? split : kMaxSplit;
 }
@@ -236,8 +287,7 @@ __device__ inline void build_decode_list(const AttnArgs& a) {
       }
     }
     __syncthreads();
-    split = choose_split(16 * static_cast<int64_t>(pages), longest, R, capacity, a.num_cus, a.head_dim,
-                         a.num_kv_heads, decodes, others && !a.decode_only);
+    split = choose_split(16 * static_cast<int64_t>(pages), longest, decodes, others && !a.decode_only, a.rule);
   }
   // 64 buckets of 2^bucket_shift sizes span every split length: the smallest
   // shift with 64 << shift >= split (a partial split holds 1 .. split - 1
