@@ -259,7 +259,7 @@ bool fast_cache(const mvllm_kv_cache* cache, int64_t group) {
   const int64_t es = dtype_bytes(dtype);
   return (dtype == MVLLM_DTYPE_BF16 || dtype == MVLLM_DTYPE_F16) && group <= 16 &&
          decode_supported(cache->head_dim, cache->block_size, decode_split_override()) &&
-         32 * cache->stride[2] < (int64_t{1} << 32) &&  // 16 rows within a 32-bit byte offset
+         (cache->head_dim == 128 || rows_within_32_bits(cache->stride[2])) &&
          cache->stride[4] == 1 && cache->stride[3] == cache->head_dim && vec16(cache->stride[0], es) &&
          vec16(cache->stride[1], es) && vec16(cache->stride[2], es) && aligned16(cache->data);
 }

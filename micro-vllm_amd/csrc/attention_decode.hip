@@ -239,7 +239,7 @@ struct DecodeTuning {
 
 DecodeTuning decode_tuning(const AttnArgs& a) {
   DecodeTuning t;
-  t.lds_pipeline = a.block_size % 16 == 0 && a.split_tokens <= kMaxSplit;
+  t.lds_pipeline = a.block_size % 16 == 0 && a.split_tokens <= kMaxSplit && rows_within_32_bits(a.c_s[2]);
   t.waves = 4;
   t.stages = a.head_dim == 64 ? kStages<64> : a.head_dim == 96 ? kStages<96> : kStages<128>;
   t.prefetch = false;
