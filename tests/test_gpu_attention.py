@@ -258,10 +258,10 @@ def test_decode_kernel_group_sizes_and_context_boundaries(device, dtype, hq, hkv
     ids=["9-splits", "17-splits", "48-splits"],
 )
 def test_decode_combine_of_many_splits(device, requests, longest):
-    """Split lengths follow the batch (about two items per CU, at least 64
-    tokens), so smaller batches split each request more finely: on 256 CUs
-    these batches reach 9, 17 and 48 splits per request, which the combine
-    merges from one round of loads (up to 16 and 32) or in passes."""
+    """Split lengths follow the batch, so smaller batches split each request
+    more finely: on 256 CUs the longest request of these batches has about 4, 11
+    and 27 splits (their names are the counts that their tables' reach would
+    give), each merged from one round of loads."""
 
     rng = np.random.default_rng(requests)
     lengths = rng.integers(1, longest + 1, size=requests)

@@ -4,7 +4,9 @@ Batches at the ends of the rule that picks the split length (every request at
 the table's full reach, so the work list is as full as it gets; one long
 context beside many short ones; more requests than the list builder's
 threads; contexts around the shortest split), and at every size of merge
-round (up to 2, 4, 8, 16, 24, 32 and more splits), against the oracle.
+round (up to 2, 4, 8, 16, 24, 32 and more splits: the two "merge-rounds" batches
+give 1-2, 4, 8, 12, 16 and 32 and 5, 11, 21, 23 and 30 on 256 CUs, "one-long" 40),
+against the oracle.
 """
 
 from __future__ import annotations
@@ -28,6 +30,7 @@ BATCHES = {
     "many-requests": [1 + (37 * i) % 400 for i in range(1100)],
     "around-the-shortest-split": [191, 192, 193, 207, 208, 209, 383, 384, 385],
     "merge-rounds": [300, 700, 1500, 3000, 4500, 6100, 12_000],
+    "merge-rounds-short": [300, 700, 1300, 1450, 1900],
     "single": [6145],
     "whole-even": [1000 + r % 20 for r in range(110)],
     "whole-short": [1 + (r * 7) % 320 for r in range(200)],

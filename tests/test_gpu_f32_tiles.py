@@ -28,6 +28,15 @@ def test_groups_tiles_and_specs(device, d, hq, hkv, bs, spec):
     run_and_check(q, k, v, cache, md, torch.float32)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize(("hq", "hkv"), [(16, 8), (16, 1)], ids=str)
+def test_long_contexts(device, d, hq, hkv):
+    """Contexts of many rounds of the eight waves' tiles, one of them a chunk."""
+
+    q, k, v, cache, md = build_case(device, torch.float32, [20_000, 8193, 9001], [1, 1, 7], hq, hkv, d, 16, seed=d)
+    run_and_check(q, k, v, cache, md, torch.float32)
+
+
 @pytest.mark.parametrize("requests", [1, 63, 64, 65, 700, 4100])
 def test_request_search(device, requests):
     """The 64-ary search over one, two and three rounds, empty requests between."""
