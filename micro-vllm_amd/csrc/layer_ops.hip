@@ -388,8 +388,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(SiluArgs a) {
       static_cast<uint32_t>(Act<T>::store(r[0])) | (static_cast<uint32_t>(Act<T>::store(r[1])) << 16);
 }
 
-// Eight elements per thread and row, ROWS rows per thread, all loads issued
-// before the arithmetic.
+// Eight elements per thread, both loads issued before the arithmetic.
 //
 // The bound is HBM (6 bytes per output element), but the library's expf and
 // the IEEE division take ~60 vector instructions per element, more than the
@@ -399,79 +398,66 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(SiluArgs a) {
 // correction: both within an ulp or so, as the library's, before the rounding
 // to 16 bits. A vector with an |x| of 80 or more, where 1 + exp(-x) leaves the
 // range of the reciprocal, or a NaN takes the library's functions. 8,192 rows
-// of 14,336: 179 us before (3.9 TB/s), 127 us now (5.5 TB/s).
-template <typename T, int ROWS>
+// of 14,336 in a kernel trace, between a layer's other kernels: 195.7 us before
+// (3.6 TB/s), 136.0 now (5.2; 122 back to back). Two
+// rows per thread, all loads first, are no faster at any size (back to back
+// 124.9 us against 122.0; 1,170 rows 18.9 and 18.1, 146 rows 6.7 and 6.7).
+template <typename T>
 __global__ __launch_bounds__(128) void silu_mul_rows_kernel(SiluArgs a) {
   const int chunk = static_cast<int>(blockIdx.x) * 128 + threadIdx.x;
   if (8 * chunk >= a.inter) return;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.y) * ROWS;
-  uint4 gv[ROWS], uv[ROWS];
+  const int64_t row = blockIdx.y;
+  const uint16_t* g = a.gate_up + row * a.in_stride + 8 * chunk;
+  const uint4 gv = *reinterpret_cast<const uint4*>(g);
+  const uint4 uv = *reinterpret_cast<const uint4*>(g + a.inter);
+  const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w};
+  const uint32_t uw[4] = {uv.x, uv.y, uv.z, uv.w};
+  float x[8], s[8];
+  float most = 0.f;
+  bool number = true;
 #pragma unroll
-  for (int k = 0; k < ROWS; ++k) {
-    const int64_t row = row0 + k < a.rows ? row0 + k : a.rows - 1;
-    const uint16_t* g = a.gate_up + row * a.in_stride + 8 * chunk;
-    gv[k] = *reinterpret_cast<const uint4*>(g);
-    uv[k] = *reinterpret_cast<const uint4*>(g + a.inter);
+  for (int e = 0; e < 8; ++e) {
+    x[e] = Act<T>::load((gw[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
+    most = fmaxf(most, fabsf(x[e]));
+    number = number && x[e] == x[e];
   }
-#pragma unroll
-  for (int k = 0; k < ROWS; ++k) {
-    const uint32_t gw[4] = {gv[k].x, gv[k].y, gv[k].z, gv[k].w};
-    const uint32_t uw[4] = {uv[k].x, uv[k].y, uv[k].z, uv[k].w};
-    float x[8], s[8];
-    float most = 0.f;
-    bool number = true;
+  if (most < 80.f && number) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      x[e] = Act<T>::load((gw[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
-      most = fmaxf(most, fabsf(x[e]));
-      number = number && x[e] == x[e];
+      constexpr float kLog2e = 1.44269504f;           // log2(e) rounded to float
+      constexpr float kLog2eLow = 1.92596303e-8f;     // log2(e) - kLog2e
+      constexpr float kLn2 = 0.693147181f;
+      const float t = x[e] * -kLog2e;
+      const float low = __builtin_fmaf(x[e], -kLog2eLow, __builtin_fmaf(x[e], -kLog2e, -t));
+      const float e0 = __builtin_amdgcn_exp2f(t);
+      const float d = 1.f + __builtin_fmaf(e0, low * kLn2, e0);
+      float y = __builtin_amdgcn_rcpf(d);
+      y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
+      const float q = x[e] * y;
+      // The sign is x's: the correction turns -0 into +0.
+      s[e] = Act<T>::round(copysignf(__builtin_fmaf(__builtin_fmaf(-d, q, x[e]), y, q), x[e]));
     }
-    if (most < 80.f && number) {
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        constexpr float kLog2e = 1.44269504f;           // log2(e) rounded to float
-        constexpr float kLog2eLow = 1.92596303e-8f;     // log2(e) - kLog2e
-        constexpr float kLn2 = 0.693147181f;
-        const float t = x[e] * -kLog2e;
-        const float low = __builtin_fmaf(x[e], -kLog2eLow, __builtin_fmaf(x[e], -kLog2e, -t));
-        const float e0 = __builtin_amdgcn_exp2f(t);
-        const float d = 1.f + __builtin_fmaf(e0, low * kLn2, e0);
-        float y = __builtin_amdgcn_rcpf(d);
-        y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
-        const float q = x[e] * y;
-        // The sign is x's: the correction turns -0 into +0.
-        s[e] = Act<T>::round(copysignf(__builtin_fmaf(__builtin_fmaf(-d, q, x[e]), y, q), x[e]));
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s[e] = silu_any<T>(x[e]);
-    }
-    uint32_t ow[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float p0 = s[2 * e] * Act<T>::load(uw[e] & 0xFFFFu);
-      float p1 = s[2 * e + 1] * Act<T>::load(uw[e] >> 16);
-      // Opaque, so that product and fp16 rounding are not merged into a
-      // mixed-precision fma, whose +0 addend loses the sign of a zero.
-      asm volatile("" : "+v"(p0), "+v"(p1));
-      ow[e] = static_cast<uint32_t>(Act<T>::store(p0)) | (static_cast<uint32_t>(Act<T>::store(p1)) << 16);
-    }
-    if (row0 + k < a.rows)
-      *reinterpret_cast<uint4*>(a.out + (row0 + k) * a.out_stride + 8 * chunk) = uint4{ow[0], ow[1], ow[2], ow[3]};
+    for (int e = 0; e < 8; ++e) s[e] = silu_any<T>(x[e]);
   }
+  uint32_t ow[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float p0 = s[2 * e] * Act<T>::load(uw[e] & 0xFFFFu);
+    float p1 = s[2 * e + 1] * Act<T>::load(uw[e] >> 16);
+    // Opaque, so that product and fp16 rounding are not merged into a
+    // mixed-precision fma, whose +0 addend loses the sign of a zero.
+    asm volatile("" : "+v"(p0), "+v"(p1));
+    ow[e] = static_cast<uint32_t>(Act<T>::store(p0)) | (static_cast<uint32_t>(Act<T>::store(p1)) << 16);
+  }
+  *reinterpret_cast<uint4*>(a.out + row * a.out_stride + 8 * chunk) = uint4{ow[0], ow[1], ow[2], ow[3]};
 }
 
 template <typename T>
 void launch_silu_rows(const SiluArgs& a, hipStream_t s) {
   const unsigned x = static_cast<unsigned>((a.inter / 8 + 127) / 128);
-  // Two rows per thread once the grid holds 8 workgroups of two waves per
-  // SIMD-filling round of 256 CUs without them (more loads in flight); one
-  // row below that, where the launch itself is the time (8.7 us for 256 rows
-  // of 3,072 and for one row alike).
-  if (static_cast<int64_t>(x) * a.rows >= 16384)
-    hipLaunchKernelGGL((silu_mul_rows_kernel<T, 2>), dim3(x, static_cast<unsigned>((a.rows + 1) / 2)), dim3(128), 0, s, a);
-  else
-    hipLaunchKernelGGL((silu_mul_rows_kernel<T, 1>), dim3(x, static_cast<unsigned>(a.rows)), dim3(128), 0, s, a);
+  hipLaunchKernelGGL(silu_mul_rows_kernel<T>, dim3(x, static_cast<unsigned>(a.rows)), dim3(128), 0, s, a);
 }
 
 // ------------------------------------------------------------ argmax_rows

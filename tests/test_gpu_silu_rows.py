@@ -38,8 +38,8 @@ def test_every_gate_value(device, dtype, factor):
 
 @pytest.mark.parametrize(("rows", "inter"), [(1, 8), (3, 1024), (5, 1032), (257, 3072), (1171, 14336)])
 def test_row_and_column_remainders(device, rows, inter):
-    """One and two rows per thread (the last shape), odd row counts, row
-    widths that end inside a workgroup, and a padded row stride."""
+    """Odd row counts, row widths that end inside a workgroup, and a padded row
+    stride."""
 
     wide = torch.randn((rows, 2 * inter + 16), device=device).to(torch.bfloat16)
     gate_up = wide[:, : 2 * inter]
