@@ -123,7 +123,8 @@ int mvllm_kv_write(const mvllm_tensor3* key, const mvllm_tensor3* value,
  * Bytes of device workspace mvllm_paged_attention / mvllm_attention_forward
  * need for this batch geometry: the split-KV partial results of the decode
  * kernel, the decode and prefill work lists and the counters of finished
- * splits, which the library writes before it reads them (the caller need not initialise the workspace).
+ * splits, which the library writes before it reads them (the caller need not
+ * initialise the workspace).
  * Decode positions must stay below 2^31 (block-table width * block size).
  * Depends only on
  * shapes, never on device data, so it can be sized before graph capture.

@@ -81,8 +81,8 @@ struct AttnArgs {
   // first; r = -1 marks an empty slot. Written by the item kernel before the
   // prefill kernel reads it.
   PrefillItem* items;
-  // Decode work list: one record per (request, split), full splits first, then the partial last splits from the largest; r = -1 marks an
-  // empty slot.
+  // Decode work list: one record per (request, split), full splits first, then
+  // the partial last splits from the largest; r = -1 marks an empty slot.
   DecodeItem* decode_items;
   // Per request, written with the decode work list: (query token, number of
   // splits), or (0, -1) for a request that is not a single-query decode. The
@@ -145,7 +145,8 @@ bool prefill_supported(const AttnArgs& a, int32_t dtype);
 
 // The one-launch attention step: decode and prefill workgroups in one grid
 // (attention_prefill.hip), for batches whose decode part runs the pipelined
-// kernel with its default shape (kStepDecodeWaves waves, two stages).
+// kernel with its default shape (kStepDecodeWaves waves; two stages at head_dim
+// 128, three at 96, four at 64).
 constexpr int kStepDecodeWaves = 4;
 bool decode_step_eligible(const AttnArgs& a);
 // The split-KV decode kernels cover this head_dim with this block size and

@@ -266,8 +266,8 @@ bool fast_cache(const mvllm_kv_cache* cache, int64_t group) {
 
 // head_dim 64 and 96 take the MFMA kernels because the generic kernel scores
 // one key per lane without matrix instructions: a batch of 30 decodes (128 to
-// 2,048 keys) and two chunks of ~230 tokens with 32/8 heads of 64 took 1,414 us
-// per forward there and takes 47 us here. Both are still answered by the
+// 2,048 keys) and two chunks of ~230 tokens with 32/8 heads of 64 took 1,405 us
+// per forward there and takes 34.7 us here. Both are still answered by the
 // generic kernel, which needs no workspace and has no limits on reach or grid; calls outside the work
 // lists' limits therefore go there instead of failing. At head_dim 128 the
 // limits are errors of their own (bind_workspace, the launchers).

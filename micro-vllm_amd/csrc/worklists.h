@@ -165,8 +165,8 @@ inline SplitRule split_rule(const AttnArgs& a) {
 
 // Slots of the decode work list and of the decode grid, from shapes alone: at
 // most `capacity` (the workspace's) and no more than choose_split can fill. A
-// slot that stays empty still costs a workgroup's dispatch (~4 ns: 1,500 of
-// them took 6 of the 37 us of 30 decodes and two chunks at head_dim 64).
+// slot that stays empty still costs a workgroup's dispatch (~4 ns, 6 us for
+// 1,500 of them).
 // Splits of 2,048 tokens fit every one of the bounds.
 // `decodes`: the batch looks like decodes alone. Beside prefill work spare slots
 // cost more than their dispatch: the work is then spread over the CUs unevenly (8

@@ -17,7 +17,7 @@ from test_gpu_attention import build_case, operator, run_and_check
 pytestmark = pytest.mark.gpu
 
 # One to two splits, every size of merge round and two rounds (17,000 tokens in
-# splits of 256), and requests that are not split.
+# splits of about 272), and requests that are not split.
 LENGTHS = [1, 64, 65, 130, 260, 700, 1300, 1700, 3000, 17_000]
 
 
