@@ -155,6 +155,8 @@ bool decode_supported(int64_t head_dim, int64_t block_size, int64_t split_tokens
 // 16 rows of this stride lie within a 32-bit byte offset, as the pipelined
 // decode kernel addresses them (the general one, at head_dim 128, does not).
 inline bool rows_within_32_bits(int64_t token_stride) { return 32 * token_stride < (int64_t{1} << 32); }
+// The batch's decodes run on the general split kernel.
+bool decode_general(const AttnArgs& a);
 int64_t decode_step_blocks(const AttnArgs& a);  // decode workgroups of the step grid
 // `prefill_first`: the prefill workgroups lead the grid (else the decode ones).
 int launch_step(const AttnArgs& a, int32_t dtype, bool prefill_first, hipStream_t s, hipEvent_t start,

@@ -340,12 +340,13 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
   a.split_fixed = decode_split_override();
   a.split_tokens = a.split_fixed ? a.split_fixed : kMaxSplit;
   a.num_cus = device_cu_count();
+  const bool general = decode_general(a);
+  a.merge_apart = general || merge_apart(a, batch) ? 1 : 0;
   a.item_capacity = a.split_fixed ? d.item_capacity
                                   : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
-                                               d.item_capacity, a.num_cus, D, a.num_kv_heads, looks_like_decodes(batch));
+                                               d.item_capacity, a.num_cus, D, a.num_kv_heads, looks_like_decodes(batch), general);
   a.decode_only = batch->max_query_len == 1 ? 1 : 0;
-  a.merge_apart = merge_apart(a, batch) ? 1 : 0;
-  a.rule = split_rule(a);
+  a.rule = split_rule(a, general);
   a.ws_acc = reinterpret_cast<float*>(w);
   a.ws_ml = reinterpret_cast<float2*>(w + d.acc_bytes);
   a.items = reinterpret_cast<PrefillItem*>(w + d.acc_bytes + d.ml_bytes);

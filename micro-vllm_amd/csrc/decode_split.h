@@ -161,8 +161,9 @@ __device__ __forceinline__ void merge_request(const AttnArgs& a, int64_t base, i
 // request with one split gets its output directly; otherwise the partial goes
 // to the workspace, and the workgroup that completes the request (for its
 // group of KV heads, `head_group`) merges the partials. `flag`: an LDS word
-// that no wave uses any more once all have entered.
-template <typename T, int D>
+// that no wave uses any more once all have entered. MERGE false: a launch of its
+// own merges every batch (the merge's registers are not needed).
+template <typename T, int D, bool MERGE>
 __device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem& item, int h, bool live, int head_group,
                                              int head_groups, float m, float lt, const float4_t (&acc)[D / 16],
                                              int32_t* flag) {
@@ -195,21 +196,23 @@ __device__ __forceinline__ void finish_split(const AttnArgs& a, const DecodeItem
                          static_cast<uint64_t>(__float_as_uint(m)) | (static_cast<uint64_t>(__float_as_uint(lt)) << 32),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (a.merge_apart) return;
-  // This wave's partials have reached the point all XCDs read from.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  int32_t* const counter = a.done + static_cast<int64_t>(item.r) * head_groups + head_group;
-  if (threadIdx.x == 0) {
-    // Counts to ns and wraps to zero for the next launch, in one operation: a
-    // reset of its own would lose counts that another launch on this workspace
-    // added in between, and leave the counter off for every later one.
-    const uint32_t last = static_cast<uint32_t>(item.ns) - 1;
-    *flag = atomicInc(reinterpret_cast<unsigned int*>(counter), last) == last;
+  if constexpr (MERGE) {
+    if (a.merge_apart) return;
+    // This wave's partials have reached the point all XCDs read from.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int32_t* const counter = a.done + static_cast<int64_t>(item.r) * head_groups + head_group;
+    if (threadIdx.x == 0) {
+      // Counts to ns and wraps to zero for the next launch, in one operation: a
+      // reset of its own would lose counts that another launch on this workspace
+      // added in between, and leave the counter off for every later one.
+      const uint32_t last = static_cast<uint32_t>(item.ns) - 1;
+      *flag = atomicInc(reinterpret_cast<unsigned int*>(counter), last) == last;
+    }
+    __syncthreads();
+    if (!*flag || !live) return;
+    merge_request<T, D>(a, item.base, item.qs, __builtin_amdgcn_readfirstlane(h) * G, G, item.ns);
   }
-  __syncthreads();
-  if (!*flag || !live) return;
-  merge_request<T, D>(a, item.base, item.qs, __builtin_amdgcn_readfirstlane(h) * G, G, item.ns);
 }
 
 // Output rows that no split writes, kTidyTokens tokens and as many requests
@@ -618,7 +621,7 @@ __device__ __forceinline__ void decode_split_lds_body(const AttnArgs& a, uint8_t
 
   const float lt = sum_xor32_f(sum_xor16_f(l));
   // The flag lies in the first wave's K tile: written after every wave's loop.
-  finish_split<T, D>(a, item, h, live, static_cast<int>(wg % groups), groups, m, lt, acc, reinterpret_cast<int32_t*>(smem));
+  finish_split<T, D, true>(a, item, h, live, static_cast<int>(wg % groups), groups, m, lt, acc, reinterpret_cast<int32_t*>(smem));
 }
 
 }  // namespace dec

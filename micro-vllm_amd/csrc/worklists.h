@@ -127,6 +127,10 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 //   prefill work 16 up to 128 tokens each where one wave merges more than four
 //   heads (a context of 2,000 and a chunk of 40 with 32/4 heads: 25.8 with 64,
 //   22.2 with 128).
+// The general split kernel (block sizes that are not multiples of 16) keeps four
+// waves per SIMD and waits longer for each tile: two items per CU of 64 to 1,024
+// tokens whatever the heads, and no requests left whole (17 contexts of up to 1,670
+// with 10 heads in blocks of 8: 46.8 by the rule above, 34.6 so).
 // At least total / (capacity - R), so that the items fit the list: a request
 // of v tokens has at most v / split + 1 splits. (2,048-token splits always fit:
 // see item_slots.)
@@ -144,7 +148,8 @@ inline int32_t full_items(int32_t cus, int32_t num_kv_heads) { return num_kv_hea
 inline int32_t full_split(int32_t num_kv_heads) { return num_kv_heads == 1 ? 128 : num_kv_heads < 4 ? 192 : 256; }
 
 // The rule's numbers for a shape. Rates turn tokens into a split length.
-inline SplitRule split_rule(const AttnArgs& a) {
+// `general`: the general split kernel runs.
+inline SplitRule split_rule(const AttnArgs& a, bool general) {
   const int32_t heads = a.num_kv_heads, cus = a.num_cus;
   const float width = a.head_dim / 128.f;
   SplitRule r;
@@ -160,6 +165,12 @@ inline SplitRule split_rule(const AttnArgs& a) {
   r.beside_most = heads == 4 ? 768 : kMaxSplit;
   r.merge_apart = a.merge_apart;
   r.beside_merge = !a.merge_apart && a.group > 4 ? 16 : 0;
+  if (general) {
+    r.small = r.full = r.beside_small = r.beside_full = width / (2.f * cus);
+    r.least = kSmallSplit;
+    r.whole_decodes = INT32_MAX;
+    r.beside_most = kMostSplit;
+  }
   return r;
 }
 
@@ -172,14 +183,15 @@ inline SplitRule split_rule(const AttnArgs& a) {
 // cost more than their dispatch: the work is then spread over the CUs unevenly (8
 // decodes of 2,000 and a chunk of 500 with 32/4 heads: 27.5, 32.0 with 96 more).
 inline int64_t item_slots(int64_t requests, int64_t reach, int64_t capacity, int64_t cus, int64_t head_dim,
-                          int32_t num_kv_heads, bool decodes) {
+                          int32_t num_kv_heads, bool decodes, bool general) {
   auto least = [](int64_t x, int64_t y) { return x < y ? x : y; };
   auto larger = [](int64_t x, int64_t y) { return x > y ? x : y; };
   const int64_t tokens = requests * reach;
   const int64_t small = (decodes ? small_items(static_cast<int32_t>(cus), num_kv_heads) : 96) * 128 / head_dim + 1;
   const int64_t full = least(full_items(static_cast<int32_t>(cus), num_kv_heads) * 128LL / head_dim,
                              tokens / full_split(num_kv_heads)) + 1;
-  const int64_t slots = requests + larger(larger(small, full), tokens / kMostSplit + 1);
+  const int64_t any = least(2 * cus * 128 / head_dim, tokens / kSmallSplit) + 1;
+  const int64_t slots = requests + larger(general ? any : larger(small, full), tokens / kMostSplit + 1);
   return least(least(slots, requests * ((reach + kSmallSplit - 1) / kSmallSplit)), capacity);
 }
 

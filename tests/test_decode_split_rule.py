@@ -40,9 +40,9 @@ int main() {
     // The workspace's slots, whose split length is 64 to 2,048 (16 or more asked for).
     const int64_t layout = 64 << (rng() % 6);
     const int64_t capacity = a.num_requests * ((reach + 15 + layout) / layout);
-    const bool decodes = rng() % 2;
-    a.item_capacity = item_slots(a.num_requests, reach, capacity, a.num_cus, a.head_dim, a.num_kv_heads, decodes);
-    a.rule = split_rule(a);
+    const bool decodes = rng() % 2, general = rng() % 4 == 0;
+    a.item_capacity = item_slots(a.num_requests, reach, capacity, a.num_cus, a.head_dim, a.num_kv_heads, decodes, general);
+    a.rule = split_rule(a, general);
     for (int trial = 0; trial < 4; ++trial, ++batches) {
       const int64_t least = trial == 0 ? reach : trial == 1 ? 1 : log_int(1, reach);
       const bool others = trial == 3;
