@@ -369,7 +369,7 @@ __device__ __forceinline__ float silu_any(float x) {
   return Act<T>::round(x / (1.f + expf(-x)));
 }
 
-// Two elements per thread: rows that are not 16-byte aligned.
+// Two elements per thread: rows that are not 16-byte aligned, and narrow ones.
 template <typename T>
 __global__ __launch_bounds__(256) void silu_mul_kernel(SiluArgs a) {
   const int64_t row = blockIdx.y;
@@ -792,9 +792,11 @@ extern "C" int mvllm_silu_mul(const void* gate_up, int64_t in_stride, void* out,
              static_cast<int32_t>(intermediate)};
   const dim3 grid(static_cast<unsigned>((intermediate / 2 + 255) / 256), static_cast<unsigned>(rows));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // 16-byte aligned rows, in and out (the up half starts `intermediate` elements in).
-  const bool vec = mult8(intermediate) && mult8(in_stride) && mult8(out_stride) && aligned16(gate_up) && aligned16(out) &&
-                   intermediate <= INT32_MAX;
+  // 16-byte aligned rows, in and out (the up half starts `intermediate` elements
+  // in), wide enough for half a workgroup's vectors (4,096 rows of 64: 4.1 us two
+  // elements per thread, 4.9 eight; of 512 4.7 and 4.9; of 1,024 6.9 and 6.5).
+  const bool vec = intermediate >= 512 && mult8(intermediate) && mult8(in_stride) && mult8(out_stride) &&
+                   aligned16(gate_up) && aligned16(out) && intermediate <= INT32_MAX;
   if (vec && dtype == MVLLM_DTYPE_BF16)
     launch_silu_rows<bf16_t>(a, s);
   else if (vec)
