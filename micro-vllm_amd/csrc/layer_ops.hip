@@ -535,21 +535,29 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
-// One workgroup per row. Eight vectors of 16 bytes in flight per lane: the
-// next four are loaded while four are searched.
+// One workgroup per row.
 //
-// The search is two-level, which takes a third of the vector instructions of
-// an element-by-element one: per vector only its maximum is formed (v_max3)
-// and compared with the lane's best, which remembers the vector; the element
-// is looked up in that one vector at the end. Indices grow along a lane's
-// walk and a strictly greater value is needed to replace the best, so the
-// first of equal values stays. NaN (the maximum, by torch's rule) is passed
-// over by v_max3 and only noted; a row that holds one is searched again
-// element by element. Vectors past the row's end re-read its last one, which
-// changes nothing: the smaller index of equal candidates wins. The bound is
-// HBM: 256 bf16 rows of 151,936 (78 MB) took 18.6 us element by element with
-// four vectors in flight, 13.0 us now (6.0 TB/s).
-template <typename T>
+// WIDE: eight vectors of 16 bytes in flight per lane, the next four loaded
+// while four are searched, and a two-level search, which takes a third of the
+// vector instructions of an element-by-element one: per vector only its maximum
+// is formed (v_max3) and compared with the lane's best, which remembers the
+// vector; the element is looked up in that one vector at the end. Indices grow
+// along a lane's walk and a strictly greater value is needed to replace the
+// best, so the first of equal values stays. NaN (the maximum, by torch's rule)
+// is passed over by v_max3 and only noted; a row that holds one is searched
+// again element by element. Vectors past the row's end re-read its last one,
+// which changes nothing: the smaller index of equal candidates wins. The bound
+// is HBM: 256 bf16 rows of 151,936 (78 MB) take 13.0 us (6.0 TB/s), element by
+// element with four vectors in flight 18.6.
+//
+// Otherwise element by element: the wide form's fixed costs (loads past a short
+// row's end, and the look-up, one more round trip) show in narrow rows, and its
+// registers cost where several workgroups share a CU. us, element by element and
+// wide: bf16 1 x 4,096 3.4 and 4.3, 257 x 16,384 5.9 and 7.7, x 64,000 13.1 and
+// 10.8; 400 x 32,000 8.8 and 9.9; 1,024 x 128,256 46 and 55. fp32, whose vectors
+// hold four: 16 x 48,000 7.2 and 7.1, x 64,000 8.6 and 7.9, x 151,936 16.1 and
+// 11.3; 128 x 151,936 19.0 and 20.8; 1,024 x 64,000 42 and 55.
+template <typename T, bool WIDE>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(ArgmaxArgs a) {
   const int64_t row = blockIdx.x;
   const uint8_t* base = a.logits + row * a.row_stride * a.esize;
@@ -557,8 +565,26 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(ArgmaxArgs 
   const int tid = threadIdx.x;
   constexpr int P = Logit<T>::kPerVec;
   const int64_t nvec = a.vec ? a.cols / P : 0;
-  if (nvec > 0) {
-    const uint4* vp = reinterpret_cast<const uint4*>(base);
+  const uint4* vp = reinterpret_cast<const uint4*>(base);
+  auto each = [&] {
+    for (int64_t v0 = tid; v0 < nvec; v0 += 4LL * kArgmaxThreads) {
+      uint4 buf[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t v = v0 + static_cast<int64_t>(u) * kArgmaxThreads;
+        buf[u] = v < nvec ? vp[v] : uint4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t v = v0 + static_cast<int64_t>(u) * kArgmaxThreads;
+        if (v < nvec) {
+#pragma unroll
+          for (int e = 0; e < P; ++e) lane_state.see(Logit<T>::get(buf[u], e), static_cast<uint32_t>(v * P + e));
+        }
+      }
+    }
+  };
+  if constexpr (WIDE) {
     typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
     auto load = [&](int64_t v) {
       const uint4v w = __builtin_nontemporal_load(reinterpret_cast<const uint4v*>(vp + (v < nvec ? v : nvec - 1)));
@@ -606,16 +632,17 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(ArgmaxArgs 
     lane_state.best_idx = static_cast<uint32_t>(best_v * P + first);
     if (__syncthreads_or(nan)) {
       lane_state = ArgmaxLane();
-      for (int64_t c = tid; c < nvec * P; c += kArgmaxThreads)
-        lane_state.see(Logit<T>::get1(base + c * a.esize), static_cast<uint32_t>(c));
+      each();
     }
-    // The tail past the last whole vector, by the first lanes.
-    const int64_t tail = nvec * P + tid;
-    if (tail < a.cols) lane_state.see(Logit<T>::get1(base + tail * a.esize), static_cast<uint32_t>(tail));
+  } else if (a.vec) {
+    each();
   } else {
     for (int64_t c = tid; c < a.cols; c += kArgmaxThreads)
       lane_state.see(Logit<T>::get1(base + c * a.esize), static_cast<uint32_t>(c));
   }
+  // The tail past the last whole vector, by the first lanes.
+  const int64_t tail = nvec * P + tid;
+  if (a.vec && tail < a.cols) lane_state.see(Logit<T>::get1(base + tail * a.esize), static_cast<uint32_t>(tail));
   uint64_t k = lane_state.key();
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) k = max_u64(k, __shfl_xor(k, m, 64));
@@ -630,6 +657,15 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(ArgmaxArgs 
     a.out[row] = idx;
     if (a.out_copy) a.out_copy[row] = idx;
   }
+}
+
+template <typename T>
+void launch_argmax(const ArgmaxArgs& a, hipStream_t s) {
+  const int64_t vectors = a.vec ? a.cols / Logit<T>::kPerVec : 0;
+  const bool wide = sizeof(T) == 4 ? vectors >= 16000 && a.rows <= 64 : vectors >= 4000 && a.rows <= 320;
+  const dim3 grid(static_cast<unsigned>(a.rows));
+  if (wide) hipLaunchKernelGGL((argmax_rows_kernel<T, true>), grid, dim3(kArgmaxThreads), 0, s, a);
+  else hipLaunchKernelGGL((argmax_rows_kernel<T, false>), grid, dim3(kArgmaxThreads), 0, s, a);
 }
 
 bool half_dtype(int32_t d) { return d == MVLLM_DTYPE_BF16 || d == MVLLM_DTYPE_F16; }
@@ -869,13 +905,9 @@ extern "C" int mvllm_argmax_rows(const void* logits, int64_t rows, int64_t cols,
   a.esize = esize;
   a.vec = aligned16(logits) && (row_stride * esize) % 16 == 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<unsigned>(rows));
-  if (dtype == MVLLM_DTYPE_BF16)
-    hipLaunchKernelGGL(argmax_rows_kernel<bf16_t>, grid, dim3(kArgmaxThreads), 0, s, a);
-  else if (dtype == MVLLM_DTYPE_F16)
-    hipLaunchKernelGGL(argmax_rows_kernel<f16_t>, grid, dim3(kArgmaxThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL(argmax_rows_kernel<float>, grid, dim3(kArgmaxThreads), 0, s, a);
+  if (dtype == MVLLM_DTYPE_BF16) launch_argmax<bf16_t>(a, s);
+  else if (dtype == MVLLM_DTYPE_F16) launch_argmax<f16_t>(a, s);
+  else launch_argmax<float>(a, s);
   MVLLM_LAUNCH_CHECK("argmax_rows_kernel");
   return MVLLM_OK;
 }

@@ -17,14 +17,16 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("vectors", [1, 2, 1023, 1025, 4096, 4097, 8192, 12_000])
+@pytest.mark.parametrize("vectors", [1, 2, 1023, 1025, 3999, 4000, 4097, 8192, 16_001])
 @pytest.mark.parametrize("tail", [0, 3])
-def test_widths_ties_and_nan(device, dtype, vectors, tail):
+@pytest.mark.parametrize("rows", [12, 401], ids=["few", "many"])
+def test_widths_ties_and_nan(device, dtype, vectors, tail, rows):
+    """12 rows of 4,000 vectors or more (fp32: 16,000) take the two-level search,
+    401 rows and narrower ones the element-wise one."""
     per = 4 if dtype == torch.float32 else 8
     cols = vectors * per + tail
     gen = torch.Generator(device=device).manual_seed(cols)
     stride = (vectors + 1) * per  # rows stay 16-byte aligned
-    rows = 12
     logits = torch.empty((rows, stride), dtype=dtype, device=device)[:, :cols]
     logits.copy_(torch.randint(-300, 300, (rows, cols), generator=gen, device=device).to(dtype) / 64)
     assert logits.data_ptr() % 16 == 0 and logits.stride(0) * logits.element_size() % 16 == 0
