@@ -41,6 +41,7 @@ struct SplitRule {
   float whole;                      // longest request answered whole, per token of the batch
   int32_t whole_decodes;            // requests that fill the chip by themselves
   int32_t least;                    // a shorter split than this is only for few tokens
+  int32_t shortest;                 // no split is shorter
   int32_t beside_most;              // longest split beside prefill work
   int32_t merge_apart;              // the partials are merged by a launch of their own
   int32_t beside_merge;             // splits per request beside prefill work, up to 128 tokens each (0: no bound)

@@ -341,7 +341,7 @@ int bind_workspace(AttnArgs& a, const mvllm_batch* batch, int64_t Hq, int64_t D,
   a.split_tokens = a.split_fixed ? a.split_fixed : kMaxSplit;
   a.num_cus = device_cu_count();
   const bool general = decode_general(a);
-  a.merge_apart = general || merge_apart(a, batch) ? 1 : 0;
+  a.merge_apart = (general ? general_merges(a.width * a.block_size, a.split_fixed) : merge_apart(a, batch)) ? 1 : 0;
   a.item_capacity = a.split_fixed ? d.item_capacity
                                   : item_slots(batch->num_requests, batch->block_table_width * batch->block_size,
                                                d.item_capacity, a.num_cus, D, a.num_kv_heads, looks_like_decodes(batch), general);

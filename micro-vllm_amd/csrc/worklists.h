@@ -137,6 +137,7 @@ __device__ inline void copy_kv_row(const KvRowArgs& a, int64_t token, int first,
 constexpr int kDecodeListThreads = 1024;
 constexpr int kSizeBuckets = 64;  // sizes of a partial split, split / 64 tokens (rounded up to a power of two) each
 constexpr int32_t kSmallSplit = 64, kMostSplit = 1024;
+constexpr int32_t kGeneralWhole = 128;  // reach up to which the general split kernel answers requests whole
 
 // Items (of 128-wide tokens) that a batch is split into, at most, by the rule above.
 inline int32_t small_items(int32_t cus, int32_t num_kv_heads) {
@@ -146,6 +147,13 @@ inline int32_t small_items(int32_t cus, int32_t num_kv_heads) {
 }
 inline int32_t full_items(int32_t cus, int32_t num_kv_heads) { return num_kv_heads < 4 ? 4 * cus : 2 * cus; }
 inline int32_t full_split(int32_t num_kv_heads) { return num_kv_heads == 1 ? 128 : num_kv_heads < 4 ? 192 : 256; }
+
+// The general split kernel leaves its merge to a launch, which a batch without
+// splits does not need: up to 128 tokens one wave answers a request about as fast
+// as two and the merge (a context of 102 with 16/1 heads in blocks of 8: 15.0 us,
+// 16.3 split; 229 of up to 78 with 48/8 22.8, 26.5 with the launch), of 160 not (8
+// with 16/8 heads: 21.6, 18.5).
+inline bool general_merges(int64_t reach, int64_t split_fixed) { return split_fixed || reach > kGeneralWhole; }
 
 // The rule's numbers for a shape. Rates turn tokens into a split length.
 // `general`: the general split kernel runs.
@@ -162,12 +170,14 @@ inline SplitRule split_rule(const AttnArgs& a, bool general) {
   r.whole = heads * a.head_dim / (0.04f * 1.55e6f);
   r.whole_decodes = (3 * cus + 4 * ((heads + 3) / 4) - 1) / (4 * ((heads + 3) / 4));
   r.least = full_split(heads);
+  r.shortest = kSmallSplit;
   r.beside_most = heads == 4 ? 768 : kMaxSplit;
   r.merge_apart = a.merge_apart;
   r.beside_merge = !a.merge_apart && a.group > 4 ? 16 : 0;
   if (general) {
     r.small = r.full = r.beside_small = r.beside_full = width / (2.f * cus);
-    r.least = kSmallSplit;
+    // Without the merge launch (general_merges) no request may be split.
+    r.least = r.shortest = a.merge_apart ? kSmallSplit : kGeneralWhole;
     r.whole_decodes = INT32_MAX;
     r.beside_most = kMostSplit;
   }
@@ -207,7 +217,7 @@ __host__ __device__ inline int32_t choose_split(int64_t total, int32_t longest, 
   const int32_t most = beside_prefill ? rule.beside_most : kMostSplit;
   int32_t split = up16(tokens * (beside_prefill ? rule.beside_full : rule.full));
   int32_t least = up16(tokens * (beside_prefill ? rule.beside_small : rule.small));
-  least = least < kSmallSplit ? kSmallSplit : least > rule.least ? rule.least : least;
+  least = least < rule.shortest ? rule.shortest : least > rule.least ? rule.least : least;
   if (beside_prefill && rule.beside_merge > 0) {
     const int32_t few = longest / rule.beside_merge < 112 ? (longest / rule.beside_merge + 16) & ~15 : 128;
     least = least < few ? few : least;

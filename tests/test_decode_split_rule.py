@@ -1,5 +1,6 @@
 """The rule that picks the decode splits' length, on the host: every split of a
-batch fits the work list, whatever the shape and the lengths."""
+batch fits the work list, whatever the shape and the lengths, and the general
+kernel splits nothing where it has no merge launch."""
 
 from __future__ import annotations
 
@@ -41,6 +42,7 @@ int main() {
     const int64_t layout = 64 << (rng() % 6);
     const int64_t capacity = a.num_requests * ((reach + 15 + layout) / layout);
     const bool decodes = rng() % 2, general = rng() % 4 == 0;
+    if (general) a.merge_apart = general_merges(reach, 0);
     a.item_capacity = item_slots(a.num_requests, reach, capacity, a.num_cus, a.head_dim, a.num_kv_heads, decodes, general);
     a.rule = split_rule(a, general);
     for (int trial = 0; trial < 4; ++trial, ++batches) {
@@ -60,7 +62,8 @@ int main() {
       int64_t items = 0;
       for (int64_t v : tokens) items += (v + split - 1) / split;
       whole += split >= longest;
-      if (split < 16 || split % 16 || split > kMaxSplit || items > a.item_capacity) {
+      if (split < 16 || split % 16 || split > kMaxSplit || items > a.item_capacity ||
+          (general && !a.merge_apart && split < longest)) {
         std::printf("requests %lld reach %lld heads %d group %d dim %d slots %lld split %d items %lld\n",
                     (long long)a.num_requests, (long long)reach, a.num_kv_heads, a.group, a.head_dim,
                     (long long)a.item_capacity, split, (long long)items);

@@ -42,6 +42,20 @@ def test_dims_and_the_general_kernel(device, d, dtype, hq, hkv, bs):
     run_and_check(q, k, v, cache, md, dtype)
 
 
+@pytest.mark.parametrize("longest", [20, 64, 65, 120, 128, 136])
+@pytest.mark.parametrize("chunk", [0, 3])
+@pytest.mark.parametrize(("hq", "hkv", "bs"), [(16, 8, 8), (14, 2, 24), (32, 32, 8)], ids=str)
+def test_the_general_kernel_without_splits(device, longest, chunk, hq, hkv, bs):
+    """Tables that reach at most 128 tokens: no request is split and no merge launched."""
+
+    lengths = [longest, 1, max(1, longest - 9)] * 20 + [longest] * (chunk > 0)
+    qlens = [1] * 60 + [chunk] * (chunk > 0)
+    q, k, v, cache, md = build_case(device, torch.bfloat16, lengths, qlens, hq, hkv, 128, bs, seed=longest)
+    run_and_check(q, k, v, cache, dataclasses.replace(md, max_query_len=max(1, chunk)), torch.bfloat16)
+    plan = AttentionPlan(md, hq, cache)
+    assert torch.equal(hip_attention_over_cache(q, cache, md, plan=plan), hip_attention_over_cache(q, cache, md))
+
+
 @pytest.mark.parametrize(("requests", "n"), [(40, 600), (190, 300), (200, 300), (33, 1500)])
 @pytest.mark.parametrize(("hq", "hkv"), [(4, 1), (16, 4), (16, 16)], ids=str)
 def test_batches_around_the_rules_ends(device, requests, n, hq, hkv):
